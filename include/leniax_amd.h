@@ -171,6 +171,14 @@ int lx_potential_direct_adjoint(const lx_rule* rule, const float* state_d, int64
                                 int32_t kh, int32_t kw, const float* dpot_d, float* dstate_d, float* dkern_d,
                                 void* stream);
 
+/* The same with a workspace of lx_potential_direct_adjoint_size bytes for the kernel side's partial
+ * sums, which then runs on the matrix cores over tiles of the worlds (without one: one workgroup per
+ * kernel tap over all worlds).  Deterministic: the partial sums are added in a fixed order. */
+int lx_potential_direct_adjoint_size(const lx_rule* rule, int64_t B, int32_t kh, int32_t kw, size_t* bytes);
+int lx_potential_direct_adjoint_work(const lx_rule* rule, const float* state_d, int64_t B, const float* kern_d,
+                                     int32_t kh, int32_t kw, const float* dpot_d, float* dstate_d,
+                                     float* dkern_d, void* work_d, void* stream);
+
 /* leniax/core.py:163-199 get_field (+ weighted_sum/weighted_mean):
  * field_d [B][C][dims] = sum_k w[c][k] g_k(potential_k) (/ sum_k w[c][k]).
  * gf_d [K][2] (m, s) and w_d [C][K] per world with strides gf_bstride / w_bstride floats (0: shared). */

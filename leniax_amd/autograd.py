@@ -496,18 +496,23 @@ class _PotentialDirect(torch.autograd.Function):
         maxk = Kr.shape[0] // C
         slots = core._slots(C, maxk, ctx.meta)
         kh, kw = int(Kr.shape[2]), int(Kr.shape[3])
-        kern = Kr[list(slots), 0].contiguous()
+        kern = Kr[_slot_index(slots, Kr.device), 0].contiguous()
         rule = core._rule(A.shape[2:], C, len(slots), [s // maxk for s in slots])
         need_A, need_K = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dA = torch.empty_like(A) if need_A else None
         dk = torch.empty_like(kern) if need_K else None
         gc = g.contiguous()
-        _lib.call('lx_potential_direct_adjoint', ctypes.byref(rule), engine.ptr(A), N, engine.ptr(kern), kh, kw,
-                  engine.ptr(gc), engine.ptr(dA), engine.ptr(dk), engine.stream_ptr())
+        work = None
+        if need_K:  # partial sums of the kernel side, held until the call has enqueued its kernels
+            nb = ctypes.c_size_t(0)
+            _lib.call('lx_potential_direct_adjoint_size', ctypes.byref(rule), N, kh, kw, ctypes.byref(nb))
+            work = torch.empty(max(int(nb.value), 256), dtype=torch.uint8, device=A.device)
+        _lib.call('lx_potential_direct_adjoint_work', ctypes.byref(rule), engine.ptr(A), N, engine.ptr(kern), kh, kw,
+                  engine.ptr(gc), engine.ptr(dA), engine.ptr(dk), engine.ptr(work), engine.stream_ptr())
         dK = None
         if need_K:
             dK = torch.zeros_like(Kr)
-            dK[list(slots), 0] = dk
+            dK[_slot_index(slots, Kr.device), 0] = dk
         return dA, dK, None, None
 
 
