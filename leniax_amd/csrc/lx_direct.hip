@@ -5,10 +5,10 @@
 //
 //   U[b][k][y][x] = sum_{i<kh, j<kw} A[b][cin k][(y + i - ph) mod H][(x + j - pw) mod W] * kern[k][i][j]
 //
-// One workgroup computes a TH x TW tile of one (world, kernel) output: the input tile and its
-// halo are staged in LDS (wrap indexing), each thread keeps a 1 x 4 strip of outputs and slides
-// a 4-wide register window along each kernel row, so that one LDS read feeds 4 FMAs; the kernel
-// taps are uniform (scalar loads).  Any world size; kernels up to 64 x 64.
+// The potential and its reverse are sums of products over a sliding window: contractions of the
+// staged image with a Toeplitz matrix of the taps, taken on the matrix cores in float32
+// (v_mfma_f32_4x4x1: 16 independent 4 x 4 outer products per instruction, twice the rate of the
+// vector unit's multiply-adds).  Any world size; kernels up to 64 x 64.
 #include <algorithm>
 #include <type_traits>
 
@@ -16,11 +16,12 @@
 
 namespace {
 
-constexpr int TH = 16, TW = 64, MAXK = 64;
+constexpr int MAXK = 64, TX = 64;  // largest kernel side; output columns of a workgroup
+typedef float f4v __attribute__((ext_vector_type(4)));
 
-// LDS tile row length: the output tile, the kernel's halo and one spare column (the window's
-// last shift reads it), rounded up to a multiple of 4 so that rows start 16-byte aligned
-__host__ __device__ inline int tile_cols(int kw) { return (TW + kw + 3) & ~3; }
+// LDS row stride of at least `need` floats: 16 or 48 mod 64, so that the four rows of four 16-byte
+// pieces that 16 lanes read at once lie in different banks
+__host__ __device__ inline int bank_stride(int need) { return (need - 16 + 31) / 32 * 32 + 16; }
 
 // Stage rows [y0 - qh, y0 - qh + trows) x columns [x0 - qw, x0 - qw + tcols) of an H x W
 // image, wrapped, into tile[trows][stride]: each thread keeps one column (one modulo per thread,
@@ -39,123 +40,173 @@ LX_DEV bool stage_tile(float* tile, const float* img, int H, int W, int y0, int 
     gx += gx < 0 ? W : 0;
     int gy = (y0 + r0 - qh) % H;
     gy += gy < 0 ? H : 0;
-    // 8 rows per round: the loads are all issued before the first LDS write waits on them.
+    // 16 rows per round: the loads are all issued before the first LDS write waits on them.
     // The row advances by nsplit, i.e. by step = nsplit mod H < H, so one conditional
     // subtraction keeps gy in [0, H) for any world height.
+    constexpr int BATCH = 16;
     const int step = nsplit % H;
-    for (int rb = r0; rb < trows; rb += 8 * nsplit) {
-      float v[8];
-      int rows[8];
+    for (int rb = r0; rb < trows; rb += BATCH * nsplit) {
+      float v[BATCH];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        rows[u] = rb + u * nsplit;
-        v[u] = rows[u] < trows ? img[int64_t(gy) * W + gx] : 0.f;
+      for (int u = 0; u < BATCH; ++u) {
+        v[u] = rb + u * nsplit < trows ? img[int64_t(gy) * W + gx] : 0.f;
         gy += step;
         gy -= gy >= H ? H : 0;
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (rows[u] < trows) {
-          tile[rows[u] * stride + c] = v[u];
-          odd |= not_finite(v[u]);
-        }
+      for (int u = 0; u < BATCH; ++u) {
+        if (rb + u * nsplit < trows) tile[(rb + u * nsplit) * stride + c] = v[u];
+        odd |= not_finite(v[u]);
+      }
     }
   }
   return odd;
 }
 
-// acc[e] += sum_{j < kw} k_j row[e + j], e < 4, j in increasing order (k_j = kr[j], or kr[kw-1-j]
-// when FLIP): taps in blocks of 4 against an 8-wide window read 16 bytes at a time (16 FMAs per
-// two LDS reads, no register shifts), the remaining taps one at a time.
-template <bool FLIP>
-LX_DEV void row_taps(const float* row, const float* kr, int kw, float (&acc)[4]) {
-  float4 lo = *reinterpret_cast<const float4*>(row);
-  int j = 0;
-  for (; j + 4 <= kw; j += 4) {
-    const float4 hi = *reinterpret_cast<const float4*>(row + j + 4);
-    const float w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float kv = FLIP ? kr[kw - 1 - (j + t)] : kr[j + t];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = fmaf(kv, w[e + t], acc[e]);
-    }
-    lo = hi;
-  }
-  float w0 = lo.x, w1 = lo.y, w2 = lo.z, w3 = lo.w;
-  for (; j < kw; ++j) {
-    const float kv = FLIP ? kr[kw - 1 - j] : kr[j];
-    acc[0] = fmaf(kv, w0, acc[0]);
-    acc[1] = fmaf(kv, w1, acc[1]);
-    acc[2] = fmaf(kv, w2, acc[2]);
-    acc[3] = fmaf(kv, w3, acc[3]);
-    w0 = w1; w1 = w2; w2 = w3; w3 = row[j + 4];
-  }
-}
-
 struct DirectArgs {
   const float* A;
   const float* kern;
-  float* U;
   int H, W, C, K, kh, kw, ph, pw;
+  int vec;  // rows of U (or dA) take 16-byte stores
   int cin[LX_MAX_K];
 };
 
-__global__ __launch_bounds__(256) void direct_kernel(DirectArgs a) {
-  extern __shared__ __align__(16) float tile[];  // (TH + kh - 1) rows x tile_cols(kw) columns
-  const int tcols = tile_cols(a.kw);
-  const int trows = TH + a.kh - 1;
-  const int x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
-  const int64_t bk = blockIdx.z;
-  const int64_t b = bk / a.K;
-  const int k = int(bk - b * a.K);
-  const float* A = a.A + (b * a.C + a.cin[k]) * int64_t(a.H) * a.W;
-  stage_tile(tile, A, a.H, a.W, y0, x0, a.ph, a.pw, trows, tcols, tcols);
-  __syncthreads();
-  const int ty = threadIdx.x / (TW / 4), tx4 = (threadIdx.x % (TW / 4)) * 4;
-  const float* kk = a.kern + int64_t(k) * a.kh * a.kw;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < a.kh; ++i) row_taps<false>(tile + (ty + i) * tcols + tx4, kk + i * a.kw, a.kw, acc);
-  const int y = y0 + ty;
-  if (y < a.H) {
-    float* out = a.U + (bk * a.H + y) * int64_t(a.W) + x0 + tx4;
+// Columns of the input that the 4 outputs of a lane's block read, in quads: taps 0..kw-1 of 4 shifts
+__host__ __device__ inline int tap_quads(int kw) { return (kw + 3 + 3) / 4; }
+// tap row stride: >= 4 quads + 3, 4 mod 8 (the four tap rows 4 apart that a wave reads: different banks)
+__host__ __device__ inline int tap_stride(int kw) { return (4 * tap_quads(kw) + 3 + 3) / 8 * 8 + 4; }
+__host__ __device__ inline int direct_stride(int kw) { return bank_stride(TX - 4 + 4 * tap_quads(kw)); }
+size_t direct_lds(int R, int kh, int kw) {
+  return (size_t(16 * R + kh - 1) * direct_stride(kw) + size_t(kh + 1) * tap_stride(kw)) * sizeof(float);
+}
+
+// The potential (ADJ: the state side of its reverse, dA[b][c] = sum over the kernels k fed by c of the
+// correlation of dU[b][k] with the flipped kernel, wrap-padded with kh - 1 - ph before).  A workgroup
+// computes 16 R rows x 64 columns of one image, a wave 4 R x 64: in lane 4 b + n, accumulator g holds
+// the outputs of row 4 g + n at columns 4 b .. 4 b + 3.  For input row s of the wave's window and
+// column jj of a block's, the instruction takes the lane's input value (row n + s, column 4 b + jj)
+// times the four taps k[s - 4 g][jj - m], m < 4 (zero outside the kernel): one 16-byte LDS read feeds
+// 4 R instructions, and one register holds the taps of 4 columns and R accumulators, broadcast by
+// block, so 7 quads of columns take 28 tap columns for a 25-tap row (1.12x the products).  Each output
+// adds its products in the order of i, then j.  A tile that holds a value that is not finite is summed
+// product by product, so that none meets a zero beside the kernel.
+// Measured, 128 worlds of 128^2, 25 x 25 taps, R = 2: potential 60 -> 52 us (50 TFLOP/s of the taps), state
+// side 94 -> 54 us (the vector units' window kernel before took its flipped taps one by one); 12 us of
+// it stage the tiles, the instructions themselves need 25.
+template <int R, bool ADJ>
+__global__ __launch_bounds__(256) void direct_mfma_kernel(DirectArgs a, const float* in, float* out) {
+  extern __shared__ __align__(16) float lds[];
+  const int S = direct_stride(a.kw), TS = tap_stride(a.kw), Q = tap_quads(a.kw), rows = 16 * R + a.kh - 1;
+  float* tile = lds;
+  float* taps = lds + rows * S;
+  const int x0 = blockIdx.x * TX, y0 = blockIdx.y * 16 * R;
+  const int nout = ADJ ? a.C : a.K;
+  const int64_t b = blockIdx.z / nout;
+  const int o = int(blockIdx.z - b * nout);  // the kernel, or (ADJ) the channel
+  const int lane = threadIdx.x & 63, wy = (threadIdx.x >> 6) * 4 * R;
+  const int n = lane & 3, blk = lane >> 2;
+  const bool busy = y0 + wy < a.H;  // the wave has rows of the image
+  f4v acc[R];
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (x0 + tx4 + e < a.W) out[e] = acc[e];
+  for (int g = 0; g < R; ++g) acc[g] = f4v{0.f, 0.f, 0.f, 0.f};
+  for (int k = ADJ ? 0 : o; k < (ADJ ? a.K : o + 1); ++k) {
+    if (ADJ && a.cin[k] != o) continue;
+    const int64_t img = ADJ ? b * a.K + k : b * a.C + a.cin[k];
+    const int qh = ADJ ? a.kh - 1 - a.ph : a.ph, qw = ADJ ? a.kw - 1 - a.pw : a.pw;
+    __syncthreads();  // the previous kernel's tile is consumed
+    const bool odd = stage_tile(tile, in + img * a.H * a.W, a.H, a.W, y0, x0, qh, qw, rows, TX - 4 + 4 * Q, S);
+    const float* kk = a.kern + int64_t(k) * a.kh * a.kw;
+    for (int e = threadIdx.x; e < (a.kh + 1) * TS; e += 256) {
+      const int i = e / TS, j = e - i * TS - 3;
+      const bool in_row = i < a.kh && j >= 0 && j < a.kw;
+      taps[e] = !in_row ? 0.f : ADJ ? kk[(a.kh - 1 - i) * a.kw + a.kw - 1 - j] : kk[i * a.kw + j];
+    }
+    const bool slow = __syncthreads_or(odd);
+    if (!busy) continue;
+    if (!slow) {
+      // lane 16 g + 4 e + m of the tap register: k[s - 4 g][4 q + e - m]
+      const int tg = lane >> 4;
+      const float* tcol = taps + ((lane >> 2) & 3) - n + 3;
+      const float* col = tile + (wy + n) * S + 4 * blk;
+      const int last = a.kh - 1 + 4 * (R - 1);
+      for (int s = 0; s <= last; ++s) {
+        const int ti = unsigned(s - 4 * tg) < unsigned(a.kh) ? s - 4 * tg : a.kh;  // row kh holds zeros
+        const float* trow = tcol + ti * TS;
+        const float* irow = col + s * S;
+        // 4 quads' reads are in flight together, then their instructions
+        for (int q0 = 0; q0 < Q; q0 += 4) {
+          float4 v[4];
+          float t[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int q = q0 + u < Q ? q0 + u : 0;
+            v[u] = *reinterpret_cast<const float4*>(irow + 4 * q);
+            t[u] = trow[4 * q];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (q0 + u >= Q) break;
+            auto column = [&](auto e_c, float x) {
+              constexpr int E = decltype(e_c)::value;
+              acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(t[u], x, acc[0], 4, E, 0);
+              if constexpr (R > 1) acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(t[u], x, acc[1], 4, 4 + E, 0);
+            };
+            column(std::integral_constant<int, 0>{}, v[u].x);
+            column(std::integral_constant<int, 1>{}, v[u].y);
+            column(std::integral_constant<int, 2>{}, v[u].z);
+            column(std::integral_constant<int, 3>{}, v[u].w);
+          }
+        }
+      }
+    } else {
+      for (int i = 0; i < a.kh; ++i)
+        for (int j = 0; j < a.kw; ++j) {
+          const float t = taps[i * TS + j + 3];
+          const float* v = tile + (wy + n + i) * S + 4 * blk + j;
+#pragma unroll
+          for (int g = 0; g < R; ++g)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) acc[g][m] = fmaf(t, v[4 * g * S + m], acc[g][m]);
+        }
+    }
+  }
+  const int x = x0 + 4 * blk;
+  if (!busy || x >= a.W) return;
+#pragma unroll
+  for (int g = 0; g < R; ++g) {
+    const int y = y0 + wy + 4 * g + n;
+    if (y >= a.H) continue;
+    float* dst = out + (int64_t(blockIdx.z) * a.H + y) * a.W + x;
+    if (a.vec) {
+      *reinterpret_cast<f4v*>(dst) = acc[g];
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (x + m < a.W) dst[m] = acc[g][m];
+    }
   }
 }
 
-// Reverse of the direct potential, state side: dA[b][c] = sum over kernels k fed by c of the
-// correlation of dU[b][k] with the flipped kernel, wrap-padded with kh - 1 - ph before (grid:
-// tiles x B * C).  The tile of each kernel's dU is staged in LDS in turn.
-__global__ __launch_bounds__(256) void direct_adj_kernel(DirectArgs a, const float* dU, float* dA) {
-  extern __shared__ __align__(16) float tile[];
-  const int tcols = tile_cols(a.kw);
-  const int trows = TH + a.kh - 1;
-  const int x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
-  const int64_t bc = blockIdx.z;
-  const int64_t b = bc / a.C;
-  const int c = int(bc - b * a.C);
-  const int qh = a.kh - 1 - a.ph, qw = a.kw - 1 - a.pw;
-  const int ty = threadIdx.x / (TW / 4), tx4 = (threadIdx.x % (TW / 4)) * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int k = 0; k < a.K; ++k) {
-    if (a.cin[k] != c) continue;
-    const float* G = dU + (b * a.K + k) * int64_t(a.H) * a.W;
-    __syncthreads();  // the previous kernel's tile is consumed
-    stage_tile(tile, G, a.H, a.W, y0, x0, qh, qw, trows, tcols, tcols);
-    __syncthreads();
-    const float* kk = a.kern + int64_t(k) * a.kh * a.kw;
-    for (int i = 0; i < a.kh; ++i)  // flipped rows and columns
-      row_taps<true>(tile + (ty + i) * tcols + tx4, kk + (a.kh - 1 - i) * a.kw, a.kw, acc);
-  }
-  const int y = y0 + ty;
-  if (y < a.H) {
-    float* out = dA + (bc * a.H + y) * int64_t(a.W) + x0 + tx4;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (x0 + tx4 + e < a.W) out[e] = acc[e];
-  }
+// The launch for `images` output images: R = 2 halves the LDS reads per instruction (52 against 64 us at
+// the size above; R = 4 measured 58, its tiles leave two workgroups per CU); R = 1 where R = 2 would
+// leave CUs with fewer than two workgroups (512) or its tile exceeds 64 KB of LDS.
+template <bool ADJ>
+void launch_direct(DirectArgs a, int64_t images, const float* in, float* out, hipStream_t st) {
+  a.vec = a.W % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  auto grid = [&](int R) {
+    return dim3(unsigned((a.W + TX - 1) / TX), unsigned((a.H + 16 * R - 1) / (16 * R)), unsigned(images));
+  };
+  auto fits = [&](int R) {
+    const dim3 g = grid(R);
+    return int64_t(g.x) * g.y * g.z >= 512 && direct_lds(R, a.kh, a.kw) <= 65536;
+  };
+  auto go = [&](auto r_c) {
+    constexpr int R = decltype(r_c)::value;
+    hipLaunchKernelGGL((direct_mfma_kernel<R, ADJ>), grid(R), dim3(256), direct_lds(R, a.kh, a.kw), st, a, in, out);
+  };
+  if (fits(2)) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 1>{});
 }
 
 // Reverse of the direct potential, kernel side: dK[k][i][j] = sum over worlds and cells of
@@ -197,16 +248,11 @@ __global__ __launch_bounds__(256) void direct_kgrad_kernel(DirectArgs a, int64_t
 // in a fixed order, so the gradient is deterministic.  In the matrix form every LDS value feeds 4
 // multiply-adds of its lane and the pass is bound by LDS reads and MFMA issue (the one-block-per-tap
 // kernel above re-reads both images for every tap with a division and two remainders per product).
-// A row stride of 16 mod 64 floats puts the four rows n of a read in different banks.
 // Measured, 128 worlds of 128^2 with a 25 x 25 kernel: 3457 -> 59 + 5 us (2.6 GFLOP of taps: 41 TFLOP/s),
 // error against 64 bits 1.6e-6 -> 4.7e-7 (shorter chains of additions).
 constexpr int kGY = 16, kGX = 64, kGridRows = 1024, kGSets = 4;
-typedef float f4v __attribute__((ext_vector_type(4)));
 
-__host__ __device__ inline int kgrad_stride(int kw) {  // >= kGX + 4 ceil(kw / 4), 16 mod 64
-  const int need = kGX + ((kw + 3) & ~3);
-  return ((need - 16 + 63) / 64) * 64 + 16;
-}
+__host__ __device__ inline int kgrad_stride(int kw) { return bank_stride(kGX + ((kw + 3) & ~3)); }
 __host__ __device__ inline int kgrad_rows(int kh) { return kGY - 1 + ((kh + 3) & ~3); }
 constexpr int kGDU = kGX + 4;  // dU tile row: 3 columns before, one spare
 
@@ -344,7 +390,7 @@ int64_t kgrad_part_rows(const lx_rule* r, int64_t B, int kh, int kw) {
 
 DirectArgs direct_args(const lx_rule* rule, const float* A, const float* kern, int kh, int kw) {
   DirectArgs a;
-  a.A = A; a.kern = kern; a.U = nullptr;
+  a.A = A; a.kern = kern; a.vec = 0;
   a.H = rule->dims[0]; a.W = rule->dims[1]; a.C = rule->C; a.K = rule->K;
   a.kh = kh; a.kw = kw; a.ph = kh / 2; a.pw = kw / 2;
   for (int k = 0; k < LX_MAX_K; ++k) a.cin[k] = k < rule->K ? rule->cin[k] : 0;
@@ -370,9 +416,7 @@ int direct_adjoint(const char* fn, const lx_rule* rule, const float* state_d, in
   if (B * rule->C > 65535) return lx_fail(LX_ENOTSUP, "%s: B * C > 65535", fn);
   const DirectArgs a = direct_args(rule, state_d, kern_d, kh, kw);
   if (dstate_d) {
-    const size_t lds = size_t(TH + kh - 1) * size_t(tile_cols(kw)) * sizeof(float);
-    const dim3 grid(unsigned((a.W + TW - 1) / TW), unsigned((a.H + TH - 1) / TH), unsigned(B * rule->C));
-    hipLaunchKernelGGL(direct_adj_kernel, grid, dim3(256), lds, st, a, dpot_d, dstate_d);
+    launch_direct<true>(a, B * rule->C, dpot_d, dstate_d, st);
   }
   if (dkern_d && work) {
     const int64_t rows = kgrad_part_rows(rule, B, kh, kw);
@@ -439,11 +483,8 @@ extern "C" int lx_potential_direct(const lx_rule* rule, const float* state_d, in
   if (B == 0) return LX_OK;
   if (!state_d || !kern_d || !potential_d) return lx_fail(LX_EINVAL, "NULL pointer");
   if (B * rule->K > 65535) return lx_fail(LX_ENOTSUP, "lx_potential_direct: B * K > 65535");
-  DirectArgs a = direct_args(rule, state_d, kern_d, kh, kw);
-  a.U = potential_d;
-  const size_t lds = size_t(TH + kh - 1) * size_t(tile_cols(kw)) * sizeof(float);
-  const dim3 grid(unsigned((a.W + TW - 1) / TW), unsigned((a.H + TH - 1) / TH), unsigned(B * rule->K));
-  hipLaunchKernelGGL(direct_kernel, grid, dim3(256), lds, (hipStream_t)stream, a);
+  const DirectArgs a = direct_args(rule, state_d, kern_d, kh, kw);
+  launch_direct<false>(a, B * rule->K, state_d, potential_d, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? LX_OK : lx_fail(LX_EDEVICE, "direct potential launch: %s", hipGetErrorString(e));
 }

@@ -62,3 +62,42 @@ def test_kernel_gradient_of_a_state_that_is_not_finite():
     pot = core.get_potential(torch.as_tensor(A).cuda(), tK, _padding(5, 5))
     got = torch.autograd.grad(pot, tK, torch.as_tensor(dU).cuda())[0].cpu().numpy()
     assert np.all(np.isposinf(got)), got
+
+
+@pytest.mark.parametrize('N,C,maxk,H,W,kh,kw', SHAPES + [(70, 2, 1, 64, 128, 6, 11), (600, 1, 1, 20, 36, 7, 3)])
+def test_potential_and_state_gradient_match_float64(N, C, maxk, H, W, kh, kw):
+    """Every output is kh kw (times the kernels of a channel) multiply-adds of positive terms in a row:
+    a relative error of at most that many times 2^-24.  The last two shapes fill the chip (R = 2)."""
+    from leniax_amd import core
+    print('direct', (N, C, maxk, H, W, kh, kw), flush=True)
+    rng = np.random.default_rng(kh * 100 + H)
+    A = rng.uniform(size=(N, C, H, W)).astype(np.float32)
+    K = rng.uniform(size=(C * maxk, 1, kh, kw)).astype(np.float32)
+    dU = rng.uniform(size=(N, C * maxk, H, W)).astype(np.float32)
+    tA = torch.as_tensor(A).cuda().requires_grad_()
+    pot = core.get_potential(tA, torch.as_tensor(K).cuda(), _padding(kh, kw))
+    dA = torch.autograd.grad(pot, tA, torch.as_tensor(dU).cuda())[0].cpu().numpy()
+    refU, refA = np.zeros(dU.shape), np.zeros(A.shape)
+    for i in range(kh):
+        for j in range(kw):
+            move = (kh // 2 - i, kw // 2 - j)
+            for k in range(C * maxk):
+                refU[:, k] += float(K[k, 0, i, j]) * np.roll(A[:, k // maxk].astype(np.float64), move, axis=(1, 2))
+                refA[:, k // maxk] += float(K[k, 0, i, j]) * np.roll(dU[:, k].astype(np.float64),
+                                                                     (-move[0], -move[1]), axis=(1, 2))
+    errs = [float(np.max(np.abs(x - r) / r)) for x, r in ((pot.detach().cpu().numpy(), refU), (dA, refA))]
+    print('  rel err', errs)
+    assert errs[0] <= kh * kw * 2.0 ** -24 and errs[1] <= kh * kw * maxk * 2.0 ** -24
+
+
+def test_potential_of_a_state_that_is_not_finite():
+    """Exactly the cells whose window holds the infinite cell are infinite."""
+    from leniax_amd import core
+    A = np.full((1, 1, 40, 80), 0.5, np.float32)
+    A[0, 0, 7, 60] = np.inf
+    K = np.full((1, 1, 5, 6), 0.25, np.float32)
+    pot = core.get_potential(torch.as_tensor(A).cuda(), torch.as_tensor(K).cuda(), _padding(5, 6))[0, 0].cpu().numpy()
+    rows, cols = np.nonzero(np.isinf(pot))
+    assert not np.isnan(pot).any()
+    assert sorted(set(rows)) == list(range(5, 10)) and sorted(set(cols)) == list(range(58, 64)) and len(rows) == 30
+    np.testing.assert_allclose(pot[~np.isinf(pot)], 30 * 0.125, rtol=30 * 2.0 ** -24)
