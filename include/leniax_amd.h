@@ -196,6 +196,11 @@ int lx_update(const lx_rule* rule, const float* state_d, int64_t B, const void* 
               int64_t dt_bstride, float* state_out_d, float* field_d, float* potential_d, void* work_d,
               void* stream);
 
+/* lx_update with one dt for every world, by value (no device scalar to fill first). */
+int lx_update_dt(const lx_rule* rule, const float* state_d, int64_t B, const void* K_half_d, int64_t k_bstride,
+                 const float* gf_d, int64_t gf_bstride, const float* w_d, int64_t w_bstride, float dt,
+                 float* state_out_d, float* field_d, float* potential_d, void* work_d, void* stream);
+
 /* lx_update that also writes the forward spectra of the input state, rfftn(state) as
  * [B][C][dims[:-1]][dims[-1]/2+1] complex64, to state_spec_d: the recompute step of the adjoint,
  * whose kernel-spectrum gradient needs them (lx_adjoint_potential). */

@@ -64,12 +64,18 @@ def _workspace(rule, B):
     return buf
 
 
-def _dt_tensor(dt, N):
+def _dt_scalar(dt):
+    """A host scalar's float32 value, None for tensors and per-world arrays."""
     if isinstance(dt, (int, float, np.floating, np.integer)) or (isinstance(dt, np.ndarray) and dt.size == 1):
+        return float(np.float32(np.asarray(dt).reshape(-1)[0]))
+    return None
+
+
+def _dt_tensor(dt, N):
+    value = _dt_scalar(dt)
+    if value is not None:
         # a scalar: filled on the device (no pageable host copy, which would wait for the stream)
-        t = torch.full((1,), float(np.float32(np.asarray(dt).reshape(-1)[0])), dtype=torch.float32,
-                       device=engine.device())
-        return t, 0
+        return torch.full((1,), value, dtype=torch.float32, device=engine.device()), 0
     t = engine.as_device(dt).reshape(-1)
     if t.numel() not in (1, N):
         raise ValueError(f'dt must be a scalar or have one value per world ({N}), got {t.numel()}')
@@ -314,13 +320,15 @@ def fused_update(state, K, gf_params, weights, dt, tc_indices, growth_fn_t, weig
     kbs = 0 if K.shape[0] == 1 else int(Kh[0].numel())
     gf = _pad_gf(engine.as_device(gf_params), len(slots))
     w = engine.as_device(weights)
-    dt_t, dts = _dt_tensor(dt, N)
+    dt_v = _dt_scalar(dt)
+    dt_t, dts = _dt_tensor(dt, N) if dt_v is None else (None, 0)
     new = out if out is not None else torch.empty_like(A)
     dims = tuple(A.shape[2:])
     field = torch.empty((N, C) + dims, dtype=torch.float32, device=A.device) if want_field else None
     pot = torch.empty((N, len(slots)) + dims, dtype=torch.float32, device=A.device) if want_potential else None
-    _lib.call('lx_update', ctypes.byref(rule), engine.ptr(A), N, engine.ptr(Kh), kbs, engine.ptr(gf),
-              _per_world_stride(gf, N, 'gf'), engine.ptr(w), _per_world_stride(w, N, 'weights'), engine.ptr(dt_t), dts,
+    name, dt_args = ('lx_update', (engine.ptr(dt_t), dts)) if dt_v is None else ('lx_update_dt', (dt_v,))
+    _lib.call(name, ctypes.byref(rule), engine.ptr(A), N, engine.ptr(Kh), kbs, engine.ptr(gf),
+              _per_world_stride(gf, N, 'gf'), engine.ptr(w), _per_world_stride(w, N, 'weights'), *dt_args,
               engine.ptr(new), engine.ptr(field), engine.ptr(pot), engine.ptr(_workspace(rule, N)),
               engine.stream_ptr())
     return new, field, pot

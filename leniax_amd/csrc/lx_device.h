@@ -395,13 +395,14 @@ LX_DEV void twl_mulc(float2* x, const float2* twl) {
   }
 }
 
-template <int P, int TPR, bool INV>
-LX_DEV void fft_xlds(float2* x, int t, const float2* twl, float2* xch) {
+// ``mul(x)`` multiplies x[k] by the lane's twiddles (forward) or their conjugates (inverse)
+template <int P, int TPR, bool INV, class MUL>
+LX_DEV void fft_xlds_mul(float2* x, int t, MUL&& mul, float2* xch) {
   constexpr int J = P / TPR, RS = xch_row(P);
   static_assert(P % TPR == 0 && J >= 1, "fft_xlds needs P >= TPR");
   if constexpr (!INV) {
     fft_reg<P, false>(x);
-    twl_mul<P>(x, twl);
+    mul(x);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 #pragma unroll
     for (int k = 0; k < P; k += 2) {
@@ -452,9 +453,17 @@ LX_DEV void fft_xlds(float2* x, int t, const float2* twl, float2* xch) {
       x[k + 1] = make_float2(v.z, v.w);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    twl_mulc<P>(x, twl);
+    mul(x);
     fft_reg<P, true>(x);
   }
+}
+
+template <int P, int TPR, bool INV>
+LX_DEV void fft_xlds(float2* x, int t, const float2* twl, float2* xch) {
+  fft_xlds_mul<P, TPR, INV>(x, t, [&](float2* y) {
+    if constexpr (INV) twl_mulc<P>(y, twl);
+    else twl_mul<P>(y, twl);
+  }, xch);
 }
 
 // ----------------------------------------------------------------- growth functions

@@ -24,33 +24,9 @@
 #include <type_traits>
 #include <vector>
 
-#include "lx_internal.h"
+#include "lx_pass.h"
 
 namespace {
-
-// lanes per transform of the row passes: 8 from 96 points up (96 = 8 lanes x 12 points through
-// the DPP network rather than 4 x 24 through LDS: half the registers of rows_inv, 3 waves per
-// SIMD instead of 2)
-constexpr int row_tpr(int L) { return L <= 64 ? 4 : (L <= 192 ? 8 : 16); }
-// lanes per transform of the line passes: as the rows, except the plain forward and inverse
-// passes (modes 1 and 2) at 96 points, which take 4 x 24 through LDS: they stay at 4 waves per
-// SIMD there (101 and 112 VGPRs) and run 10% faster than on the network (the convolution pass,
-// at 173 VGPRs with 4 lanes, is as fast on 8)
-constexpr int line_tpr(int L, int mode) { return L == 96 && mode != 0 ? 4 : row_tpr(L); }
-
-template <int L, int T = row_tpr(L)>
-struct Lanes {
-  static constexpr int TPR = T;
-  static constexpr int P = L / TPR;                                // points per lane
-  static constexpr bool XL = P % TPR == 0;                         // cross-lane step through LDS
-  static constexpr int XRS = xch_row(P);                           // group scratch row stride
-  static constexpr int XCH = 256 * XRS;                            // scratch of a 256-thread block
-  static_assert(TPR == 4 || TPR == 8 || TPR == 16, "lane groups of 4, 8 or 16");
-  static_assert(TPR * XRS >= L + 2, "a group's scratch holds one transform plus two");
-};
-
-template <int V>
-using IntC = std::integral_constant<int, V>;
 
 bool len_ok(int n) {
   switch (n) {
@@ -137,25 +113,32 @@ int ensure_tw(hipStream_t stream) {
   return LX_OK;
 }
 
+template <int L>
+int tables_of(hipStream_t st, LxPassTables* out) {
+  static std::atomic<const float2*> tw[kMaxDevices], twl[kMaxDevices];  // set once the tables are built
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return lx_fail(LX_EDEVICE, "hipGetDevice failed or device index out of range");
+  if (!tw[dev].load(std::memory_order_acquire)) {
+    if (int rc = ensure_tw<L>(st)) return rc;
+    void *p = nullptr, *q = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_tw<L>)) != hipSuccess ||
+        hipGetSymbolAddress(&q, HIP_SYMBOL((g_twl<L, row_tpr(L)>))) != hipSuccess)
+      return lx_fail(LX_EDEVICE, "twiddle table address");
+    twl[dev].store(static_cast<const float2*>(q), std::memory_order_relaxed);
+    tw[dev].store(static_cast<const float2*>(p), std::memory_order_release);
+  }
+  out->tw = tw[dev].load(std::memory_order_acquire);
+  out->twl = twl[dev].load(std::memory_order_relaxed);
+  return LX_OK;
+}
+
 int launched(const char* what) {
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? LX_OK : lx_fail(LX_EDEVICE, "%s launch: %s", what, hipGetErrorString(e));
 }
 
 unsigned blocks_for(int64_t threads) { return unsigned((threads + 255) / 256); }
-
-// Frequency held by register e of lane t after a forward group transform: with the LDS
-// exchange e = j TPR + k2 holds (J t + j) + P k2; with the DPP network e holds e + P bitrev(t).
-template <int L, int T = row_tpr(L)>
-LX_DEV int freq_of(int t, int e) {
-  using LC = Lanes<L, T>;
-  if constexpr (LC::XL) {
-    constexpr int J = LC::P / LC::TPR;
-    return J * t + e / LC::TPR + LC::P * (e % LC::TPR);
-  } else {
-    return e + LC::P * bitrev_n(t, LC::TPR);
-  }
-}
 
 // Length-L transform over a lane group: natural order (data[TPR m + t] in x[m]) <-> the
 // frequency layout of freq_of; xch is the group's LDS scratch.
@@ -165,8 +148,6 @@ LX_DEV void fft_group(float2* x, int t, int lane, float2* xch) {
   if constexpr (LC::XL) fft_xlds<LC::P, LC::TPR, INV>(x, t, g_twl<L, T> + t * twl_row(LC::P), xch);
   else fft_lanes<LC::P, LC::TPR, INV>(x, t, lane, g_tw<L>);
 }
-
-LX_DEV void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 // XCD-aware block order.  The hardware deals a grid's workgroups to the 8 XCDs in turn (block b
 // runs on XCD b % 8 as that XCD's (b / 8)-th block); each XCD has its own L2.  The logical block
@@ -211,27 +192,6 @@ int make_geom(int ndim, const int32_t* dims, Geom& g) {
   }
   g.half = g.rows * g.WH;
   return LX_OK;
-}
-
-// ---------------------------------------------------------------- batched-run indirection
-// The kernels of lx_run's multi-pass path (LIST = true) step the worlds of a live list: slot s of
-// the list holds world list[s], slots >= *nlive are empty.  The per-step temporaries (spectra S,
-// U, the row-pair records) are indexed by slot; what persists (the state, carry, parameters,
-// spectra, statistics) by world.  World b's state after t of its steps lives in X0 (t even) or X1
-// (t odd), t = carry[b].t: worlds advance in lockstep inside a step but start at different steps.
-struct RunView {
-  const int32_t* list;
-  const int32_t* nlive;
-  const lx_carry* carry;
-  float* X0;
-  float* X1;
-  int64_t world_elems;  // C * cells floats per world
-};
-
-// the state buffer holding world b's current state
-LX_DEV float* run_state(const RunView& v, int64_t b, bool next) {
-  const bool odd = ((v.carry[b].t & 1) != 0) != next;
-  return (odd ? v.X1 : v.X0) + b * v.world_elems;
 }
 
 // ---------------------------------------------------------------- rows forward
@@ -287,47 +247,6 @@ __global__ __launch_bounds__(256) void rows_fwd_kernel(const float* __restrict__
 }
 
 // ---------------------------------------------------------------- lines along a leading axis
-struct LineArgs {
-  const float2* S;
-  float2* U;
-  const float2* Kh;
-  int64_t k_bstride;
-  int64_t nlines;      // images * A * WH
-  int WH, A;
-  int64_t a_stride, st, img_elems;
-  int C, K;            // images per world (channels) and kernels (mode 0)
-  int cin[LX_MAX_K];   // mode 0: kernel k reads channel cin[k]
-  int mode;            // 0: conv, 1: forward in place, 2: inverse S -> U
-  int conjk;           // mode 0: multiply by conj(K) (adjoint of the potential)
-  // mode 0: Kh holds real quadrants (float [world][K][L/2 + 1][WH], 2-D): the spectrum of kernel
-  // k at frequency f of a line is the real value at row min(f, L - f); k_elems: the elements (float2,
-  // or float for quadrants) of one kernel's spectrum
-  int kquad;
-  int64_t k_elems;
-  // mode 0, optional: the forward spectra of the input images, FA [img][half]
-  float2* FA;
-  // mode 0, optional: dspec[b][k] += X_k * conj(FAin[b][acc_cin[k]]) (kernel-spectrum gradient)
-  const float2* FAin;
-  float2* dspec;
-  int C_fa;
-  int acc_cin[LX_MAX_K];
-  // batched run (LIST kernels): nlines is the lines of one slot's slot_imgs images; the spectra
-  // of a slot's lines are those of world list[slot]
-  const int32_t* list;
-  const int32_t* nlive;
-  int xcd;  // blocks in XCD-contiguous order (xcd_block) or in launch order
-};
-
-LineArgs line_args() {
-  LineArgs a;
-  a.S = nullptr; a.U = nullptr; a.Kh = nullptr; a.k_bstride = 0; a.nlines = 0;
-  a.WH = 0; a.A = 1; a.a_stride = 0; a.st = 0; a.img_elems = 0; a.C = 1; a.K = 0;
-  for (int k = 0; k < LX_MAX_K; ++k) { a.cin[k] = -1; a.acc_cin[k] = 0; }
-  a.mode = 0; a.conjk = 0; a.kquad = 0; a.k_elems = 0; a.FA = nullptr; a.FAin = nullptr; a.dspec = nullptr; a.C_fa = 1;
-  a.list = nullptr; a.nlive = nullptr; a.xcd = 1;
-  return a;
-}
-
 // One launch per mode (MODE 0: conv, 1: forward in place, 2: inverse), so that each keeps
 // only its own registers.  Offsets inside an image are 32-bit; loads are issued in batches
 // of 8 (sched_barrier) so that addresses and values are not all held at once.
@@ -434,110 +353,6 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a) {
 #pragma unroll
       for (int m = 0; m < P; ++m) dst[(TPR * m + t) * st] = y[m];
     }
-  }
-}
-
-// The convolution pass of one channel and one kernel on a latency-bound grid (a few worlds): the
-// line's kernel spectrum is loaded before the forward transform, so that its latency overlaps the
-// transform instead of following it.  The same arithmetic as lines_kernel's mode 0.
-template <int L, int T, bool KQ = false>
-__global__ __launch_bounds__(256) void lines_conv1_kernel(LineArgs a) {
-  using LC = Lanes<L, T>;
-  constexpr int TPR = LC::TPR, P = LC::P;
-  __shared__ __align__(16) float2 xch_all[LC::XL ? LC::XCH : 2];
-  const int lane = threadIdx.x & 63;
-  const int t = threadIdx.x % TPR;
-  float2* xch = xch_all + (LC::XL ? (threadIdx.x / TPR) * (TPR * LC::XRS) : 0);
-  const int64_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : int64_t(blockIdx.x);
-  const int64_t lid = (blk * 256 + threadIdx.x) / TPR;
-  const bool live = lid < a.nlines;
-  const int64_t per_img = int64_t(a.A) * a.WH;
-  const int64_t img = live ? lid / per_img : 0;  // one channel: image = world
-  const int rem = live ? int(lid - img * per_img) : 0;
-  const int aa = rem / a.WH;
-  const int off = aa * int(a.a_stride) + (rem - aa * a.WH);
-  const int st = int(a.st);
-  const float2* src = a.S + img * a.img_elems + off;
-  float2 x[P], kv[P];
-#pragma unroll
-  for (int m = 0; m < P; ++m) x[m] = src[(TPR * m + t) * st];
-  if constexpr (KQ) {
-    const float* kq = reinterpret_cast<const float*>(a.Kh) + img * a.k_bstride + off;
-#pragma unroll
-    for (int e = 0; e < P; ++e) {
-      const int f = freq_of<L, T>(t, e);
-      kv[e] = make_float2(kq[(f <= L / 2 ? f : L - f) * st], 0.f);
-    }
-  } else {
-    const float2* kk = a.Kh + img * a.k_bstride + off;
-#pragma unroll
-    for (int e = 0; e < P; ++e) kv[e] = kk[freq_of<L, T>(t, e) * st];
-  }
-  fft_group<L, false, T>(x, t, lane, xch);
-  if (a.FA && live) {
-    float2* fa = a.FA + img * a.img_elems + off;
-#pragma unroll
-    for (int e = 0; e < P; ++e) fa[freq_of<L, T>(t, e) * st] = x[e];
-  }
-  const float csign = a.conjk ? -1.f : 1.f;
-#pragma unroll
-  for (int e = 0; e < P; ++e) x[e] = cmul(x[e], make_float2(kv[e].x, csign * kv[e].y));
-  fft_group<L, true, T>(x, t, lane, xch);
-  float2* dst = a.U + img * a.img_elems + off;
-  if (live) {
-#pragma unroll
-    for (int m = 0; m < P; ++m) dst[(TPR * m + t) * st] = x[m];
-  }
-}
-
-// The convolution pass of the adjoint potential with the kernel-spectrum gradient, one channel and
-// one kernel (the reverse steps of lx_adjoint_step and of a run): the line's kernel spectrum, state
-// spectrum and gradient accumulator are loaded before the forward transform, so that their latency
-// overlaps it instead of following it (the single-world gradient is bound by these chains).  The
-// same arithmetic as lines_kernel's mode 0 with dspec.
-template <int L, int T>
-__global__ __launch_bounds__(256) void lines_gradk_kernel(LineArgs a) {
-  using LC = Lanes<L, T>;
-  constexpr int TPR = LC::TPR, P = LC::P;
-  __shared__ __align__(16) float2 xch_all[LC::XL ? LC::XCH : 2];
-  const int lane = threadIdx.x & 63;
-  const int t = threadIdx.x % TPR;
-  float2* xch = xch_all + (LC::XL ? (threadIdx.x / TPR) * (TPR * LC::XRS) : 0);
-  const int64_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : int64_t(blockIdx.x);
-  const int64_t lid = (blk * 256 + threadIdx.x) / TPR;
-  const bool live = lid < a.nlines;
-  const int64_t per_img = int64_t(a.A) * a.WH;
-  const int64_t img = live ? lid / per_img : 0;  // one channel: image = world
-  const int rem = live ? int(lid - img * per_img) : 0;
-  const int aa = rem / a.WH;
-  const int off = aa * int(a.a_stride) + (rem - aa * a.WH);
-  const int st = int(a.st);
-  const float2* src = a.S + img * a.img_elems + off;
-  const float2* kk = a.Kh + img * a.k_bstride + off;
-  const float2* fa = a.FAin + img * a.img_elems + off;
-  float2* ds = a.dspec + img * a.img_elems + off;
-  float2 x[P], kv[P], fv[P], dv[P];
-#pragma unroll
-  for (int m = 0; m < P; ++m) x[m] = src[(TPR * m + t) * st];
-#pragma unroll
-  for (int e = 0; e < P; ++e) {
-    const int o = freq_of<L, T>(t, e) * st;
-    kv[e] = kk[o];
-    fv[e] = fa[o];
-    dv[e] = ds[o];
-  }
-  fft_group<L, false, T>(x, t, lane, xch);
-  const float csign = a.conjk ? -1.f : 1.f;
-#pragma unroll
-  for (int e = 0; e < P; ++e) {
-    if (live) ds[freq_of<L, T>(t, e) * st] = cadd(dv[e], cmulc(x[e], fv[e]));
-    x[e] = cmul(x[e], make_float2(kv[e].x, csign * kv[e].y));
-  }
-  fft_group<L, true, T>(x, t, lane, xch);
-  float2* dst = a.U + img * a.img_elems + off;
-  if (live) {
-#pragma unroll
-    for (int m = 0; m < P; ++m) dst[(TPR * m + t) * st] = x[m];
   }
 }
 
@@ -673,54 +488,11 @@ __global__ __launch_bounds__(256) void conv_staged_kernel(LineArgs a) {
 }
 
 // ---------------------------------------------------------------- rows inverse + field + update
-struct RowArgs {
-  const float2* U;
-  const float* A;
-  float* A_out;
-  float* field;
-  float* pot;
-  const float* gf;
-  int64_t gf_bs;
-  const float* w;
-  int64_t w_bs;
-  const float* dt;
-  int64_t dt_bs;
-  int64_t npairs;  // images * rows / 2
-  int64_t rows;    // rows per image
-  int C, K;
-  int gfk[LX_MAX_K];
-  int state_fn, average;
-  int update;      // 0: potential only
-  // selection mode: weight of kernel k in channel c is (cin[k] == c), growth is the identity and the
-  // update is A_out = A + G (no gf / w / dt reads).  Used for the potential alone, the adjoint of the
-  // potential (lambda += correlations) and the inverse real FFT.
-  int sel;
-  int cin[LX_MAX_K];
-  // statistics mode: the step's world sums of leniax/statistics.py:35-126 over each row pair's
-  // input state, field and potential, LX_PAIR_REC floats per pair at part[pair index] (sA, sG,
-  // nA, nG, nU, sAy[3], sGy[3], sAyy[3]), in the re-centred coordinates of the carried shift
-  float* part;
-  const lx_stat_carry* carry;
-  int ndim, d0, d1;  // rows = d0 d1 (d0 = 1 for 2-D worlds)
-  // batched run (LIST kernels): npairs is the pairs of one slot; state from / to rv's buffers, the
-  // carry is rv.carry; with hist_B > 0, field and pot (and cells_hist, when set) are the run's
-  // histories [max_steps][hist_B][C or K][dims], written at the world's step
-  RunView rv;
-  float* cells_hist;
-  int64_t hist_B;
-  // the reverse step's gradient scalars, summed by fin.blocks workgroups after the row pairs' (not in
-  // the statistics or LIST kernels)
-  LxAdjFinish fin;
-};
-
 // UNI: every wave's row pairs lie in one image (the host checks that the pairs per image are a
 // multiple of the pairs per wave), so the world's weights and growth parameters are the same for
 // the whole wave: the wave copies them into LDS once instead of loading them from global memory
 // in each kernel iteration, and its branches on them are uniform.
-// PF (latency-bound grids, the last worlds of a batched run): the rows of the next kernel the loop
-// transforms are loaded into registers while it transforms the current one (36 more VGPRs at 256
-// points); the same arithmetic, in the same order.
-template <int W, bool STATS, bool UNI, bool LIST = false, bool PF = false>
+template <int W, bool STATS, bool UNI, bool LIST = false>
 __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
   using LC = Lanes<W>;
   constexpr int TPR = LC::TPR, P = LC::P, WH = W / 2 + 1;
@@ -775,50 +547,6 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
   float den = 0.f;
   float nU = 0.f;  // statistics: potential cells above eps, over the kernels this channel owns
   float2 x[P];
-  constexpr int NI = (WH + TPR - 1) / TPR;  // staged points of a row per lane
-  float2 pf0[PF ? NI : 1], pf1[PF ? NI : 1];
-  uint32_t act = 0;  // PF: the kernels the loop transforms (it skips the others)
-  auto load_rows = [&](int k) {
-    const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;
-    const float2* u1 = u0 + WH;
-    const int tl = threadIdx.x % TPR;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int col = tl + TPR * i;
-      if (col < WH) {
-        pf0[i] = u0[col];
-        pf1[i] = u1[col];
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, before the transform that follows
-  };
-  // PF: the pair's input state, loaded before the transforms as well
-  float av0[PF ? P : 1], av1[PF ? P : 1];
-  if constexpr (PF) {
-    if (a.update && live) {
-      const float* Ap = LIST ? run_state(a.rv, bw, false) + (int64_t(c) * a.rows + r2) * W
-                             : a.A + (img * a.rows + r2) * int64_t(W);
-      const int tl = threadIdx.x % TPR;
-#pragma unroll
-      for (int m = 0; m < P; ++m) {
-        av0[m] = Ap[TPR * m + tl];
-        av1[m] = Ap[W + TPR * m + tl];
-      }
-    }
-    for (int k = 0; k < a.K; ++k) {
-      const float wk = a.sel ? (a.cin[k] == c ? 1.f : 0.f) : pw[c * a.K + k];
-      int owner = 0;
-      if (a.sel) {
-        owner = a.cin[k];
-      } else {
-        for (int cc = a.C - 1; cc >= 0; --cc)
-          if (pw[cc * a.K + k] != 0.f) owner = cc;
-      }
-      const bool own = owner == c;
-      if (!(wk == 0.f && !(a.pot != nullptr && own) && !(STATS && own))) act |= 1u << k;
-    }
-    if (act) load_rows(__builtin_ctz(act));
-  }
   for (int k = 0; k < a.K; ++k) {
     const float wk = a.sel ? (a.cin[k] == c ? 1.f : 0.f) : pw[c * a.K + k];
     den = add_nc(den, wk);
@@ -838,27 +566,14 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
     // stage the two rows' half spectra (coalesced), then repack them as one complex row:
     // Z[k] = A[k] + i B[k], A[k] = conj(A[W-k]) above W/2; DC and Nyquist are real
     wave_lds_fence();
-    if constexpr (PF) {
+    const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;
+    const float2* u1 = u0 + WH;
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int col = t + TPR * i;
-        if (col < WH) {
-          xch[col] = pf0[i];
-          xch[WH + col] = pf1[i];
-        }
-      }
-      const uint32_t rest = act & ~((2u << k) - 1u);
-      if (rest) load_rows(__builtin_ctz(rest));
-    } else {
-      const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;
-      const float2* u1 = u0 + WH;
-#pragma unroll
-      for (int i = 0; i < (WH + TPR - 1) / TPR; ++i) {
-        const int col = t + TPR * i;
-        if (col < WH) {
-          xch[col] = u0[col];
-          xch[WH + col] = u1[col];
-        }
+    for (int i = 0; i < (WH + TPR - 1) / TPR; ++i) {
+      const int col = t + TPR * i;
+      if (col < WH) {
+        xch[col] = u0[col];
+        xch[WH + col] = u1[col];
       }
     }
     wave_lds_fence();
@@ -926,7 +641,7 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
     }
   }
   if (!a.update || !live) return;
-  const float dtw = a.sel ? 1.f : a.dt[bw * a.dt_bs];
+  const float dtw = a.sel ? 1.f : a.dt ? a.dt[bw * a.dt_bs] : a.dt_val;
   const int64_t off = (img * a.rows + r2) * int64_t(W);
   const float* Ain = a.A + off;
   float* Aout = a.A_out + off;
@@ -940,101 +655,31 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
     fld = a.field ? a.field + hist_off : nullptr;
     chist = a.cells_hist ? a.cells_hist + hist_off : nullptr;
   }
-  // statistics: per row sums of A, A z, A z^2, G+, G+ z (z the re-centred column) and counts
-  float sAr0 = 0.f, sAr1 = 0.f, sAz = 0.f, sAzz = 0.f, sGr0 = 0.f, sGr1 = 0.f, sGz = 0.f, nA = 0.f, nG = 0.f;
-  int sh[3] = {0, 0, 0};  // carried shift reduced into [0, size) along (d0, d1, W)
-  if (STATS) {
-    auto modp = [](int v, int m) { v %= m; return v < 0 ? v + m : v; };
-    const lx_carry& cc = LIST ? a.rv.carry[bw] : a.carry[b].c;
-    if (a.ndim == 3) sh[0] = modp(cc.shift[0], a.d0);
-    sh[1] = modp(cc.shift[a.ndim - 2], a.d1);
-    sh[2] = modp(cc.shift[a.ndim - 1], W);
-  }
+  PairSums sums;  // statistics mode
+  int sh[3] = {0, 0, 0};
+  if (STATS) pair_shift(LIST ? a.rv.carry[bw] : a.carry[b].c, a.ndim, a.d0, a.d1, W, sh);
 #pragma unroll
   for (int m = 0; m < P; ++m) {
     const int col = TPR * m + t;
     float g0 = G0[m], g1 = G1[m];
     if (a.average) { g0 = (g0 / den); g1 = (g1 / den); }
     if (fld) { fld[col] = g0; fld[W + col] = g1; }
-    float v0, v1;
-    if constexpr (PF) {
-      v0 = av0[m];
-      v1 = av1[m];
-    } else {
-      v0 = Ain[col];
-      v1 = Ain[W + col];
-    }
+    const float v0 = Ain[col], v1 = Ain[W + col];
     if (LIST && chist) { chist[col] = v0; chist[W + col] = v1; }
     if (STATS) {
       int zc = col - sh[2];
       zc += zc < 0 ? W : 0;
       const float cz = float(zc - W / 2);
-      const float gp0 = g0 != g0 ? g0 : fmaxf(g0, 0.f), gp1 = g1 != g1 ? g1 : fmaxf(g1, 0.f);
-      sAr0 += v0;
-      sAr1 += v1;
-      const float vs = v0 + v1, gs2 = gp0 + gp1;
-      sAz = fmaf(vs, cz, sAz);
-      sAzz = fmaf(vs * cz, cz, sAzz);
-      sGr0 += gp0;
-      sGr1 += gp1;
-      sGz = fmaf(gs2, cz, sGz);
-      nA += (v0 > LX_EPS ? 1.f : 0.f) + (v1 > LX_EPS ? 1.f : 0.f);
-      nG += (gp0 > LX_EPS ? 1.f : 0.f) + (gp1 > LX_EPS ? 1.f : 0.f);
+      sums.add(v0, v1, g0, g1, cz);
     }
-    float n0, n1;
-    if (a.state_fn == LX_STATE_V2) {
-      n0 = add_nc(mul_nc(v0, sub_nc(1.f, dtw)), mul_nc(dtw, g0));
-      n1 = add_nc(mul_nc(v1, sub_nc(1.f, dtw)), mul_nc(dtw, g1));
-    } else {
-      n0 = add_nc(v0, mul_nc(dtw, g0));
-      n1 = add_nc(v1, mul_nc(dtw, g1));
-      if (a.state_fn == LX_STATE_V1) {
-        n0 = n0 < 0.f ? 0.f : (n0 > 1.f ? 1.f : n0);
-        n1 = n1 < 0.f ? 0.f : (n1 > 1.f ? 1.f : n1);
-      }
-    }
+    const float n0 = step_value(a.state_fn, v0, g0, dtw), n1 = step_value(a.state_fn, v1, g1, dtw);
     Aout[col] = n0;
     Aout[W + col] = n1;
   }
   if constexpr (STATS) {
-    // re-centred row coordinates of the pair's two rows: (x, y) in 3-D, y in 2-D
-    float cx[2], cy[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = int(r2) + i;
-      int x = row / a.d1, y = row - (row / a.d1) * a.d1;
-      x -= sh[0]; x += x < 0 ? a.d0 : 0;
-      y -= sh[1]; y += y < 0 ? a.d1 : 0;
-      cx[i] = float(x - a.d0 / 2);
-      cy[i] = float(y - a.d1 / 2);
-    }
-    const bool d3 = a.ndim == 3;
-    float rec[LX_PAIR_REC];
-    rec[0] = sAr0 + sAr1;
-    rec[1] = sGr0 + sGr1;
-    rec[2] = nA;
-    rec[3] = nG;
-    rec[4] = nU;
-    const float ay = fmaf(sAr0, cy[0], sAr1 * cy[1]), ayy = fmaf(sAr0 * cy[0], cy[0], sAr1 * cy[1] * cy[1]);
-    const float gy = fmaf(sGr0, cy[0], sGr1 * cy[1]);
-    const float ax = fmaf(sAr0, cx[0], sAr1 * cx[1]), axx = fmaf(sAr0 * cx[0], cx[0], sAr1 * cx[1] * cx[1]);
-    const float gx = fmaf(sGr0, cx[0], sGr1 * cx[1]);
-    rec[5] = d3 ? ax : ay;     rec[6] = d3 ? ay : sAz;   rec[7] = d3 ? sAz : 0.f;
-    rec[8] = d3 ? gx : gy;     rec[9] = d3 ? gy : sGz;   rec[10] = d3 ? sGz : 0.f;
-    rec[11] = d3 ? axx : ayy;  rec[12] = d3 ? ayy : sAzz; rec[13] = d3 ? sAzz : 0.f;
-    for (int i = 14; i < LX_PAIR_REC; ++i) rec[i] = 0.f;
-    // sum over the pair's TPR lanes (a butterfly: every lane ends with the same sums), then
-    // lane t stores fields t, t + TPR, ...
-#pragma unroll
-    for (int off2 = TPR / 2; off2 >= 1; off2 >>= 1)
-#pragma unroll
-      for (int i = 0; i < 14; ++i) rec[i] += __shfl_xor(rec[i], off2, 64);
     // the pair's index rebuilt from (img, r2), which stay live for the update, rather than pr
     // kept live over the kernel loop (two registers more at the loop's peak)
-    float* dst = a.part + (img * half_rows + (r2 >> 1)) * LX_PAIR_REC;
-#pragma unroll
-    for (int e = 0; e < LX_PAIR_REC; ++e)
-      if (e % TPR == t) dst[e] = rec[e];
+    pair_record<TPR>(sums, nU, sh, r2, a.ndim, a.d0, a.d1, t, a.part + (img * half_rows + (r2 >> 1)) * LX_PAIR_REC);
   }
 }
 
@@ -1076,18 +721,6 @@ int launch_lines_v(LineArgs la, int L, int64_t lines, LineVariant v, hipStream_t
               hipLaunchKernelGGL((conv_staged_kernel<LL, LIST, KQ>), grid, dim3(256), 0, st, la);
               return launched("conv (staged)");
             }
-          }
-          // latency-bound grids (less than two blocks per CU) only: its registers cost occupancy
-          if constexpr (!KQ) {
-            if (!LIST && la.dspec && !la.FA && la.C == 1 && la.K == 1 && la.C_fa == 1 && la.acc_cin[0] == 0 &&
-                la.cin[0] == 0 && grid.x < 512) {
-              hipLaunchKernelGGL((lines_gradk_kernel<LL, T>), grid, dim3(256), 0, st, la);
-              return launched("lines (kernel gradient)");
-            }
-          }
-          if (!LIST && !la.dspec && la.C == 1 && la.K == 1 && la.cin[0] == 0 && grid.x < 512) {
-            hipLaunchKernelGGL((lines_conv1_kernel<LL, T, KQ>), grid, dim3(256), 0, st, la);
-            return launched("lines (convolution, one kernel)");
           }
           hipLaunchKernelGGL((lines_kernel<LL, 0, LIST, T, KQ>), grid, dim3(256), 0, st, la);
           return launched("lines");
@@ -1176,6 +809,8 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
   la.k_elems = la.kquad ? int64_t(g.L[0] / 2 + 1) * g.WH : g.half;
   la.nlines = nimg * g.A[axis] * int64_t(g.WH);
   const int L = g.L[axis];
+  int taken = 0;
+  if (int rc = lx_small_conv(la, L, la.nlines, false, st, &taken); rc || taken) return rc;
   if (int rc = dispatch_len(L, [&](auto l) { return ensure_tw<decltype(l)::value>(st); })) return rc;
   // timing is safe where the pass can run again on its own inputs: a convolution into another
   // buffer with no accumulated kernel gradient, an out-of-place inverse; in-place passes are timed
@@ -1215,17 +850,14 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
 int launch_rows_inv(const Geom& g, RowArgs ra, int64_t nimg, hipStream_t st) {
   ra.rows = g.rows;
   ra.npairs = nimg * (g.rows / 2);
+  if (ra.part && ra.fin.blocks) return lx_fail(LX_EINVAL, "rows_inv: statistics and gradient sums together");
+  int taken = 0;
+  if (int rc = lx_small_rows(ra, g.W, nimg, false, st, &taken); rc || taken) return rc;
   return dispatch_len(g.W, [&](auto w) {
     constexpr int W = decltype(w)::value;
     if (int rc = ensure_tw<W>(st)) return rc;
     const dim3 grid(blocks_for(ra.npairs * Lanes<W>::TPR) + unsigned(ra.fin.blocks));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;  // waves never straddle images
-    if (ra.part && ra.fin.blocks) return lx_fail(LX_EINVAL, "rows_inv: statistics and gradient sums together");
-    if (!ra.part && grid.x < 512) {  // latency-bound: loads issued ahead of the transforms
-      if (uni) hipLaunchKernelGGL((rows_inv_kernel<W, false, true, false, true>), grid, dim3(256), 0, st, ra);
-      else hipLaunchKernelGGL((rows_inv_kernel<W, false, false, false, true>), grid, dim3(256), 0, st, ra);
-      return launched("rows_inv");
-    }
     if (ra.part) {
       if (uni) hipLaunchKernelGGL((rows_inv_kernel<W, true, true>), grid, dim3(256), 0, st, ra);
       else hipLaunchKernelGGL((rows_inv_kernel<W, true, false>), grid, dim3(256), 0, st, ra);
@@ -1240,7 +872,7 @@ int launch_rows_inv(const Geom& g, RowArgs ra, int64_t nimg, hipStream_t st) {
 RowArgs row_args(const lx_rule* rule) {
   RowArgs ra;
   ra.U = nullptr; ra.A = nullptr; ra.A_out = nullptr; ra.field = nullptr; ra.pot = nullptr;
-  ra.gf = nullptr; ra.gf_bs = 0; ra.w = nullptr; ra.w_bs = 0; ra.dt = nullptr; ra.dt_bs = 0;
+  ra.gf = nullptr; ra.gf_bs = 0; ra.w = nullptr; ra.w_bs = 0; ra.dt = nullptr; ra.dt_bs = 0; ra.dt_val = 0.f;
   ra.npairs = 0; ra.rows = 0; ra.C = rule->C; ra.K = rule->K;
   for (int k = 0; k < LX_MAX_K; ++k) {
     ra.gfk[k] = k < rule->K ? rule->gf[k] : 0;
@@ -1271,7 +903,7 @@ int fwd_leading(const Geom& g, float2* X, int64_t nimg, hipStream_t st) {
 int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, int64_t k_bs, const float* gf,
                int64_t gf_bs, const float* w, int64_t w_bs, const float* dt, int64_t dt_bs, float* A_out,
                float* field, float* pot, void* work, hipStream_t st, int sel, float2* FA = nullptr,
-               float* part = nullptr, const lx_stat_carry* carry = nullptr) {
+               float* part = nullptr, const lx_stat_carry* carry = nullptr, float dt_val = 0.f) {
   Geom g;
   if (int rc = make_geom(rule->ndim, rule->dims, g)) return rc;
   const int C = rule->C, K = rule->K;
@@ -1298,7 +930,7 @@ int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, i
   if (rc) return rc;
   RowArgs ra = row_args(rule);
   ra.U = U; ra.A = A; ra.A_out = A_out; ra.field = field; ra.pot = pot;
-  ra.gf = gf; ra.gf_bs = gf_bs; ra.w = w; ra.w_bs = w_bs; ra.dt = dt; ra.dt_bs = dt_bs;
+  ra.gf = gf; ra.gf_bs = gf_bs; ra.w = w; ra.w_bs = w_bs; ra.dt = dt; ra.dt_bs = dt_bs; ra.dt_val = dt_val;
   ra.update = A_out != nullptr; ra.sel = sel;
   ra.part = part; ra.carry = carry;
   return launch_rows_inv(g, ra, B * C, st);
@@ -1346,6 +978,10 @@ int irfft(const Geom& g, int64_t n, const float2* X, float* x, float2* work, hip
 
 }  // namespace
 
+int lx_pass_tables(int L, hipStream_t st, LxPassTables* out) {
+  return dispatch_len(L, [&](auto l) { return tables_of<decltype(l)::value>(st, out); });
+}
+
 // ====================================================================== entry points
 extern "C" int lx_workspace_size(const lx_rule* rule, int64_t B, size_t* bytes) {
   int rc = lx_check_rule(rule);
@@ -1375,6 +1011,22 @@ extern "C" int lx_update(const lx_rule* rule, const float* state_d, int64_t B, c
   if (state_out_d == state_d) return lx_fail(LX_EINVAL, "lx_update: state_out must not alias state");
   return plain_step(rule, state_d, B, K_half_d, k_bstride, gf_d, gf_bstride, w_d, w_bstride, dt_d, dt_bstride,
                     state_out_d, field_d, potential_d, work_d, (hipStream_t)stream, 0);
+}
+
+extern "C" int lx_update_dt(const lx_rule* rule, const float* state_d, int64_t B, const void* K_half_d,
+                            int64_t k_bstride, const float* gf_d, int64_t gf_bstride, const float* w_d,
+                            int64_t w_bstride, float dt, float* state_out_d, float* field_d, float* potential_d,
+                            void* work_d, void* stream) {
+  int rc = lx_check_rule(rule);
+  if (rc) return rc;
+  Geom g;
+  if ((rc = make_geom(rule->ndim, rule->dims, g))) return rc;
+  if (B < 0) return lx_fail(LX_EINVAL, "B < 0");
+  if (B == 0) return LX_OK;
+  if (!state_d || !K_half_d || !gf_d || !w_d || !state_out_d || !work_d) return lx_fail(LX_EINVAL, "NULL pointer");
+  if (state_out_d == state_d) return lx_fail(LX_EINVAL, "lx_update_dt: state_out must not alias state");
+  return plain_step(rule, state_d, B, K_half_d, k_bstride, gf_d, gf_bstride, w_d, w_bstride, nullptr, 0, state_out_d,
+                    field_d, potential_d, work_d, (hipStream_t)stream, 0, nullptr, nullptr, nullptr, dt);
 }
 
 extern "C" int lx_update_with_spectra(const lx_rule* rule, const float* state_d, int64_t B, const void* K_half_d,
@@ -1727,6 +1379,10 @@ int run_lines(const PassesRun& r, const RunView& rv, int bucket, int axis, LineA
   la.list = rv.list; la.nlive = rv.nlive;
   const int L = g.L[axis];
   const int64_t lines = la.nlines * bucket;
+  if (!tune) {
+    int taken = 0;
+    if (int rc = lx_small_conv(la, L, lines, true, st, &taken); rc || taken) return rc;
+  }
   const LineVariant v = choose_lines(la, L, lines, true, tune, st,
                                      [&](LineVariant c) { return launch_lines_v<true>(la, L, lines, c, st); });
   return tune ? LX_OK : launch_lines_v<true>(la, L, lines, v, st);
@@ -1801,14 +1457,13 @@ int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
   ra.field = a->field_hist_d; ra.pot = a->potential_hist_d; ra.cells_hist = a->cells_hist_d; ra.hist_B = a->B;
   ra.rows = g.rows;
   ra.npairs = slot_pairs;
-  rc = dispatch_len(g.W, [&](auto w) {
+  int taken = 0;
+  rc = lx_small_rows(ra, g.W, int64_t(bucket) * C, true, st, &taken);
+  if (!rc && !taken) rc = dispatch_len(g.W, [&](auto w) {
     constexpr int W = decltype(w)::value;
     const dim3 grid(blocks_for(bucket * slot_pairs * Lanes<W>::TPR));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;
-    if (grid.x < 512) {  // the bucket of the last few worlds: latency-bound
-      if (uni) hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, true>), grid, dim3(256), 0, st, ra);
-      else hipLaunchKernelGGL((rows_inv_kernel<W, true, false, true, true>), grid, dim3(256), 0, st, ra);
-    } else if (uni) {
+    if (uni) {
       hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true>), grid, dim3(256), 0, st, ra);
     } else {
       hipLaunchKernelGGL((rows_inv_kernel<W, true, false, true>), grid, dim3(256), 0, st, ra);
