@@ -657,7 +657,7 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
   }
   PairSums sums;  // statistics mode
   int sh[3] = {0, 0, 0};
-  if (STATS) pair_shift(LIST ? a.rv.carry[bw] : a.carry[b].c, a.ndim, a.d0, a.d1, W, sh);
+  if (STATS) pair_shift(LIST ? a.rv.carry[bw] : *pair_carry(a.carry, a.carry_bytes, b), a.ndim, a.d0, a.d1, W, sh);
 #pragma unroll
   for (int m = 0; m < P; ++m) {
     const int col = TPR * m + t;
@@ -879,7 +879,7 @@ RowArgs row_args(const lx_rule* rule) {
     ra.cin[k] = k < rule->K ? rule->cin[k] : -1;
   }
   ra.state_fn = rule->state_fn; ra.average = rule->average; ra.update = 0; ra.sel = 0;
-  ra.part = nullptr; ra.carry = nullptr;
+  ra.part = nullptr; ra.carry = nullptr; ra.carry_bytes = 0;
   ra.rv = RunView{nullptr, nullptr, nullptr, nullptr, nullptr, 0};
   ra.cells_hist = nullptr; ra.hist_B = 0;
   ra.fin = LxAdjFinish{};
@@ -903,7 +903,7 @@ int fwd_leading(const Geom& g, float2* X, int64_t nimg, hipStream_t st) {
 int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, int64_t k_bs, const float* gf,
                int64_t gf_bs, const float* w, int64_t w_bs, const float* dt, int64_t dt_bs, float* A_out,
                float* field, float* pot, void* work, hipStream_t st, int sel, float2* FA = nullptr,
-               float* part = nullptr, const lx_stat_carry* carry = nullptr, float dt_val = 0.f) {
+               float* part = nullptr, const void* carry = nullptr, int carry_bytes = 0, float dt_val = 0.f) {
   Geom g;
   if (int rc = make_geom(rule->ndim, rule->dims, g)) return rc;
   const int C = rule->C, K = rule->K;
@@ -932,7 +932,7 @@ int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, i
   ra.U = U; ra.A = A; ra.A_out = A_out; ra.field = field; ra.pot = pot;
   ra.gf = gf; ra.gf_bs = gf_bs; ra.w = w; ra.w_bs = w_bs; ra.dt = dt; ra.dt_bs = dt_bs; ra.dt_val = dt_val;
   ra.update = A_out != nullptr; ra.sel = sel;
-  ra.part = part; ra.carry = carry;
+  ra.part = part; ra.carry = static_cast<const char*>(carry); ra.carry_bytes = carry_bytes;
   return launch_rows_inv(g, ra, B * C, st);
 }
 
@@ -1026,7 +1026,7 @@ extern "C" int lx_update_dt(const lx_rule* rule, const float* state_d, int64_t B
   if (!state_d || !K_half_d || !gf_d || !w_d || !state_out_d || !work_d) return lx_fail(LX_EINVAL, "NULL pointer");
   if (state_out_d == state_d) return lx_fail(LX_EINVAL, "lx_update_dt: state_out must not alias state");
   return plain_step(rule, state_d, B, K_half_d, k_bstride, gf_d, gf_bstride, w_d, w_bstride, nullptr, 0, state_out_d,
-                    field_d, potential_d, work_d, (hipStream_t)stream, 0, nullptr, nullptr, nullptr, dt);
+                    field_d, potential_d, work_d, (hipStream_t)stream, 0, nullptr, nullptr, nullptr, 0, dt);
 }
 
 extern "C" int lx_update_with_spectra(const lx_rule* rule, const float* state_d, int64_t B, const void* K_half_d,
@@ -1067,7 +1067,7 @@ extern "C" int lx_step_stats(const lx_rule* rule, const float* state_d, int64_t 
   hipStream_t st = (hipStream_t)stream;
   if ((rc = plain_step(rule, state_d, B, K_half_d, k_bstride, gf_d, gf_bstride, w_d, w_bstride, dt_d, dt_bstride,
                        state_out_d, field_d, potential_d, work_d, st, 0, nullptr, part,
-                       static_cast<const lx_stat_carry*>(carry_d))))
+                       carry_d, int(sizeof(lx_stat_carry)))))
     return rc;
   return lx_pair_stats_launch(rule, part, B, pairs, R, T, carry_d, stats_d, st);
 }
@@ -1267,7 +1267,7 @@ __global__ void run_start_kernel(RunCtl c, int64_t B, int slots) {
 
 struct RunStatArgs {
   RunCtl c;
-  int par;             // the list this step reads
+  int par;             // the list this step reads (-1: slot b is world b, nothing is retired)
   const float* part;   // [slots][C][pairs] row-pair records
   int64_t pairs;
   int C, ndim;
@@ -1284,9 +1284,12 @@ struct RunStatArgs {
 // carry, the heuristics and the stop decision (a stop, or the world's last step, frees the slot).
 __global__ __launch_bounds__(kPairThreads) void run_stats_kernel(RunStatArgs a) {
   const int slot = blockIdx.x;
-  const int32_t* list = a.par ? a.c.list1 : a.c.list0;
-  if (slot >= a.c.nlive[a.par]) return;  // block-uniform
-  const int64_t b = list[slot];
+  int64_t b = slot;
+  if (a.par >= 0) {
+    const int32_t* list = a.par ? a.c.list1 : a.c.list0;
+    if (slot >= a.c.nlive[a.par]) return;  // block-uniform
+    b = list[slot];
+  }
   const lx_sums s = lx_block_pair_sums(a.part + int64_t(slot) * a.C * a.pairs * LX_PAIR_REC, a.C, a.pairs);
   if (threadIdx.x != 0) return;
   lx_carry cr = a.c.carry[b];
@@ -1295,7 +1298,7 @@ __global__ __launch_bounds__(kPairThreads) void run_stats_kernel(RunStatArgs a) 
                                    a.cells_total, out);
   const int done = stop || cr.t >= a.max_steps;
   a.c.carry[b] = cr;
-  a.c.done[slot] = done;
+  if (a.par >= 0) a.c.done[slot] = done;
   if (done) {
     if (a.n_out) a.n_out[b] = cr.n;
     if (a.steps_out) a.steps_out[b] = cr.t;
@@ -1414,6 +1417,21 @@ int tune_run_lines(const PassesRun& r, int bucket, hipStream_t st) {
   return rc;
 }
 
+RunStatArgs run_stat_args(const PassesRun& r, int par) {
+  const lx_rule* rule = r.rule;
+  const lx_run_args* a = r.a;
+  const Geom& g = r.g;
+  const int C = rule->C;
+  RunStatArgs sa;
+  sa.c = r.ctl; sa.par = par; sa.part = r.part; sa.pairs = g.rows / 2; sa.C = C; sa.ndim = rule->ndim;
+  for (int i = 0; i < 3; ++i) sa.dims[i] = i < rule->ndim ? rule->dims[i] : 1;
+  sa.R2 = (float)((double)a->R * (double)a->R); sa.R = a->R; sa.dt = (float)(1.0 / (double)a->T);
+  sa.stop_policy = a->stop_policy; sa.min_steps = a->min_steps; sa.max_steps = a->max_steps;
+  sa.cells_total = float(cells_per_world(rule) * C);
+  sa.stats = a->stats_d; sa.n_out = a->n_d; sa.steps_out = a->steps_d;
+  return sa;
+}
+
 // one step over the live list of parity `par`, grids sized for `bucket` slots
 int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
   const lx_rule* rule = r.rule;
@@ -1471,19 +1489,48 @@ int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
     return launched("rows_inv (run)");
   });
   if (rc) return rc;
-  RunStatArgs sa;
-  sa.c = r.ctl; sa.par = par; sa.part = r.part; sa.pairs = g.rows / 2; sa.C = C; sa.ndim = rule->ndim;
-  for (int i = 0; i < 3; ++i) sa.dims[i] = i < rule->ndim ? rule->dims[i] : 1;
-  sa.R2 = (float)((double)a->R * (double)a->R); sa.R = a->R; sa.dt = (float)(1.0 / (double)a->T);
-  sa.stop_policy = a->stop_policy; sa.min_steps = a->min_steps; sa.max_steps = a->max_steps;
-  sa.cells_total = float(cells_per_world(rule) * C);
-  sa.stats = a->stats_d; sa.n_out = a->n_d; sa.steps_out = a->steps_d;
+  const RunStatArgs sa = run_stat_args(r, par);
   hipLaunchKernelGGL(run_stats_kernel, dim3(unsigned(bucket)), dim3(kPairThreads), 0, st, sa);
   if (bucket <= 64)
     hipLaunchKernelGGL(run_control_kernel<64>, dim3(1), dim3(64), 0, st, r.ctl, par, r.slots, a->B);
   else
     hipLaunchKernelGGL(run_control_kernel<kCtlThreads>, dim3(1), dim3(kCtlThreads), 0, st, r.ctl, par, r.slots, a->B);
   return launched("run statistics / control");
+}
+
+// A run that retires no world before its last step and has every world in flight: the steps are enqueued
+// as they are, without a live list, graphs or reads of the live count.  (A graph of 8 or 32 steps was
+// captured and instantiated per call and one replay more than needed was launched: 10 steps of 64 worlds
+// launched 24.)  World b's states alternate between X1 and cells_d so that the last step writes
+// cells_d; with a history, step t reads frame t and writes frame t + 1.
+int run_every_step(const PassesRun& r, float* X1, hipStream_t st) {
+  const lx_rule* rule = r.rule;
+  const lx_run_args* a = r.a;
+  const int64_t B = a->B, elems = B * rule->C * cells_per_world(rule), pots = B * rule->K * cells_per_world(rule);
+  const float* cur = a->cells0_d;
+  float* first = a->cells_hist_d;  // where the initial states are needed as well
+  if (!first && a->cells0_d == a->cells_d && a->max_steps % 2) first = X1;  // the first step would write its input
+  if (first) {
+    if (hipMemcpyAsync(first, a->cells0_d, size_t(elems) * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess)
+      return lx_fail(LX_EDEVICE, "lx_run: copy of the initial states failed");
+    cur = first;
+  }
+  const RunStatArgs sa = run_stat_args(r, -1);
+  for (int t = 0; t < a->max_steps; ++t) {
+    const bool last = t + 1 == a->max_steps;
+    float* next = last ? a->cells_d
+                  : a->cells_hist_d ? a->cells_hist_d + (t + 1) * elems
+                                    : ((a->max_steps - 1 - t) % 2 ? X1 : a->cells_d);
+    if (int rc = plain_step(rule, cur, B, a->K_half_d, a->k_bstride, a->gf_d, a->gf_bstride, a->w_d, a->w_bstride,
+                            a->dt_d, a->dt_bstride, next, a->field_hist_d ? a->field_hist_d + t * elems : nullptr,
+                            a->potential_hist_d ? a->potential_hist_d + t * pots : nullptr, r.S, st, 0, nullptr,
+                            r.part, r.ctl.carry, int(sizeof(lx_carry))))
+      return rc;
+    hipLaunchKernelGGL(run_stats_kernel, dim3(unsigned(B)), dim3(kPairThreads), 0, st, sa);
+    if (int rc = launched("run statistics")) return rc;
+    cur = next;
+  }
+  return LX_OK;
 }
 
 // twiddle tables of every length the step uses, built before a capture starts
@@ -1595,6 +1642,15 @@ int lx_passes_run(const lx_rule* rule, const lx_run_args* a, hipStream_t st) {
     r.rv[p] = RunView{p ? r.ctl.list1 : r.ctl.list0, r.ctl.nlive + p, r.ctl.carry, X0, X1, elems};
   int rc = warm_tables(r.g, st);
   if (rc) return rc;
+  if (a->stop_policy == LX_STOP_NONE && a->B == cap) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+      return lx_fail(LX_EDEVICE, "lx_run: the multi-pass run cannot be captured");
+    hipLaunchKernelGGL(run_start_kernel, dim3(std::min(blocks_for(a->B), 4096u)), dim3(256), 0, st, r.ctl, a->B,
+                       r.slots);
+    if ((rc = launched("run start"))) return rc;
+    return run_every_step(r, X1, st);
+  }
   if (a->cells_d != a->cells0_d &&
       hipMemcpyAsync(a->cells_d, a->cells0_d, size_t(a->B * elems) * sizeof(float), hipMemcpyDeviceToDevice, st) !=
           hipSuccess)

@@ -137,7 +137,8 @@ struct RowArgs {
   // input state, field and potential, LX_PAIR_REC floats per pair at part[pair index] (sA, sG,
   // nA, nG, nU, sAy[3], sGy[3], sAyy[3]), in the re-centred coordinates of the carried shift
   float* part;
-  const lx_stat_carry* carry;
+  const char* carry;  // world b's lx_carry at carry + b carry_bytes
+  int carry_bytes;
   int ndim, d0, d1;  // rows = d0 d1 (d0 = 1 for 2-D worlds)
   // batched run (LIST kernels): npairs is the pairs of one slot; state from / to rv's buffers, the
   // carry is rv.carry; with hist_B > 0, field and pot (and cells_hist, when set) are the run's
@@ -177,6 +178,10 @@ struct PairSums {
     nG += (gp0 > LX_EPS ? 1.f : 0.f) + (gp1 > LX_EPS ? 1.f : 0.f);
   }
 };
+
+LX_DEV const lx_carry* pair_carry(const char* carry, int bytes, int64_t b) {
+  return reinterpret_cast<const lx_carry*>(carry + b * bytes);
+}
 
 // the carried shift reduced into [0, size) along (d0, d1, W)
 LX_DEV void pair_shift(const lx_carry& cc, int ndim, int d0, int d1, int W, int (&sh)[3]) {

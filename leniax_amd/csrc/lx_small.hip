@@ -176,7 +176,8 @@ struct SmallRows {
   LxAdjFinish fin;
   // statistics, LIST
   float* part;
-  const lx_stat_carry* carry;
+  const char* carry;
+  int carry_bytes;
   int ndim, d0, d1;
   RunView rv;
   float* cells_hist;
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
       int64_t r2;
       const int b = world(q, r2);
       int sh[3];
-      pair_shift(LIST ? a.rv.carry[a.rv.list[b]] : a.carry[b].c, a.ndim, a.d0, a.d1, W, sh);
+      pair_shift(LIST ? a.rv.carry[a.rv.list[b]] : *pair_carry(a.carry, a.carry_bytes, b), a.ndim, a.d0, a.d1, W, sh);
       const float* x = vg + pc * 4 * W;
       PairSums sums;
 #pragma unroll
@@ -542,7 +543,7 @@ int lx_small_rows(const RowArgs& a, int W, int64_t images, bool list, hipStream_
   r.npairs = int(a.npairs / C); r.half_rows = int(a.rows / 2); r.C = C; r.K = K; r.RP = RP;
   r.state_fn = a.state_fn; r.average = a.average; r.update = a.update; r.sel = a.sel;
   r.fin = a.fin; r.fin_blocks = 0;
-  r.part = a.part; r.carry = a.carry; r.ndim = a.ndim; r.d0 = a.d0; r.d1 = a.d1; r.rv = a.rv;
+  r.part = a.part; r.carry = a.carry; r.carry_bytes = a.carry_bytes; r.ndim = a.ndim; r.d0 = a.d0; r.d1 = a.d1; r.rv = a.rv;
   r.cells_hist = a.cells_hist; r.hist_B = a.hist_B;
   if (a.fin.blocks) {  // one wave per gradient element
     const int64_t nout = (a.fin.g_gf ? (a.fin.gf_bs ? a.fin.B : 1) * 2 : 0) +
