@@ -170,7 +170,7 @@ extern "C" int lx_grad_run_backward(const lx_rule* rule, const lx_grad_run_args*
   LxAdj11 ac;
   if (chain && (rc = lx_adj11_init(rule, a->B, a->gf_d, a->gf_bstride, a->w_d, a->w_bstride, a->dt_d,
                                    a->dt_bstride, a->K_half_d, a->k_bstride, a->ste, lam, a->grad_gf_d,
-                                   a->grad_w_d, a->grad_dt_d, work, adj_work, stream, &ac)))
+                                   a->grad_w_d, a->grad_dt_d, work, adj_work, stream, sU, sA, &ac)))
     return rc;
   for (int seg = l.nckpt - 1; seg >= 0; --seg) {
     const int t0 = seg * c, L = std::min(c, a->steps - t0);

@@ -9,7 +9,8 @@
 //              growth g_k, weighted sum into G_c, then the update
 //
 //   2-D [H][W]:    rows_fwd, lines(H, conv), rows_inv                            (3 passes)
-//   3-D [D][H][W]: rows_fwd, lines(H, fwd), lines(D, conv), lines(H, inv), rows_inv  (5 passes)
+//   3-D [D][H][W]: rows_fwd, lines(H, fwd), lines(D, conv), lines(H, inv), rows_inv  (5 passes; planes of
+//                  32 to 128 points a side take the rows and the lines along H together, lx_plane.hip)
 //
 // Transform lengths: 2^k in [16, 512] and 3 * 2^k in [48, 384].  A length-L transform is
 // spread over a group of TPR lanes of one wave (P = L / TPR points per lane): an in-register
@@ -20,6 +21,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <initializer_list>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -149,6 +151,14 @@ LX_DEV void fft_group(float2* x, int t, int lane, float2* xch) {
   else fft_lanes<LC::P, LC::TPR, INV>(x, t, lane, g_tw<L>);
 }
 
+// The same over the strided lane groups of the line passes.
+template <int L, bool INV, int T>
+LX_DEV void fft_group_strided(float2* x, int t, int lane, float2* xch) {
+  using LC = Lanes<L, T>;
+  if constexpr (LC::XL) fft_xlds<LC::P, LC::TPR, INV>(x, t, g_twl<L, T> + t * twl_row(LC::P), xch);
+  else fft_strided<LC::P, LC::TPR, INV>(x, t, lane, g_tw<L>);
+}
+
 // XCD-aware block order.  The hardware deals a grid's workgroups to the 8 XCDs in turn (block b
 // runs on XCD b % 8 as that XCD's (b / 8)-th block); each XCD has its own L2.  The logical block
 // of b is chosen so that every XCD runs one contiguous range of logical blocks: neighbouring
@@ -256,12 +266,14 @@ template <int L, int MODE, bool LIST = false, int T = line_tpr(L, MODE), bool KQ
 __global__ __launch_bounds__(256) void lines_kernel(LineArgs a) {
   using LC = Lanes<L, T>;
   constexpr int TPR = LC::TPR, P = LC::P;
-  __shared__ __align__(16) float2 xch_all[LC::XL ? LC::XCH : 2];
+  using SG = Strided<TPR>;
+  __shared__ __align__(16) float2 xch_all[LC::XL ? 256 / TPR * strided_scratch<L, TPR>() : 2];
   const int lane = threadIdx.x & 63;
-  const int t = threadIdx.x % TPR;
-  float2* xch = xch_all + (LC::XL ? (threadIdx.x / TPR) * (TPR * LC::XRS) : 0);
+  const int t = SG::point(lane);
+  const int line = (threadIdx.x >> 6) * SG::G + SG::line(lane);  // of the block's
+  float2* xch = xch_all + (LC::XL ? line * strided_scratch<L, TPR>() : 0);
   const int64_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : int64_t(blockIdx.x);
-  const int64_t lid = (blk * 256 + threadIdx.x) / TPR;
+  const int64_t lid = blk * (256 / TPR) + line;
   int64_t nlines = a.nlines;
   if constexpr (LIST) {
     nlines *= *a.nlive;
@@ -285,7 +297,7 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a) {
       y[e] = src[freq_of<L, TPR>(t, e) * st];
       if ((e & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
-    fft_group<L, true, TPR>(y, t, lane, xch);
+    fft_group_strided<L, true, TPR>(y, t, lane, xch);
     float2* dst = a.U + img * a.img_elems + off;
     if (live) {
 #pragma unroll
@@ -298,7 +310,7 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a) {
     x[m] = src[(TPR * m + t) * st];
     if ((m & 7) == 7) __builtin_amdgcn_sched_barrier(0);
   }
-  fft_group<L, false, TPR>(x, t, lane, xch);
+  fft_group_strided<L, false, TPR>(x, t, lane, xch);
   if constexpr (MODE == 1) {  // forward only, in place
     float2* dst = const_cast<float2*>(src);
     if (live) {
@@ -317,7 +329,7 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a) {
     if (a.cin[k] != c) continue;
     // an opaque copy of the lane index: the per-kernel addresses and twiddle loads are then
     // recomputed in each iteration instead of being hoisted out of the loop and kept live
-    int t = threadIdx.x % TPR;
+    int t = SG::point(threadIdx.x & 63);
     __asm__ volatile("" : "+v"(t));
     if (a.dspec && live) {
       const float2* fa = a.FAin + (b * a.C_fa + a.acc_cin[k]) * a.img_elems + off;
@@ -347,7 +359,7 @@ __global__ __launch_bounds__(256) void lines_kernel(LineArgs a) {
         if ((e & 7) == 7) __builtin_amdgcn_sched_barrier(0);
       }
     }
-    fft_group<L, true, TPR>(y, t, lane, xch);
+    fft_group_strided<L, true, TPR>(y, t, lane, xch);
     float2* dst = a.U + (b * a.K + k) * a.img_elems + off;
     if (live) {
 #pragma unroll
@@ -811,6 +823,7 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
   const int L = g.L[axis];
   int taken = 0;
   if (int rc = lx_small_conv(la, L, la.nlines, false, st, &taken); rc || taken) return rc;
+  if (int rc = lx_shared_conv(la, L, nimg, st, &taken); rc || taken) return rc;
   if (int rc = dispatch_len(L, [&](auto l) { return ensure_tw<decltype(l)::value>(st); })) return rc;
   // timing is safe where the pass can run again on its own inputs: a convolution into another
   // buffer with no accumulated kernel gradient, an out-of-place inverse; in-place passes are timed
@@ -889,14 +902,44 @@ RowArgs row_args(const lx_rule* rule) {
   return ra;
 }
 
-// forward transform of every image along the leading axes (after rows_fwd), in place
-int fwd_leading(const Geom& g, float2* X, int64_t nimg, hipStream_t st) {
-  for (int ax = g.naxes - 1; ax >= 0; --ax) {
+// Whether a 3-D pass takes the plane kernels: their sides, and arrays that start on 16 bytes.
+bool takes_planes(const Geom& g, std::initializer_list<const void*> arrays) {
+  if (g.naxes != 2 || !lx_plane_takes(g.L[1], g.W)) return false;
+  for (const void* p : arrays)
+    if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+  return true;
+}
+
+// forward transform of real images along every axis but the convolution axis
+int fwd_inner(const Geom& g, const float* A, float2* S, int64_t nimg, hipStream_t st) {
+  if (takes_planes(g, {A})) return lx_plane_fwd(g.L[1], g.W, A, S, nimg * g.L[0], st);
+  if (int rc = launch_rows_fwd(g, A, S, nimg, st)) return rc;
+  if (g.naxes == 1) return LX_OK;
+  LineArgs la = line_args();
+  la.S = S; la.mode = 1;
+  return launch_lines(g, 1, la, nimg, st);
+}
+
+// forward transform of real images along every axis
+int fwd_all(const Geom& g, const float* A, float2* X, int64_t nimg, hipStream_t st) {
+  if (int rc = fwd_inner(g, A, X, nimg, st)) return rc;
+  LineArgs la = line_args();
+  la.S = X; la.mode = 1;
+  return launch_lines(g, 0, la, nimg, st);
+}
+
+// inverse transform of nk images of ra.U (in place) along every axis but the convolution axis, then what ra
+// asks for, over nimg images
+int inv_inner(const Geom& g, RowArgs ra, int64_t nk, int64_t nimg, hipStream_t st) {
+  ra.rows = g.rows;
+  if (!ra.part && takes_planes(g, {ra.A, ra.A_out, ra.field, ra.pot}))
+    return lx_plane_inv(ra, g.L[0], g.L[1], g.W, nimg, st);
+  if (g.naxes == 2) {
     LineArgs la = line_args();
-    la.S = X; la.mode = 1;
-    if (int rc = launch_lines(g, ax, la, nimg, st)) return rc;
+    la.S = ra.U; la.U = const_cast<float2*>(ra.U); la.mode = 2;
+    if (int rc = launch_lines(g, 1, la, nk, st)) return rc;
   }
-  return LX_OK;
+  return launch_rows_inv(g, ra, nimg, st);
 }
 
 // One leniax step (or, with sel, the potential alone).  A: [B][C][dims]; work: S then U.
@@ -909,12 +952,7 @@ int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, i
   const int C = rule->C, K = rule->K;
   float2* S = static_cast<float2*>(work);
   float2* U = S + B * C * g.half;
-  int rc = launch_rows_fwd(g, A, S, B * C, st);
-  if (!rc && g.naxes == 2) {  // forward along H
-    LineArgs la = line_args();
-    la.S = S; la.mode = 1;
-    rc = launch_lines(g, 1, la, B * C, st);
-  }
+  int rc = fwd_inner(g, A, S, B * C, st);
   if (!rc) {  // the convolution axis
     LineArgs la = line_args();
     la.S = S; la.U = U; la.Kh = static_cast<const float2*>(Kh); la.k_bstride = k_bs; la.C = C; la.K = K;
@@ -922,18 +960,13 @@ int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, i
     for (int k = 0; k < LX_MAX_K; ++k) la.cin[k] = k < K ? rule->cin[k] : -1;
     rc = launch_lines(g, 0, la, B * C, st);
   }
-  if (!rc && g.naxes == 2) {  // inverse along H, in place
-    LineArgs la = line_args();
-    la.S = U; la.U = U; la.mode = 2;
-    rc = launch_lines(g, 1, la, B * K, st);
-  }
   if (rc) return rc;
   RowArgs ra = row_args(rule);
   ra.U = U; ra.A = A; ra.A_out = A_out; ra.field = field; ra.pot = pot;
   ra.gf = gf; ra.gf_bs = gf_bs; ra.w = w; ra.w_bs = w_bs; ra.dt = dt; ra.dt_bs = dt_bs; ra.dt_val = dt_val;
   ra.update = A_out != nullptr; ra.sel = sel;
   ra.part = part; ra.carry = static_cast<const char*>(carry); ra.carry_bytes = carry_bytes;
-  return launch_rows_inv(g, ra, B * C, st);
+  return inv_inner(g, ra, B * K, B * C, st);
 }
 
 // full spectrum from the half spectrum of a real array (Hermitian extension), times scale
@@ -964,16 +997,14 @@ int half_to_full(const Geom& g, int64_t n, const float2* half, float2* full, flo
 
 // numpy.fft.irfftn (scaled by 1 / prod(dims)) of n half spectra; X untouched; work: n * half
 int irfft(const Geom& g, int64_t n, const float2* X, float* x, float2* work, hipStream_t st) {
-  for (int ax = 0; ax < g.naxes; ++ax) {
-    LineArgs la = line_args();
-    la.S = ax == 0 ? X : work; la.U = work; la.mode = 2;
-    if (int rc = launch_lines(g, ax, la, n, st)) return rc;
-  }
+  LineArgs la = line_args();
+  la.S = X; la.U = work; la.mode = 2;
+  if (int rc = launch_lines(g, 0, la, n, st)) return rc;
   lx_rule one{};
   one.ndim = g.ndim; one.C = 1; one.K = 1; one.cin[0] = 0;
   RowArgs ra = row_args(&one);
   ra.U = work; ra.pot = x; ra.sel = 1;
-  return launch_rows_inv(g, ra, n, st);
+  return inv_inner(g, ra, n, n, st);
 }
 
 }  // namespace
@@ -1094,8 +1125,7 @@ extern "C" int lx_rfft2(int32_t ndim, const int32_t* dims, int64_t n, const floa
   if (!x_d || !X_d) return lx_fail(LX_EINVAL, "NULL pointer");
   hipStream_t st = (hipStream_t)stream;
   float2* X = static_cast<float2*>(X_d);
-  if (int rc = launch_rows_fwd(g, x_d, X, n, st)) return rc;
-  return fwd_leading(g, X, n, st);
+  return fwd_all(g, x_d, X, n, st);
 }
 
 extern "C" int lx_irfft2(int32_t ndim, const int32_t* dims, int64_t n, const void* X_d, float* x_d, void* work_d,
@@ -1128,8 +1158,7 @@ extern "C" int lx_kernel_spectrum(int32_t ndim, const int32_t* dims, int64_t n, 
   if (!k_d || !K_full_d || !work_d) return lx_fail(LX_EINVAL, "NULL pointer");
   hipStream_t st = (hipStream_t)stream;
   float2* work = static_cast<float2*>(work_d);
-  if (int rc = launch_rows_fwd(g, k_d, work, n, st)) return rc;
-  if (int rc = fwd_leading(g, work, n, st)) return rc;
+  if (int rc = fwd_all(g, k_d, work, n, st)) return rc;
   return half_to_full(g, n, work, static_cast<float2*>(K_full_d), 1.f, st);
 }
 
@@ -1150,12 +1179,7 @@ extern "C" int lx_adjoint_potential(const lx_rule* rule, int64_t B, const void* 
   const int K = rule->K;
   float2* X = static_cast<float2*>(work_d);
   // the K gradient images of a world are transformed as K "channels", kernel k on image k
-  if ((rc = launch_rows_fwd(g, dpot_d, X, B * K, st))) return rc;
-  if (g.naxes == 2) {
-    LineArgs la = line_args();
-    la.S = X; la.mode = 1;
-    if ((rc = launch_lines(g, 1, la, B * K, st))) return rc;
-  }
+  if ((rc = fwd_inner(g, dpot_d, X, B * K, st))) return rc;
   {
     LineArgs la = line_args();
     la.S = X; la.U = X;  // each line is read whole before it is written back
@@ -1169,15 +1193,10 @@ extern "C" int lx_adjoint_potential(const lx_rule* rule, int64_t B, const void* 
     la.C_fa = rule->C;
     if ((rc = launch_lines(g, 0, la, B * K, st))) return rc;
   }
-  if (g.naxes == 2) {
-    LineArgs la = line_args();
-    la.S = X; la.U = X; la.mode = 2;
-    if ((rc = launch_lines(g, 1, la, B * K, st))) return rc;
-  }
   RowArgs ra = row_args(rule);
   ra.U = X; ra.A = lambda_d; ra.A_out = lambda_d;  // lambda_c += sum over kernels fed by c (in place, per element)
   ra.update = 1; ra.sel = 1; ra.average = 0; ra.state_fn = LX_STATE_SIMPLE;
-  return launch_rows_inv(g, ra, B * rule->C, st);
+  return inv_inner(g, ra, B * K, B * rule->C, st);
 }
 
 // ====================================================================== lx_run, multi-pass path
@@ -1892,7 +1911,7 @@ __global__ __launch_bounds__(256) void rows_fwd_adj_kernel(AdjRowArgs a) {
 int lx_adj11_init(const lx_rule* rule, int64_t B, const float* gf_d, int64_t gf_bstride, const float* w_d,
                   int64_t w_bstride, const float* dt_d, int64_t dt_bstride, const void* K_half_d, int64_t k_bstride,
                   int32_t ste, float* lambda_d, float* grad_gf_d, float* grad_w_d, float* grad_dt_d, void* work_d,
-                  void* adj_work_d, void* stream, LxAdj11* c) {
+                  void* adj_work_d, void* stream, const float* U, const float* A, LxAdj11* c) {
   Geom g;
   if (int rc = make_geom(rule->ndim, rule->dims, g)) return rc;
   if (!(rule->C == 1 && rule->K == 1) || B < 1 || B > 65535)
@@ -1903,8 +1922,9 @@ int lx_adj11_init(const lx_rule* rule, int64_t B, const float* gf_d, int64_t gf_
   c->lam = lambda_d; c->g_gf = grad_gf_d; c->g_w = grad_w_d; c->g_dt = grad_dt_d;
   c->X = work_d;
   c->part = lx_adj_work_11(rule, B, adj_work_d);
+  c->planes = takes_planes(g, {lambda_d, U, A});
   const int64_t pairs_per_block = 256 / lx_row_tpr(g.W);
-  c->bpw = int((g.rows / 2 + pairs_per_block - 1) / pairs_per_block);
+  c->bpw = c->planes ? int(g.L[0]) : int((g.rows / 2 + pairs_per_block - 1) / pairs_per_block);
   return LX_OK;
 }
 
@@ -1922,6 +1942,13 @@ int lx_adj11_rows(const LxAdj11& c, const float* U, const float* A, bool bridge,
   ar.accumulate = accumulate ? 1 : 0;
   ar.Sin = X;
   ar.inv_n = 1.f / float(g.rows * g.W);
+  if (c.planes) {
+    LxPlaneAdj pa;
+    pa.X = X; pa.U = U; pa.lam = c.lam; pa.A = A; pa.part = c.part; pa.gf = c.gf; pa.w = c.w; pa.dt = c.dt;
+    pa.gf_bs = c.gf_bs; pa.w_bs = c.w_bs; pa.dt_bs = c.dt_bs; pa.kind = c.rule->gf[0];
+    pa.state_fn = c.rule->state_fn; pa.ste = c.ste != 0; pa.average = c.rule->average; pa.accumulate = accumulate;
+    return lx_plane_adj(pa, g.L[0], g.L[1], g.W, c.B, bridge, st);
+  }
   return dispatch_len(g.W, [&](auto wc) {
     constexpr int W = decltype(wc)::value;
     if (int r2 = ensure_tw<W>(st)) return r2;
@@ -1951,7 +1978,7 @@ int lx_adj11_lines(const LxAdj11& c, const void* state_spec_d, void* dspec_d) {
   if (rc) return rc;
   hipStream_t st = (hipStream_t)c.stream;
   float2* X = static_cast<float2*>(c.X);
-  if (g.naxes == 2) {
+  if (g.naxes == 2 && !c.planes) {
     LineArgs la = line_args();
     la.S = X; la.mode = 1;
     if ((rc = launch_lines(g, 1, la, c.B, st))) return rc;
@@ -1966,7 +1993,7 @@ int lx_adj11_lines(const LxAdj11& c, const void* state_spec_d, void* dspec_d) {
     la.C_fa = 1;
     if ((rc = launch_lines(g, 0, la, c.B, st))) return rc;
   }
-  if (g.naxes == 2) {
+  if (g.naxes == 2 && !c.planes) {
     LineArgs la = line_args();
     la.S = X; la.U = X; la.mode = 2;
     if ((rc = launch_lines(g, 1, la, c.B, st))) return rc;
@@ -1990,6 +2017,7 @@ int lx_adj11_last(const LxAdj11& c, bool finish) {
                          (c.g_dt ? (c.dt_bs ? c.B : 1) : 0);
     f.blocks = int((nout + 3) / 4);
   }
+  if (c.planes) return lx_plane_inv(ra, g.L[0], g.L[1], g.W, c.B, (hipStream_t)c.stream);
   return launch_rows_inv(g, ra, c.B, (hipStream_t)c.stream);
 }
 
@@ -2023,7 +2051,7 @@ extern "C" int lx_adjoint_step(const lx_rule* rule, int64_t B, const float* stat
   }
   LxAdj11 c;
   if ((rc = lx_adj11_init(rule, B, gf_d, gf_bstride, w_d, w_bstride, dt_d, dt_bstride, K_half_d, k_bstride, ste,
-                          lambda_d, grad_gf_d, grad_w_d, grad_dt_d, work_d, adj_work_d, stream, &c)))
+                          lambda_d, grad_gf_d, grad_w_d, grad_dt_d, work_d, adj_work_d, stream, potential_d, state_d, &c)))
     return rc;
   if ((rc = lx_adj11_rows(c, potential_d, state_d, false, false))) return rc;
   if ((rc = lx_adj11_lines(c, state_spec_d, dspec_d))) return rc;

@@ -367,11 +367,12 @@ struct LxAdj11 {
   void* X;
   float* part;
   int bpw;  // row-pass blocks per world (partial-sum rows per world)
+  bool planes;  // 3-D: the row passes and the lines along H as plane kernels (lx_plane.hip)
 };
 int lx_adj11_init(const lx_rule* rule, int64_t B, const float* gf_d, int64_t gf_bstride, const float* w_d,
                   int64_t w_bstride, const float* dt_d, int64_t dt_bstride, const void* K_half_d, int64_t k_bstride,
                   int32_t ste, float* lambda_d, float* grad_gf_d, float* grad_w_d, float* grad_dt_d, void* work_d,
-                  void* adj_work_d, void* stream, LxAdj11* c);
+                  void* adj_work_d, void* stream, const float* U, const float* A, LxAdj11* c);
 int lx_adj11_rows(const LxAdj11& c, const float* U, const float* A, bool bridge, bool accumulate);
 int lx_adj11_lines(const LxAdj11& c, const void* state_spec_d, void* dspec_d);
 int lx_adj11_last(const LxAdj11& c, bool finish);

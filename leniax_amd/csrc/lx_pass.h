@@ -44,6 +44,89 @@ LX_DEV int freq_of(int t, int e) {
   }
 }
 
+// Lane groups of the line passes.  Neighbouring lines are neighbouring complex elements of a half-spectrum
+// row, and the texture unit takes a wave's addresses four neighbouring lanes at a time: four lanes of one
+// group (rows far apart) cost it four requests of 8 bytes, four lanes of four groups one of 32.  So lane l
+// of a wave holds point t = l / G of line l % G, G = 64 / T lines per wave.  (With a group's lanes side by
+// side the passes ran at one request per clock and CU, whatever their bytes: 16 worlds of 96^3, 7.2 M
+// elements read and written, 25 us = 56 k requests per CU.  Strided: the convolution along D of 8 worlds of
+// 96^3 29.5 -> 19.4 us.)
+template <int T>
+struct Strided {
+  static constexpr int G = 64 / T;  // lines of a wave
+  static LX_DEV int point(int lane) { return lane / G; }
+  static LX_DEV int line(int lane) { return lane % G; }
+};
+// Exchange scratch of a strided group (complex): its rows padded so that the 16-byte accesses of 16
+// consecutive lanes (16 / G points of G lines) lie in different banks.
+template <int L, int T>
+constexpr int strided_scratch() {
+  return T * xch_row(L / T) + (T == 4 ? 2 : T == 8 ? 20 : 8);
+}
+
+// p + sgn v over the lanes D apart (p the partner's value; sgn +1 in the lower lane, -1 in the upper):
+// 16 and 32 apart through the row and half swaps, which leave the lower lane's value in one register of
+// both lanes and the upper's in the other.
+template <int D>
+LX_DEV float strided_pair(float v, float sgn, int lane) {
+  if constexpr (D == 4 || D == 8) {
+    return fmaf(sgn, v, xor_fetch<D>(v, lane));
+  } else {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto r = D == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                           : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return fmaf(sgn, __builtin_bit_cast(float, unsigned(r[1])), __builtin_bit_cast(float, unsigned(r[0])));
+  }
+}
+
+// lane_stage (lx_device.h) over strided groups: the same arithmetic
+template <int P, int T, int L, bool INV, int H>
+LX_DEV void strided_stage(float2* x, int t, int lane, const float2* tw) {
+  const bool upper = (t & H) != 0;
+  const float sgn = upper ? -1.f : 1.f;
+  float2 w = make_float2(1.f, 0.f);
+  if constexpr (H > 1) {
+    const float2 tv = tw[(t & (H - 1)) * (L / (2 * H))];
+    w = upper ? make_float2(tv.x, INV ? -tv.y : tv.y) : w;
+  }
+#pragma unroll
+  for (int k = 0; k < P; ++k) {
+    const float2 o = INV && H > 1 ? cmul(x[k], w) : x[k];
+    const float2 v = make_float2(strided_pair<H * (64 / T)>(o.x, sgn, lane), strided_pair<H * (64 / T)>(o.y, sgn, lane));
+    x[k] = !INV && H > 1 ? cmul(v, w) : v;
+  }
+}
+template <int P, int T, int L, bool INV, int H>
+LX_DEV void strided_network(float2* x, int t, int lane, const float2* tw) {
+  if constexpr (INV ? H < T : H >= 1) {
+    strided_stage<P, T, L, INV, H>(x, t, lane, tw);
+    strided_network<P, T, L, INV, (INV ? H * 2 : H / 2)>(x, t, lane, tw);
+  }
+}
+// fft_lanes over strided groups
+template <int P, int T, bool INV>
+LX_DEV void fft_strided(float2* x, int t, int lane, const float2* tw) {
+  if constexpr (!INV) {
+    fft_reg<P, false>(x);
+    int j = 0;
+#pragma unroll
+    for (int k = 1; k < P; ++k) {
+      j += t;
+      x[k] = cmul(x[k], tw[j]);
+    }
+    strided_network<P, T, T * P, false, T / 2>(x, t, lane, tw);
+  } else {
+    strided_network<P, T, T * P, true, 1>(x, t, lane, tw);
+    int j = 0;
+#pragma unroll
+    for (int k = 1; k < P; ++k) {
+      j += t;
+      x[k] = cmulc(x[k], tw[j]);
+    }
+    fft_reg<P, true>(x);
+  }
+}
+
 LX_DEV void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 // ---------------------------------------------------------------- batched-run indirection
@@ -246,3 +329,24 @@ int lx_pass_tables(int L, hipStream_t st, LxPassTables* out);
 // to the shape; with *taken = 0 nothing was launched and the pass is the caller's.
 int lx_small_conv(const LineArgs& a, int L, int64_t lines, bool list, hipStream_t st, int* taken);
 int lx_small_rows(const RowArgs& a, int W, int64_t images, bool list, hipStream_t st, int* taken);
+
+// lx_plane.hip: the inner two axes of 3-D passes, one plane per workgroup (16-byte accesses: the caller's
+// states, fields and potentials start on 16 bytes), and the convolution along the outer one for worlds
+// that share a spectrum (*taken as above).
+bool lx_plane_takes(int H, int W);
+int lx_plane_fwd(int H, int W, const float* A, float2* S, int64_t planes, hipStream_t st);
+int lx_plane_inv(const RowArgs& a, int D, int H, int W, int64_t images, hipStream_t st);
+struct LxPlaneAdj {
+  float2* X;
+  const float* U;
+  float* lam;
+  const float* A;
+  float* part;
+  const float* gf;
+  const float* w;
+  const float* dt;
+  int64_t gf_bs, w_bs, dt_bs;
+  int kind, state_fn, ste, average, accumulate;
+};
+int lx_plane_adj(const LxPlaneAdj& c, int D, int H, int W, int64_t B, bool bridge, hipStream_t st);
+int lx_shared_conv(const LineArgs& a, int L, int64_t images, hipStream_t st, int* taken);

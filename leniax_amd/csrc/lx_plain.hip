@@ -563,6 +563,7 @@ int64_t adj_rows_per_image(const lx_rule* r) {
     const int W = r->dims[r->ndim - 1];
     const int64_t rows = cells_of(r) / W;
     per = std::max<int64_t>(per, (rows / 2 + 256 / lx_row_tpr(W) - 1) / (256 / lx_row_tpr(W)));
+    if (r->ndim == 3) per = std::max<int64_t>(per, r->dims[0]);  // plane kernels: one row per plane
   }
   return per;
 }

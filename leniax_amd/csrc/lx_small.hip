@@ -15,7 +15,7 @@
 namespace {
 
 // A lane group's transform with the lane's twiddles in registers (LDS exchange) or from the table.
-template <int L>
+template <int L, bool STRIDED = false>
 struct GroupFft {
   using LC = Lanes<L>;
   static constexpr int TPR = LC::TPR, P = LC::P;
@@ -40,6 +40,8 @@ struct GroupFft {
 #pragma unroll
         for (int k = 1; k < P; ++k) y[k] = INV ? cmulc(y[k], w[k]) : cmul(y[k], w[k]);
       }, xch);
+    } else if constexpr (STRIDED) {
+      fft_strided<P, TPR, INV>(x, t, lane, table);
     } else {
       fft_lanes<P, TPR, INV>(x, t, lane, table);
     }
@@ -79,15 +81,16 @@ template <int L, bool LIST, bool KQ, bool GRAD = false>
 __global__ __launch_bounds__(64) void small_conv_kernel(SmallConv a) {
   using LC = Lanes<L>;
   constexpr int TPR = LC::TPR, P = LC::P, NG = 64 / TPR;
-  __shared__ __align__(16) float2 xch_all[LC::XL ? NG * TPR * LC::XRS : 2];
+  using SG = Strided<TPR>;
+  __shared__ __align__(16) float2 xch_all[LC::XL ? NG * strided_scratch<L, TPR>() : 2];
   pin(a.S); pin(a.U); pin(a.Kh); pin(a.tw); pin(a.twl); pin(a.FA); pin(a.k_bstride); pin(a.k_elems); pin(a.img_elems);
   pin(a.cins); pin(a.total); pin(a.per_img); pin(a.WH); pin(a.a_stride); pin(a.st); pin(a.C); pin(a.K); pin(a.csign);
   if constexpr (GRAD) {
     pin(a.FAin); pin(a.dspec); pin(a.fa_cins); pin(a.C_fa);
   }
-  const int lane = threadIdx.x, t = lane % TPR;
-  float2* xch = xch_all + (LC::XL ? (lane / TPR) * (TPR * LC::XRS) : 0);
-  const int lid = int(blockIdx.x) * NG + lane / TPR;
+  const int lane = threadIdx.x, t = SG::point(lane);
+  float2* xch = xch_all + (LC::XL ? SG::line(lane) * strided_scratch<L, TPR>() : 0);
+  const int lid = int(blockIdx.x) * NG + SG::line(lane);
   int total = a.total;
   if constexpr (LIST) {
     total *= *a.nlive;  // total: of one slot's world
@@ -107,7 +110,7 @@ __global__ __launch_bounds__(64) void small_conv_kernel(SmallConv a) {
   float2 x[P], kv[P];
 #pragma unroll
   for (int m = 0; m < P; ++m) x[m] = src[(TPR * m + t) * st];
-  GroupFft<L> fft;
+  GroupFft<L, true> fft;
   fft.load(a.tw, a.twl, t);
   if constexpr (KQ) {
     const float* kq = reinterpret_cast<const float*>(a.Kh) + kb;
