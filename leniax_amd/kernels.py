@@ -13,6 +13,7 @@ lx_build_spectra): the per-individual host build of a quality-diversity loop
 """
 import ctypes
 import math
+import struct
 from dataclasses import dataclass
 from typing import Callable, Dict, List, Optional
 
@@ -239,45 +240,60 @@ def get_kernels_and_mapping(kernels_params: List, world_size: List[int], nb_chan
 
 
 # ------------------------------------------------------------------ device build (float64)
+_DESC = struct.Struct(f'=4i6d{_lib.LX_MAX_RINGS}d')  # lx_kernel_desc, packed as the C struct lays it out
+assert _DESC.size == ctypes.sizeof(_lib.lx_kernel_desc)
+_NO_RINGS = [0.] * _lib.LX_MAX_RINGS
+
+
+def _numbers(x):
+    """x as a list of numbers (struct packs ints and floats alike)."""
+    if type(x) is list and all(type(v) in (float, int) for v in x):
+        return x
+    return np.asarray(x, dtype=np.float64).reshape(-1).tolist()
+
+
+def _desc_bytes(param: Dict, R: float):
+    """The bytes of kernel_desc(param, R) and its radius (a quality-diversity batch has hundreds: packed
+    at once, not field by field through ctypes)."""
+    shape, kf = _lib.KERNEL_SHAPES.get(param['k_slug']), _lib.KERNEL_FNS.get(param['kf_slug'])
+    if shape is None:
+        raise ValueError(f"the device kernel build covers {sorted(_lib.KERNEL_SHAPES)}, not {param['k_slug']!r}")
+    if kf is None:
+        raise ValueError(f"unknown kernel function {param['kf_slug']!r}")
+    kp = param['k_params']
+    bs, kfp = _numbers(kp[1]), _numbers(param['kf_params'])
+    nb = len(bs)
+    if not 1 <= nb <= _lib.LX_MAX_RINGS:
+        raise ValueError(f'1..{_lib.LX_MAX_RINGS} rings supported, got {nb}')
+    kr = math.ceil(kp[0] * R)
+    if kr < 1:
+        raise ValueError(f'kernel radius ceil(r R) = {kr} < 1')
+    a, b, theta = (0., 0., 0.) if shape == 0 else (float(kp[2]), float(kp[3]), float(kp[4]))
+    k0, k1 = (kfp + [0., 0.])[:2]
+    return _DESC.pack(shape, kf, nb, kr, float(kp[0]), a, b, theta, k0, k1, *bs, *_NO_RINGS[nb:]), kr
+
+
 def kernel_desc(param: Dict, R: float):
     """lx_kernel_desc of one entry of kernels_params (k_slug circle_2d, ellipse_2d or
     oriented_ellipse_2d; raw kernels are arrays and stay on the host path)."""
-    slug = param['k_slug']
-    if slug not in _lib.KERNEL_SHAPES:
-        raise ValueError(f'the device kernel build covers {sorted(_lib.KERNEL_SHAPES)}, not {slug!r}')
-    if param['kf_slug'] not in _lib.KERNEL_FNS:
-        raise ValueError(f"unknown kernel function {param['kf_slug']!r}")
-    kp = param['k_params']
-    bs = [float(b) for b in np.asarray(kp[1], dtype=np.float64).reshape(-1)]
-    if not 1 <= len(bs) <= _lib.LX_MAX_RINGS:
-        raise ValueError(f'1..{_lib.LX_MAX_RINGS} rings supported, got {len(bs)}')
-    d = _lib.lx_kernel_desc()
-    d.shape = _lib.KERNEL_SHAPES[slug]
-    d.kf = _lib.KERNEL_FNS[param['kf_slug']]
-    d.nb = len(bs)
-    d.r = float(kp[0])
-    d.kr = math.ceil(kp[0] * R)
-    if d.kr < 1:
-        raise ValueError(f'kernel radius ceil(r R) = {d.kr} < 1')
-    if slug != 'circle_2d':
-        d.a, d.b, d.theta = float(kp[2]), float(kp[3]), float(kp[4])
-    kfp = [float(v) for v in np.asarray(param['kf_params'], dtype=np.float64).reshape(-1)][:2]
-    for i, v in enumerate(kfp):
-        d.kf_params[i] = v
-    for i, b in enumerate(bs):
-        d.bs[i] = b
-    return d
+    return _lib.lx_kernel_desc.from_buffer_copy(_desc_bytes(param, R)[0])
 
 
 def _descs_on_device(params: List[Dict], R: float, world_size):
     import torch
     from . import engine
-    descs = (_lib.lx_kernel_desc * len(params))(*[kernel_desc(p, R) for p in params])
-    max_kr = max(d.kr for d in descs)
+    descs = [_desc_bytes(p, R) for p in params]
+    max_kr = max(kr for _, kr in descs)
     if 2 * max_kr > min(world_size):
         raise ValueError(f'kernel of {2 * max_kr} cells does not fit the world {list(world_size)}')
-    raw = np.frombuffer(bytes(descs), dtype=np.uint8).copy()
-    return torch.as_tensor(raw).to(engine.device()), max_kr
+    dev = engine.device()
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError('kernels cannot be staged inside a stream capture (the descriptors are host data)')
+    # through pinned memory: a pageable copy waits for the stream, so that staging would wait for the
+    # batch before it
+    raw = torch.empty(len(descs) * _DESC.size, dtype=torch.uint8, pin_memory=True)
+    raw.numpy()[:] = np.frombuffer(b''.join(d for d, _ in descs), dtype=np.uint8)
+    return raw.to(dev, non_blocking=True), max_kr
 
 
 def build_kernels(params: List[Dict], world_size: List[int], R: float, basis: bool = False):
@@ -339,22 +355,30 @@ class HalfSpectra:
         return out
 
 
-def _mapping_of(kernels_params, nb_channels):
-    mapping = KernelMapping(nb_channels, len(kernels_params))
-    for kernel_idx, param in enumerate(kernels_params):
-        cin = param['c_in']
-        mapping.cin_kernels[cin].append(kernel_idx)
-        mapping.cin_gfs[cin].append(param['gf_slug'])
-        mapping.cin_gf_params[cin].append(param['gf_params'])
-        mapping.cin_kfs[cin].append(param['kf_slug'])
-        mapping.cin_k_params[cin].append(param['k_params'])
-        mapping.kernels_weight_per_channel[param['c_out']][kernel_idx] = param['h']
-    tc = []
-    max_k = max(map(len, mapping.cin_kernels))
-    for lst in mapping.cin_kernels:
-        tc += [True] * len(lst) + [False] * (max_k - len(lst))
-    mapping.true_channels = None if all(tc) else tc
-    return mapping
+def _mappings_of(configs, nb_channels):
+    """The mappings of configurations that share their kernels' input channels (sorted)."""
+    nk = len(configs[0])
+    cin_kernels = [[] for _ in range(nb_channels)]
+    for k, param in enumerate(configs[0]):
+        cin_kernels[param['c_in']].append(k)
+    max_k = max(map(len, cin_kernels))
+    true_channels = [j < len(lst) for lst in cin_kernels for j in range(max_k)]
+    true_channels = None if all(true_channels) else true_channels
+    out = []
+    for kps in configs:
+        m = KernelMapping.__new__(KernelMapping)
+        m.cin_kernels = [lst[:] for lst in cin_kernels]
+        m.cin_k_params = [[kps[k]['k_params'] for k in lst] for lst in cin_kernels]
+        m.cin_kfs = [[kps[k]['kf_slug'] for k in lst] for lst in cin_kernels]
+        m.cin_gfs = [[kps[k]['gf_slug'] for k in lst] for lst in cin_kernels]
+        m.cin_gf_params = [[kps[k]['gf_params'] for k in lst] for lst in cin_kernels]
+        weights = [[0.] * nk for _ in cin_kernels]
+        for k, param in enumerate(kps):
+            weights[param['c_out']][k] = param['h']
+        m.kernels_weight_per_channel = weights
+        m.true_channels = true_channels and true_channels[:]
+        out.append(m)
+    return out
 
 
 def build_kernel_spectra(configs_kernels_params: List[List[Dict]], world_size: List[int], nb_channels: int,
@@ -379,7 +403,7 @@ def build_kernel_spectra(configs_kernels_params: List[List[Dict]], world_size: L
     dims = (ctypes.c_int32 * 2)(H, W)
     _lib.call('lx_build_spectra', 2, dims, engine.ptr(desc_d), n, float(R), max_kr, engine.ptr(half),
               engine.ptr(work), engine.stream_ptr())
-    mappings = [_mapping_of(kp, nb_channels) for kp in sorted_cfgs]
+    mappings = _mappings_of(sorted_cfgs, nb_channels)
     K = len(sorted_cfgs[0])
     return HalfSpectra(half.reshape(len(sorted_cfgs), K, H, W // 2 + 1), mappings[0], world_size,
                        nb_channels), mappings
