@@ -36,14 +36,18 @@ struct F2 {
   // packed-row spectrum stride: blocks of P padded by one, plus one so that the Z stores and
   // gathers of 32 lanes (4 rows x 8 lanes) spread over the 64 LDS banks
   static constexpr int ZRS = TPR * (P + 1) + 1;
-  static constexpr int YRS = HALF + 2;           // column-spectrum row stride
-  static constexpr int ZSZ = HALF * ZRS;
-  static constexpr int YSZ = N * YRS;
-  static constexpr int BUF = ZSZ > YSZ ? ZSZ : YSZ;
+  // column spectra Y: rows 2r and 2r+1 take the place of packed row r, so that a wave's first Z stores of
+  // a step overwrite only rows that it has read itself (no barrier lies between those); the second row
+  // starts YRS later, for N = 128 at the offset that spreads the stores of 32 lanes (4 columns x 8 rows)
+  // over the banks
+  static constexpr int YRS = N == 128 ? 68 : HALF + 2;
+  static constexpr int BUF = HALF * ZRS;
   static constexpr int NRED = 12;
   static constexpr int J = P / TPR;              // frequencies k1 per lane after the exchange
   static constexpr int XRS = xch_row(P);         // exchange scratch row stride
   static constexpr int XG = TPR * XRS;           // exchange scratch per lane group
+  static_assert(YRS + HALF + 1 <= ZRS, "a row pair of Y fits in a row of Z");
+  static_assert(XG > N, "column 0 leaves N + 1 values in its scratch");
   LX_DEV static int zidx(int hp, int k) { return hp * ZRS + (k / P) * (P + 1) + (k % P); }
   LX_DEV static int ycol(int c) { return c + (c >= N / 4 ? 1 : 0); }
 };
@@ -87,6 +91,11 @@ LX_DEV int fresh(int v) {
   return v;
 }
 
+// 2^23 + v for 0 <= v < 2^23, by the bits: an integer OR and a subtraction issue at twice the rate of a
+// conversion
+constexpr float kTwo23 = 8388608.f;
+LX_DEV float small_float(int v) { return __uint_as_float(uint32_t(v) | 0x4B000000u); }
+
 LX_DEV float maxnan(float a, float b) { return (a != a) ? a : fmaxf(a, b); }
 
 LX_DEV float state_update(int fn, float a, float dt, float G) {
@@ -123,6 +132,13 @@ LX_DEV float field_of(float xr, const FieldK& f) {
   }
 }
 
+// A buffer over n floats of a history from off on, or over none where there is no history: its stores are
+// then dropped by the bounds check.  A branch per store cut the point loop into 96 blocks; without them
+// a recorded step of one 128 x 128 world takes 11.0 instead of 11.9 us.
+LX_DEV __amdgpu_buffer_rsrc_t hist_plane(float* hist, int64_t off, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc(hist ? hist + off : nullptr, 0, hist ? n * 4 : 0, 0x00020000);
+}
+
 template <int N, int GF, bool HIST, bool V1>
 __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
   using G = F2<N>;
@@ -131,7 +147,7 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
   __shared__ float2 buf[G::BUF];
   __shared__ __align__(16) float2 xch_all[(NT / TPR) * G::XG];
   __shared__ __align__(16) float2 twl[TPR * twl_row(P)];  // lane twiddle rows (fft_xlds)
-  __shared__ float2 kb[N];  // K0 - KN of the current world (written and read by lane group 0 alone)
+  __shared__ __align__(16) float2 kb[N];  // K0 - KN of the current world (written and read by lane group 0 alone)
   __shared__ float red[NW][G::NRED];
   __shared__ int ctrl[4];
   __shared__ lx_carry carry;  // statistics + heuristics carry of the current world (thread 0)
@@ -170,7 +186,7 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
       else ctrl[0] = i < *p.surv_count ? p.surv_list[i] : int(p.B);
     }
     __syncthreads();
-    const int64_t world = ctrl[0];
+    const int64_t world = __builtin_amdgcn_readfirstlane(ctrl[0]);
     if (world >= p.B) break;
 
     // a resumed world continues from its parked state (in the output buffer) and carry
@@ -207,7 +223,9 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
     fk.c2 = 2.f * fk.c1;
     fk.gk = (1.f / fk.s) * 0.84932180028801904272f;  // sqrt(log2(e) / 2) / s
     const float xr_eps = LX_EPS / fk.sc;  // U > eps  <=>  xr > eps / sc (exact scaling)
-    const float dtw = p.dt[world * p.dt_bstride];
+    float dtw = p.dt[world * p.dt_bstride];
+    // in VGPRs: an SGPR operand halves the issue rate of the field's FMAs
+    __asm__ volatile("" : "+v"(fk.sc), "+v"(fk.m), "+v"(fk.gk), "+v"(fk.inv_9s2), "+v"(fk.c1), "+v"(fk.c2), "+v"(dtw));
     if (tid == FIN) {
       if (p.resume) {
         carry = p.park[world];
@@ -277,7 +295,7 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
       }
     };
 
-    int t = carry.t;
+    int t = __builtin_amdgcn_readfirstlane(carry.t);
     const int t_first = t;  // first step of this residency: nothing to close before it
     const int t_end = p.limit < p.max_steps ? p.limit : p.max_steps;
     bool stopped = false;
@@ -338,7 +356,7 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
       // ---- multiply by the half spectrum; column 0 carries columns 0 and N/2:
       //      Q[f] = X[f] a[f] + conj(X[-f]) b[f], a = K0 + KN, b = K0 - KN (doubled, as the
       //      other columns).
-      //      X[-f] lives in another lane of the group: column 0 goes through its scratch.
+      //      X[-f] lives in another lane of the group: column 0 goes through its scratch, X[N] = X[0].
       {
         if (wave == 0 && r == 0) {
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -346,15 +364,18 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
           for (int j = 0; j < J; ++j)
 #pragma unroll
             for (int k2 = 0; k2 < TPR; ++k2) xch[J * q + j + P * k2] = x[j * TPR + k2];
+          if (q == 0) xch[N] = x[0];
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          const float2* xm = xch + J * (TPR - 1 - q);  // X[N - f] at constant offsets
+          const float2* kq = kb + J * q;
 #pragma unroll
           for (int j = 0; j < J; ++j) {
 #pragma unroll
             for (int k2 = 0; k2 < TPR; ++k2) {
-              const int f = J * q + j + P * k2;
-              const float2 pm = xch[(N - f) & (N - 1)];
-              x[j * TPR + k2] = cadd(cmul(x[j * TPR + k2], kreg[j * TPR + k2]), cmul(cconj(pm), kb[f]));
+              const float2 pm = xm[N - J * (TPR - 1) - j - P * k2];
+              x[j * TPR + k2] = cadd(cmul(x[j * TPR + k2], kreg[j * TPR + k2]), cmul(cconj(pm), kq[j + P * k2]));
             }
+            __builtin_amdgcn_sched_barrier(0);
           }
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         } else {
@@ -367,19 +388,19 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
       fft_xlds<P, TPR, true>(x, q, twl + fresh(q) * twl_row(P), xch);  // x[m] = column c at row h = TPR m + q (x N)
       __syncthreads();  // every column gather of Z is done before Y overwrites it
 #pragma unroll
-      for (int m = 0; m < P; ++m) buf[(TPR * m + q) * G::YRS + G::ycol(r)] = x[m];
+      for (int m = 0; m < P; ++m) buf[((TPR / 2) * m + (q >> 1)) * G::ZRS + (q & 1) * G::YRS + G::ycol(r)] = x[m];
       __syncthreads();
       // the previous step ended the world: this one is not applied (the state is unchanged)
       if (ctrl[1]) {
         stopped = true;
         break;
       }
-      const int sh0 = ctrl[2], sh1 = ctrl[3];
+      const int sh0 = __builtin_amdgcn_readfirstlane(ctrl[2]), sh1 = __builtin_amdgcn_readfirstlane(ctrl[3]);
 
       // ---- rows inverse: repack rows 2r, 2r+1 from their half spectra, k = (J q + j) + P k2:
       //      k < N/2 read directly, k > N/2 through conj(Y[N-k]); k = 0 and N/2 are real
       {
-        const int rowa = (2 * r) * G::YRS;
+        const int rowa = r * G::ZRS;
 #pragma unroll
         for (int j = 0; j < J; ++j) {
 #pragma unroll
@@ -411,15 +432,18 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
       float sa0 = 0.f, sa1 = 0.f, sg0 = 0.f, sg1 = 0.f;  // per-row sums of A and G+
       float sAy1 = 0.f, sGy1 = 0.f, sAyy1 = 0.f;         // column (x) moments
       uint32_t nA = 0, nG = 0, nU = 0;                    // per-lane counts
+      const int qs = q - sh1;
       const int64_t hist_off = (int64_t(t) * p.B + world) * cells_per_world;
+      // HIST: the step's plane of each history; one that is not kept has no bytes, and its stores are dropped
+      const auto hc = hist_plane(p.cells_hist, hist_off, N * N), hf = hist_plane(p.field_hist, hist_off, N * N),
+                 hp = hist_plane(p.pot_hist, hist_off, N * N);
+      const int hoff = 4 * (2 * r * N + q);
 #pragma unroll
       for (int m = 0; m < P; ++m) {
-        const int col = TPR * m + q;
-        const float xc = float(((col - sh1) & (N - 1)) - N / 2);
+        const float xc = small_float((qs + TPR * m) & (N - 1)) - (kTwo23 + float(N / 2));
         float am = 0.f, gpm = 0.f;
 #pragma unroll
         for (int part = 0; part < 2; ++part) {
-          const int row = 2 * r + part;
           const float xr = part ? x[m].y : x[m].x;
           const float a = part ? a1[m] : a0[m];
           const float Gf = field_of<GF>(xr, fk);
@@ -431,9 +455,10 @@ __global__ __launch_bounds__(F2<N>::NT) void fused2d_kernel(FusedParams p) {
           nG += (Gf > LX_EPS) ? 1u : 0u;
           nU += (xr > xr_eps) ? 1u : 0u;
           if constexpr (HIST) {
-            if (p.cells_hist) p.cells_hist[hist_off + row * N + col] = a;
-            if (p.field_hist) p.field_hist[hist_off + row * N + col] = Gf;
-            if (p.pot_hist) p.pot_hist[hist_off + row * N + col] = xr * fk.sc;
+            const int off = hoff + 4 * (part * N + TPR * m);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), hc, off, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(Gf), hf, off, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(xr * fk.sc), hp, off, 0, 0);
           }
           float an;
           if constexpr (V1) {  // leniax/core.py:245-272: clip(A + dt G, 0, 1)
