@@ -210,19 +210,19 @@ int make_geom(int ndim, const int32_t* dims, Geom& g) {
 // B[k] = (Z[k] - conj Z[W-k])/2i, stored with consecutive lanes on consecutive k.
 // LIST: npairs is the pairs of one slot (C rows / 2); the state comes from the slot's world.
 template <int W, bool LIST>
-__global__ __launch_bounds__(256) void rows_fwd_kernel(const float* __restrict__ A, float2* __restrict__ S,
-                                                       int64_t npairs, RunView rv) {
+LX_DEV void rows_fwd_block(const float* __restrict__ A, float2* __restrict__ S, int64_t npairs, const RunView& rv,
+                           int64_t block) {
   using LC = Lanes<W>;
   constexpr int TPR = LC::TPR, P = LC::P, WH = W / 2 + 1;
   __shared__ __align__(16) float2 xch_all[LC::XCH];
   const int lane = threadIdx.x & 63;
   const int t = threadIdx.x % TPR;
   float2* xch = xch_all + (threadIdx.x / TPR) * (TPR * LC::XRS);
-  const int64_t pr = (int64_t(blockIdx.x) * 256 + threadIdx.x) / TPR;
+  const int64_t pr = (block * 256 + threadIdx.x) / TPR;
   int64_t total = npairs;
   if constexpr (LIST) {
     total = int64_t(*rv.nlive) * npairs;
-    if (int64_t(blockIdx.x) * (256 / TPR) >= total) return;  // the block's slots are all empty
+    if (block * (256 / TPR) >= total) return;  // the block's slots are all empty
   }
   const bool live = pr < total;
   const int64_t row0 = live ? pr * 2 : 0;  // row pairs never straddle images: rows per image are even
@@ -254,6 +254,12 @@ __global__ __launch_bounds__(256) void rows_fwd_kernel(const float* __restrict__
       }
     }
   }
+}
+
+template <int W, bool LIST>
+__global__ __launch_bounds__(256) void rows_fwd_kernel(const float* __restrict__ A, float2* __restrict__ S,
+                                                       int64_t npairs, RunView rv) {
+  rows_fwd_block<W, LIST>(A, S, npairs, rv, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- lines along a leading axis
@@ -696,8 +702,16 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
 }
 
 // ---------------------------------------------------------------- launchers
-int launch_rows_fwd(const Geom& g, const float* A, float2* S, int64_t nimg, hipStream_t st) {
+// a run's statistics of the step before, to be taken along by the next step's first launch
+struct RunStatArgs;
+int launch_run_stats(const RunStatArgs& sa, hipStream_t st);
+int launch_rows_fwd_stats(const Geom& g, const float* A, float2* S, int64_t npairs, const RunStatArgs& sa,
+                          hipStream_t st);
+
+int launch_rows_fwd(const Geom& g, const float* A, float2* S, int64_t nimg, hipStream_t st,
+                    const RunStatArgs* prev = nullptr) {
   const int64_t npairs = nimg * (g.rows / 2);
+  if (prev) return launch_rows_fwd_stats(g, A, S, npairs, *prev, st);
   return dispatch_len(g.W, [&](auto w) {
     constexpr int W = decltype(w)::value;
     if (int rc = ensure_tw<W>(st)) return rc;
@@ -910,10 +924,16 @@ bool takes_planes(const Geom& g, std::initializer_list<const void*> arrays) {
   return true;
 }
 
-// forward transform of real images along every axis but the convolution axis
-int fwd_inner(const Geom& g, const float* A, float2* S, int64_t nimg, hipStream_t st) {
-  if (takes_planes(g, {A})) return lx_plane_fwd(g.L[1], g.W, A, S, nimg * g.L[0], st);
-  if (int rc = launch_rows_fwd(g, A, S, nimg, st)) return rc;
+// forward transform of real images along every axis but the convolution axis (and a run's statistics of the
+// step before)
+int fwd_inner(const Geom& g, const float* A, float2* S, int64_t nimg, hipStream_t st,
+              const RunStatArgs* prev = nullptr) {
+  if (takes_planes(g, {A})) {
+    if (prev)
+      if (int rc = launch_run_stats(*prev, st)) return rc;
+    return lx_plane_fwd(g.L[1], g.W, A, S, nimg * g.L[0], st);
+  }
+  if (int rc = launch_rows_fwd(g, A, S, nimg, st, prev)) return rc;
   if (g.naxes == 1) return LX_OK;
   LineArgs la = line_args();
   la.S = S; la.mode = 1;
@@ -946,13 +966,14 @@ int inv_inner(const Geom& g, RowArgs ra, int64_t nk, int64_t nimg, hipStream_t s
 int plain_step(const lx_rule* rule, const float* A, int64_t B, const void* Kh, int64_t k_bs, const float* gf,
                int64_t gf_bs, const float* w, int64_t w_bs, const float* dt, int64_t dt_bs, float* A_out,
                float* field, float* pot, void* work, hipStream_t st, int sel, float2* FA = nullptr,
-               float* part = nullptr, const void* carry = nullptr, int carry_bytes = 0, float dt_val = 0.f) {
+               float* part = nullptr, const void* carry = nullptr, int carry_bytes = 0, float dt_val = 0.f,
+               const RunStatArgs* prev = nullptr) {
   Geom g;
   if (int rc = make_geom(rule->ndim, rule->dims, g)) return rc;
   const int C = rule->C, K = rule->K;
   float2* S = static_cast<float2*>(work);
   float2* U = S + B * C * g.half;
-  int rc = fwd_inner(g, A, S, B * C, st);
+  int rc = fwd_inner(g, A, S, B * C, st, prev);
   if (!rc) {  // the convolution axis
     LineArgs la = line_args();
     la.S = S; la.U = U; la.Kh = static_cast<const float2*>(Kh); la.k_bstride = k_bs; la.C = C; la.K = K;
@@ -1286,6 +1307,7 @@ __global__ void run_start_kernel(RunCtl c, int64_t B, int slots) {
 
 struct RunStatArgs {
   RunCtl c;
+  int slots;           // blocks
   int par;             // the list this step reads (-1: slot b is world b, nothing is retired)
   const float* part;   // [slots][C][pairs] row-pair records
   int64_t pairs;
@@ -1301,8 +1323,7 @@ struct RunStatArgs {
 
 // One block per slot: the step's statistics of the slot's world (leniax/statistics.py:64-126), its
 // carry, the heuristics and the stop decision (a stop, or the world's last step, frees the slot).
-__global__ __launch_bounds__(kPairThreads) void run_stats_kernel(RunStatArgs a) {
-  const int slot = blockIdx.x;
+LX_DEV void run_stats_block(const RunStatArgs& a, int slot) {
   int64_t b = slot;
   if (a.par >= 0) {
     const int32_t* list = a.par ? a.c.list1 : a.c.list0;
@@ -1322,6 +1343,41 @@ __global__ __launch_bounds__(kPairThreads) void run_stats_kernel(RunStatArgs a) 
     if (a.n_out) a.n_out[b] = cr.n;
     if (a.steps_out) a.steps_out[b] = cr.t;
   }
+}
+
+__global__ __launch_bounds__(kPairThreads) void run_stats_kernel(RunStatArgs a) { run_stats_block(a, blockIdx.x); }
+
+// The forward rows of a step and, in the first blocks, the statistics of the step before: a launch of their
+// own is 5.5 us of latency (one block per world, a chain of sums and divisions), here it runs beside the rows.
+// The two share nothing: the statistics read the step's records and write the worlds' carries, which only
+// the inverse rows read and write again.  24 recorded steps of
+// one 3-channel 6-kernel 256^2 world 735 -> 641 us, 10 steps of 64 such worlds 1900 -> 1855 us.
+static_assert(kPairThreads == 256, "both parts run in blocks of 256 threads");
+template <int W>
+__global__ __launch_bounds__(256) void rows_fwd_stats_kernel(const float* __restrict__ A, float2* __restrict__ S,
+                                                             int64_t npairs, RunStatArgs a) {
+  if (int(blockIdx.x) < a.slots) {
+    run_stats_block(a, blockIdx.x);
+    return;
+  }
+  rows_fwd_block<W, false>(A, S, npairs, RunView{nullptr, nullptr, nullptr, nullptr, nullptr, 0},
+                           int64_t(blockIdx.x) - a.slots);
+}
+
+int launch_run_stats(const RunStatArgs& sa, hipStream_t st) {
+  hipLaunchKernelGGL(run_stats_kernel, dim3(unsigned(sa.slots)), dim3(kPairThreads), 0, st, sa);
+  return launched("run statistics");
+}
+
+int launch_rows_fwd_stats(const Geom& g, const float* A, float2* S, int64_t npairs, const RunStatArgs& sa,
+                          hipStream_t st) {
+  return dispatch_len(g.W, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    if (int rc = ensure_tw<W>(st)) return rc;
+    const unsigned blocks = unsigned(blocks_for(npairs * Lanes<W>::TPR)) + unsigned(sa.slots);
+    hipLaunchKernelGGL(rows_fwd_stats_kernel<W>, dim3(blocks), dim3(256), 0, st, A, S, npairs, sa);
+    return launched("rows_fwd + run statistics");
+  });
 }
 
 // One block: the next step's live list, the slots whose world goes on (in order) and then worlds
@@ -1436,13 +1492,13 @@ int tune_run_lines(const PassesRun& r, int bucket, hipStream_t st) {
   return rc;
 }
 
-RunStatArgs run_stat_args(const PassesRun& r, int par) {
+RunStatArgs run_stat_args(const PassesRun& r, int par, int slots) {
   const lx_rule* rule = r.rule;
   const lx_run_args* a = r.a;
   const Geom& g = r.g;
   const int C = rule->C;
   RunStatArgs sa;
-  sa.c = r.ctl; sa.par = par; sa.part = r.part; sa.pairs = g.rows / 2; sa.C = C; sa.ndim = rule->ndim;
+  sa.c = r.ctl; sa.slots = slots; sa.par = par; sa.part = r.part; sa.pairs = g.rows / 2; sa.C = C; sa.ndim = rule->ndim;
   for (int i = 0; i < 3; ++i) sa.dims[i] = i < rule->ndim ? rule->dims[i] : 1;
   sa.R2 = (float)((double)a->R * (double)a->R); sa.R = a->R; sa.dt = (float)(1.0 / (double)a->T);
   sa.stop_policy = a->stop_policy; sa.min_steps = a->min_steps; sa.max_steps = a->max_steps;
@@ -1508,8 +1564,7 @@ int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
     return launched("rows_inv (run)");
   });
   if (rc) return rc;
-  const RunStatArgs sa = run_stat_args(r, par);
-  hipLaunchKernelGGL(run_stats_kernel, dim3(unsigned(bucket)), dim3(kPairThreads), 0, st, sa);
+  if ((rc = launch_run_stats(run_stat_args(r, par, bucket), st))) return rc;
   if (bucket <= 64)
     hipLaunchKernelGGL(run_control_kernel<64>, dim3(1), dim3(64), 0, st, r.ctl, par, r.slots, a->B);
   else
@@ -1534,7 +1589,7 @@ int run_every_step(const PassesRun& r, float* X1, hipStream_t st) {
       return lx_fail(LX_EDEVICE, "lx_run: copy of the initial states failed");
     cur = first;
   }
-  const RunStatArgs sa = run_stat_args(r, -1);
+  const RunStatArgs sa = run_stat_args(r, -1, int(B));
   for (int t = 0; t < a->max_steps; ++t) {
     const bool last = t + 1 == a->max_steps;
     float* next = last ? a->cells_d
@@ -1543,13 +1598,11 @@ int run_every_step(const PassesRun& r, float* X1, hipStream_t st) {
     if (int rc = plain_step(rule, cur, B, a->K_half_d, a->k_bstride, a->gf_d, a->gf_bstride, a->w_d, a->w_bstride,
                             a->dt_d, a->dt_bstride, next, a->field_hist_d ? a->field_hist_d + t * elems : nullptr,
                             a->potential_hist_d ? a->potential_hist_d + t * pots : nullptr, r.S, st, 0, nullptr,
-                            r.part, r.ctl.carry, int(sizeof(lx_carry))))
+                            r.part, r.ctl.carry, int(sizeof(lx_carry)), 0.f, t ? &sa : nullptr))
       return rc;
-    hipLaunchKernelGGL(run_stats_kernel, dim3(unsigned(B)), dim3(kPairThreads), 0, st, sa);
-    if (int rc = launched("run statistics")) return rc;
     cur = next;
   }
-  return LX_OK;
+  return a->max_steps > 0 ? launch_run_stats(sa, st) : LX_OK;
 }
 
 // twiddle tables of every length the step uses, built before a capture starts
