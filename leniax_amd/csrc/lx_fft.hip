@@ -510,10 +510,12 @@ __global__ __launch_bounds__(256) void conv_staged_kernel(LineArgs a) {
 // multiple of the pairs per wave), so the world's weights and growth parameters are the same for
 // the whole wave: the wave copies them into LDS once instead of loading them from global memory
 // in each kernel iteration, and its branches on them are uniform.
-template <int W, bool STATS, bool UNI, bool LIST = false>
-__global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
+template <int W, bool STATS, bool UNI, bool LIST = false, bool FETCH = true>
+__global__ __launch_bounds__(256, FETCH ? 1 : 4) void rows_inv_kernel(RowArgs a) {
   using LC = Lanes<W>;
-  constexpr int TPR = LC::TPR, P = LC::P, WH = W / 2 + 1;
+  constexpr int TPR = LC::TPR, P = LC::P, WH = W / 2 + 1, NPRE = (WH + TPR - 1) / TPR;
+  constexpr bool PRE = FETCH && UNI && P <= 16;
+  static_assert(2 * NPRE >= P, "the state's rows fit the registers of the spectra's");
   __shared__ __align__(16) float2 xch_all[LC::XCH];
   __shared__ float wpar[UNI ? 4 : 1][UNI ? LX_MAX_C * LX_MAX_K + 2 * LX_MAX_K : 1];
   const int lane = threadIdx.x & 63;
@@ -559,26 +561,76 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
   }
   // the world's step (LIST: history rows and the state buffers follow it)
   const int64_t tw = LIST ? int64_t(a.rv.carry[bw].t) : 0;
+  // the pair's first row of the state
+  auto state_rows = [&]() -> const float* {
+    if constexpr (LIST) return run_state(a.rv, bw, false) + (int64_t(c) * a.rows + r2) * W;
+    return a.A + (img * a.rows + r2) * int64_t(W);
+  };
   float G0[P], G1[P];
 #pragma unroll
   for (int m = 0; m < P; ++m) G0[m] = G1[m] = 0.f;
   float den = 0.f;
   float nU = 0.f;  // statistics: potential cells above eps, over the kernels this channel owns
   float2 x[P];
+  // every kernel has one owner channel: it writes the kernel's potential and counts its cells
+  auto owner_of = [&](int k) {
+    if (a.sel) return int(a.cin[k]);
+    int owner = 0;
+    for (int cc = a.C - 1; cc >= 0; --cc)
+      if (pw[cc * a.K + k] != 0.f) owner = cc;
+    return owner;
+  };
+  uint32_t used = 0, owned = 0;  // PRE: the kernels that this channel takes, those it owns
+  if constexpr (PRE) {
+    for (int k = 0; k < a.K; ++k) {
+      const bool own = owner_of(k) == c;
+      const bool takes = a.sel ? own : pw[c * a.K + k] != 0.f;
+      owned |= uint32_t(own) << k;
+      used |= uint32_t(takes || (own && (STATS || a.pot != nullptr))) << k;
+    }
+    used = __builtin_amdgcn_readfirstlane(int(used));
+    owned = __builtin_amdgcn_readfirstlane(int(owned));
+  }
+  // PRE: a kernel's rows are loaded while the one before is transformed, the state's while the last is, so
+  // that a wave waits for memory once per channel instead of once per kernel and once for the state.  168
+  // VGPRs (3 waves per SIMD) instead of 127 (4): 79 -> 66 us for 64 3-channel 6-kernel worlds of 256^2 with
+  // statistics, whose 6144 waves are then two full rounds; 16 points a lane at most, as 24 and 32 are at 2
+  // waves without it, and not where a wave's lanes differ in their kernels (137 -> 175 VGPRs there).
+  float2 pre0[NPRE], pre1[NPRE];
+  auto fetch = [&](int k, int t) {
+    const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;
+    const float2* u1 = u0 + WH;
+#pragma unroll
+    for (int i = 0; i < NPRE; ++i) {
+      const int col = t + TPR * i;
+      if (col < WH) {
+        pre0[i] = u0[col];
+        pre1[i] = u1[col];
+      }
+    }
+  };
+  auto fetch_state = [&](int t) {
+    const float* in = state_rows();
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      const float v0 = in[TPR * m + t], v1 = in[W + TPR * m + t];
+      if (m & 1) {
+        pre0[m / 2].y = v0, pre1[m / 2].y = v1;
+      } else {
+        pre0[m / 2].x = v0, pre1[m / 2].x = v1;
+      }
+    }
+  };
+  if constexpr (PRE) {
+    if (used) fetch(__builtin_ctz(used), t);
+    else if (a.update) fetch_state(t);
+  }
   for (int k = 0; k < a.K; ++k) {
     const float wk = a.sel ? (a.cin[k] == c ? 1.f : 0.f) : pw[c * a.K + k];
     den = add_nc(den, wk);
-    int owner = 0;
-    if (a.sel) {
-      owner = a.cin[k];
-    } else {
-      for (int cc = a.C - 1; cc >= 0; --cc)
-        if (pw[cc * a.K + k] != 0.f) owner = cc;
-    }
-    // every kernel has one owner channel: it writes the kernel's potential and counts its cells
-    const bool own = owner == c;
+    const bool own = PRE ? (owned >> k) & 1u : owner_of(k) == c;
     const bool want_pot = a.pot != nullptr && own;
-    if (wk == 0.f && !want_pot && !(STATS && own)) continue;
+    if (PRE ? !((used >> k) & 1u) : wk == 0.f && !want_pot && !(STATS && own)) continue;
     int t = threadIdx.x % TPR;  // opaque per iteration: addresses and twiddles are not hoisted
     __asm__ volatile("" : "+v"(t));
     // stage the two rows' half spectra (coalesced), then repack them as one complex row:
@@ -587,14 +639,19 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
     const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;
     const float2* u1 = u0 + WH;
 #pragma unroll
-    for (int i = 0; i < (WH + TPR - 1) / TPR; ++i) {
+    for (int i = 0; i < NPRE; ++i) {
       const int col = t + TPR * i;
       if (col < WH) {
-        xch[col] = u0[col];
-        xch[WH + col] = u1[col];
+        xch[col] = PRE ? pre0[i] : u0[col];
+        xch[WH + col] = PRE ? pre1[i] : u1[col];
       }
     }
     wave_lds_fence();
+    if constexpr (PRE) {
+      const uint32_t rest = used >> k >> 1;
+      if (rest) fetch(k + 1 + __builtin_ctz(rest), t);
+      else if (a.update) fetch_state(t);
+    }
 #pragma unroll
     for (int e = 0; e < P; ++e) {
       const int kk = freq_of<W>(t, e);
@@ -661,18 +718,17 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
   if (!a.update || !live) return;
   const float dtw = a.sel ? 1.f : a.dt ? a.dt[bw * a.dt_bs] : a.dt_val;
   const int64_t off = (img * a.rows + r2) * int64_t(W);
-  const float* Ain = a.A + off;
   float* Aout = a.A_out + off;
   float* fld = a.field ? a.field + off : nullptr;
   float* chist = nullptr;
   if constexpr (LIST) {
     const int64_t in_world = (int64_t(c) * a.rows + r2) * W;
-    Ain = run_state(a.rv, bw, false) + in_world;
     Aout = run_state(a.rv, bw, true) + in_world;
     const int64_t hist_off = (tw * a.hist_B + bw) * a.rv.world_elems + in_world;
     fld = a.field ? a.field + hist_off : nullptr;
     chist = a.cells_hist ? a.cells_hist + hist_off : nullptr;
   }
+  const float* Ain = LIST ? state_rows() : a.A + off;
   PairSums sums;  // statistics mode
   int sh[3] = {0, 0, 0};
   if (STATS) pair_shift(LIST ? a.rv.carry[bw] : *pair_carry(a.carry, a.carry_bytes, b), a.ndim, a.d0, a.d1, W, sh);
@@ -682,7 +738,8 @@ __global__ __launch_bounds__(256) void rows_inv_kernel(RowArgs a) {
     float g0 = G0[m], g1 = G1[m];
     if (a.average) { g0 = (g0 / den); g1 = (g1 / den); }
     if (fld) { fld[col] = g0; fld[W + col] = g1; }
-    const float v0 = Ain[col], v1 = Ain[W + col];
+    const float v0 = !PRE ? Ain[col] : m & 1 ? pre0[m / 2].y : pre0[m / 2].x;
+    const float v1 = !PRE ? Ain[W + col] : m & 1 ? pre1[m / 2].y : pre1[m / 2].x;
     if (LIST && chist) { chist[col] = v0; chist[W + col] = v1; }
     if (STATS) {
       int zc = col - sh[2];
@@ -885,6 +942,16 @@ int launch_rows_inv(const Geom& g, RowArgs ra, int64_t nimg, hipStream_t st) {
     if (int rc = ensure_tw<W>(st)) return rc;
     const dim3 grid(blocks_for(ra.npairs * Lanes<W>::TPR) + unsigned(ra.fin.blocks));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;  // waves never straddle images
+    // A grid that the chip holds at once without the early loads (4 waves per SIMD on 256 CUs) but not with
+    // them (3) takes them at a second, mostly empty round: 98 against 104 us a step for 42 3-channel 6-kernel
+    // worlds of 256^2 (1008 blocks); 768 blocks and from 1536 on they win (96 -> 87 and 191 -> 179 us).
+    if constexpr (W >= 128 && Lanes<W>::P == 16) {
+      if (uni && grid.x > 768 && grid.x <= 1024) {
+        if (ra.part) hipLaunchKernelGGL((rows_inv_kernel<W, true, true, false, false>), grid, dim3(256), 0, st, ra);
+        else hipLaunchKernelGGL((rows_inv_kernel<W, false, true, false, false>), grid, dim3(256), 0, st, ra);
+        return launched("rows_inv");
+      }
+    }
     if (ra.part) {
       if (uni) hipLaunchKernelGGL((rows_inv_kernel<W, true, true>), grid, dim3(256), 0, st, ra);
       else hipLaunchKernelGGL((rows_inv_kernel<W, true, false>), grid, dim3(256), 0, st, ra);
