@@ -171,14 +171,6 @@ int lx_potential_direct_adjoint(const lx_rule* rule, const float* state_d, int64
                                 int32_t kh, int32_t kw, const float* dpot_d, float* dstate_d, float* dkern_d,
                                 void* stream);
 
-/* The same with a workspace of lx_potential_direct_adjoint_size bytes for the kernel side's partial
- * sums, which then runs on the matrix cores over tiles of the worlds (without one: one workgroup per
- * kernel tap over all worlds).  Deterministic: the partial sums are added in a fixed order. */
-int lx_potential_direct_adjoint_size(const lx_rule* rule, int64_t B, int32_t kh, int32_t kw, size_t* bytes);
-int lx_potential_direct_adjoint_work(const lx_rule* rule, const float* state_d, int64_t B, const float* kern_d,
-                                     int32_t kh, int32_t kw, const float* dpot_d, float* dstate_d,
-                                     float* dkern_d, void* work_d, void* stream);
-
 /* leniax/core.py:163-199 get_field (+ weighted_sum/weighted_mean):
  * field_d [B][C][dims] = sum_k w[c][k] g_k(potential_k) (/ sum_k w[c][k]).
  * gf_d [K][2] (m, s) and w_d [C][K] per world with strides gf_bstride / w_bstride floats (0: shared). */
@@ -195,11 +187,6 @@ int lx_update(const lx_rule* rule, const float* state_d, int64_t B, const void* 
               const float* gf_d, int64_t gf_bstride, const float* w_d, int64_t w_bstride, const float* dt_d,
               int64_t dt_bstride, float* state_out_d, float* field_d, float* potential_d, void* work_d,
               void* stream);
-
-/* lx_update with one dt for every world, by value (no device scalar to fill first). */
-int lx_update_dt(const lx_rule* rule, const float* state_d, int64_t B, const void* K_half_d, int64_t k_bstride,
-                 const float* gf_d, int64_t gf_bstride, const float* w_d, int64_t w_bstride, float dt,
-                 float* state_out_d, float* field_d, float* potential_d, void* work_d, void* stream);
 
 /* lx_update that also writes the forward spectra of the input state, rfftn(state) as
  * [B][C][dims[:-1]][dims[-1]/2+1] complex64, to state_spec_d: the recompute step of the adjoint,

@@ -4,7 +4,7 @@
 #include <math.h>
 #include <stdint.h>
 
-#include "../../include/leniax_amd.h"
+#include "../../include/leniax_amd_ext.h"
 #include "lx_device.h"
 
 #define LX_EPS 1e-7f  // leniax/constant.py:8
