@@ -232,15 +232,21 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
   float* counts = wl + RP * C * K;                               // [RP][K]
   float* vg = counts + ((groups + RP * C * K + 3) & ~3) - RP * C * K;  // STATS: [RP][C][2 rows][state, field][W]
   // the world (LIST: slot) and first row of the block's pair q (pairs past the last: the first world's)
+  // (a single world, and below a single pair, take no division: its 30 instructions at one wave's issue rate
+  // stood before the loads several times.  With the taken kernels' bits below, for one world: 13.8 -> 12.2 us
+  // with statistics at 256^2, 3 channels, 6 kernels, 9.6 -> 7.9 at 128^2, 3 channels, 15 kernels)
   auto world = [&](int q, int64_t& r2) {
-    const int wp = wp0 + q, b = wp < npairs ? wp / a.half_rows : 0;
+    const int wp = wp0 + q;
+    int b = 0;
+    if (npairs > a.half_rows) b = wp < npairs ? wp / a.half_rows : 0;
     r2 = wp < npairs ? (wp - b * a.half_rows) * 2 : 0;
     return b;
   };
+  auto pair_of = [&](int i, int per) { return RP > 1 ? i / per : 0; };
   auto params_of = [&](int b) { return LIST ? int64_t(a.rv.list[b]) : int64_t(b); };
   // ---- every load first: the groups' rows and twiddles, parameters, the state of the thread's points
   const bool mine = gi < groups;
-  const int gp = mine ? gi / K : 0, gk = mine ? gi - gp * K : 0;
+  const int gp = mine ? pair_of(gi, K) : 0, gk = mine ? gi - gp * K : 0;
   float2 p0[NI], p1[NI];
   GroupFft<W> fft;
   if (mine) {
@@ -258,12 +264,12 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
   float wreg = 0.f, gm = 0.f, gs = 1.f;
   if (a.update && !a.sel) {
     if (tid < RP * C * K) {
-      const int q = tid / (C * K);
+      const int q = pair_of(tid, C * K);
       int64_t r2;
       wreg = a.w[params_of(world(q, r2)) * a.w_bs + (tid - q * C * K)];
     }
     if (tid < groups) {
-      const int q = tid / K;
+      const int q = pair_of(tid, K);
       int64_t r2;
       const float* g = a.gf + params_of(world(q, r2)) * a.gf_bs + 2 * (tid - q * K);
       gm = g[0];
@@ -278,7 +284,7 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
     const int item = tid + 256 * it;
     dtw[it] = 1.f;
     if (a.update && item < items) {
-      const int pc = item / (2 * Q), q = pc / C, c = pc - q * C;
+      const int pc = item / (2 * Q), q = pair_of(pc, C), c = pc - q * C;
       int64_t r2;
       const int b = world(q, r2);
       const int64_t bw = params_of(b);
@@ -342,7 +348,7 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
   // ---- the potentials
   if (a.pot) {
     for (int item = tid; item < groups * 2 * Q; item += 256) {
-      const int pk = item / (2 * Q), q = pk / K, k = pk - q * K, r = item / Q & 1, col = item % Q * 4;
+      const int pk = item / (2 * Q), q = pair_of(pk, K), k = pk - q * K, r = item / Q & 1, col = item % Q * 4;
       if (wp0 + q >= npairs) continue;
       int64_t r2;
       const int b = world(q, r2);
@@ -361,20 +367,31 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
   for (int it = 0; it < IT; ++it) {
     const int item = tid + 256 * it;
     if (item >= items) break;
-    const int pc = item / (2 * Q), q = pc / C, c = pc - q * C, r = item / Q & 1, col = item % Q * 4;
+    const int pc = item / (2 * Q), q = pair_of(pc, C), c = pc - q * C, r = item / Q & 1, col = item % Q * 4;
     if (wp0 + q >= npairs) continue;
     const float* w = wl + pc * K;
     float4 G = make_float4(0.f, 0.f, 0.f, 0.f);
     float den = 0.f;
-    for (int k = 0; k < K; ++k) {
-      const float wk = a.sel ? ((int(a.cins >> (4 * k)) & 15) == c ? 1.f : 0.f) : w[k];
-      den = add_nc(den, wk);
-      if (wk == 0.f) {
-        // a kernel that feeds no channel counts (times 0) in channel 0 where its potential is wanted
-        bool skip = a.sel || c != 0 || !(STATS || a.pot);
-        for (int cc = 1; cc < C && !skip; ++cc) skip = w[cc * K + k] != 0.f;
-        if (skip) continue;
+    // the kernels with a weight here, and in channel 0 those that no channel takes (they count, times 0, where
+    // their potential is wanted): the weights' LDS reads overlap, where a test per kernel waited for each
+    uint32_t take = 0;
+    if (a.sel) {
+      for (int k = 0; k < K; ++k) take |= uint32_t((int(a.cins >> (4 * k)) & 15) == c) << k;
+    } else {
+#pragma unroll 4
+      for (int k = 0; k < K; ++k) take |= uint32_t(w[k] != 0.f) << k;
+      if (c == 0 && (STATS || a.pot)) {
+        uint32_t any = take;
+        for (int cc = 1; cc < C; ++cc)
+#pragma unroll 4
+          for (int k = 0; k < K; ++k) any |= uint32_t(w[cc * K + k] != 0.f) << k;
+        take |= ~any & ((1u << K) - 1u);
       }
+    }
+    for (; take; take &= take - 1) {
+      const int k = __builtin_ctz(take);
+      const float wk = a.sel ? 1.f : w[k];
+      den = add_nc(den, wk);
       float4 g = *reinterpret_cast<const float4*>(pots + (q * K + k) * (2 * GRS) + r * W + col);
       if (!a.sel) {
         const float4 pk = par[q * K + k];
@@ -423,7 +440,7 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
   if constexpr (STATS) {
     __syncthreads();
     for (int pc = gi; pc < RP * C; pc += 256 / TPR) {
-      const int q = pc / C, c = pc - q * C;
+      const int q = pair_of(pc, C), c = pc - q * C;
       if (wp0 + q >= npairs) continue;
       int64_t r2;
       const int b = world(q, r2);
@@ -440,6 +457,7 @@ __global__ __launch_bounds__(256) void small_rows_kernel(SmallRows a) {
       }
       float n = 0.f;
       if (c == 0 && t == 0)
+#pragma unroll 4
         for (int k = 0; k < K; ++k) n += counts[q * K + k];
       pair_record<TPR>(sums, n, sh, r2, a.ndim, a.d0, a.d1, t,
                        a.part + (int64_t(b * C + c) * a.half_rows + (r2 >> 1)) * LX_PAIR_REC);
@@ -482,7 +500,7 @@ int by_length(int L, F&& f) {
 // chip has idle issue slots for the repeated transforms and the barrier.  Beyond, measured at 12288 waves
 // (64 worlds of 256^2, 3 channels, 6 kernels, 10 steps): 2.28 ms with the general passes, 2.58 with these
 // rows, 3.08 with these lines.  Below, general -> these, us: inverse rows 10.2 -> 6.0 (1 x 256^2, one kernel),
-// 33 -> 9.6 (1 x 128^2, 3 channels, 15 kernels), 34 -> 23 (6 x 192 x 384, 5 kernels); convolution 6.7 -> 4.9,
+// 33 -> 7.9 (1 x 128^2, 3 channels, 15 kernels), 34 -> 23 (6 x 192 x 384, 5 kernels); convolution 6.7 -> 4.9,
 // 24 -> 4.9, 28 -> 12.
 constexpr int64_t kSmallWaves = 2048;
 
