@@ -511,10 +511,10 @@ __global__ __launch_bounds__(256) void conv_staged_kernel(LineArgs a) {
 // the whole wave: the wave copies them into LDS once instead of loading them from global memory
 // in each kernel iteration, and its branches on them are uniform.
 template <int W, bool STATS, bool UNI, bool LIST = false, bool FETCH = true>
-__global__ __launch_bounds__(256, FETCH ? 1 : 4) void rows_inv_kernel(RowArgs a) {
+__global__ __launch_bounds__(256, FETCH || Lanes<W>::P > 16 ? 1 : 4) void rows_inv_kernel(RowArgs a) {
   using LC = Lanes<W>;
   constexpr int TPR = LC::TPR, P = LC::P, WH = W / 2 + 1, NPRE = (WH + TPR - 1) / TPR;
-  constexpr bool PRE = FETCH && UNI && P <= 16;
+  constexpr bool PRE = FETCH && UNI;
   static_assert(2 * NPRE >= P, "the state's rows fit the registers of the spectra's");
   __shared__ __align__(16) float2 xch_all[LC::XCH];
   __shared__ float wpar[UNI ? 4 : 1][UNI ? LX_MAX_C * LX_MAX_K + 2 * LX_MAX_K : 1];
@@ -594,8 +594,8 @@ __global__ __launch_bounds__(256, FETCH ? 1 : 4) void rows_inv_kernel(RowArgs a)
   // PRE: a kernel's rows are loaded while the one before is transformed, the state's while the last is, so
   // that a wave waits for memory once per channel instead of once per kernel and once for the state.  168
   // VGPRs (3 waves per SIMD) instead of 127 (4): 79 -> 66 us for 64 3-channel 6-kernel worlds of 256^2 with
-  // statistics, whose 6144 waves are then two full rounds; 16 points a lane at most, as 24 and 32 are at 2
-  // waves without it, and not where a wave's lanes differ in their kernels (137 -> 175 VGPRs there).
+  // statistics, whose 6144 waves are then two full rounds; not where a wave's lanes differ in their kernels
+  // (137 -> 175 VGPRs there).  launch_rows_inv says for which grids.
   float2 pre0[NPRE], pre1[NPRE];
   auto fetch = [&](int k, int t) {
     const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;
@@ -942,22 +942,25 @@ int launch_rows_inv(const Geom& g, RowArgs ra, int64_t nimg, hipStream_t st) {
     if (int rc = ensure_tw<W>(st)) return rc;
     const dim3 grid(blocks_for(ra.npairs * Lanes<W>::TPR) + unsigned(ra.fin.blocks));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;  // waves never straddle images
-    // A grid that the chip holds at once without the early loads (4 waves per SIMD on 256 CUs) but not with
-    // them (3) takes them at a second, mostly empty round: 98 against 104 us a step for 42 3-channel 6-kernel
-    // worlds of 256^2 (1008 blocks); 768 blocks and from 1536 on they win (96 -> 87 and 191 -> 179 us).
-    if constexpr (W >= 128 && Lanes<W>::P == 16) {
-      if (uni && grid.x > 768 && grid.x <= 1024) {
-        if (ra.part) hipLaunchKernelGGL((rows_inv_kernel<W, true, true, false, false>), grid, dim3(256), 0, st, ra);
-        else hipLaunchKernelGGL((rows_inv_kernel<W, false, true, false, false>), grid, dim3(256), 0, st, ra);
-        return launched("rows_inv");
-      }
-    }
-    if (ra.part) {
-      if (uni) hipLaunchKernelGGL((rows_inv_kernel<W, true, true>), grid, dim3(256), 0, st, ra);
-      else hipLaunchKernelGGL((rows_inv_kernel<W, true, false>), grid, dim3(256), 0, st, ra);
-    } else {
-      if (uni) hipLaunchKernelGGL((rows_inv_kernel<W, false, true>), grid, dim3(256), 0, st, ra);
+    // Early loads (FETCH).  Up to 16 points a lane: unless the chip holds the grid at once without them (4
+    // waves per SIMD on 256 CUs) but not with them (3), where they take a second, mostly empty round: 98
+    // against 104 us a step for 42 3-channel 6-kernel worlds of 256^2 (1008 blocks); 768 blocks and from 1536
+    // on they win (96 -> 87 and 191 -> 179 us).  24 and 32 points: only where every CU has one block at most
+    // (1.25 to 1.5 times as fast there), as they hold more registers than two blocks leave.
+    constexpr bool few_points = Lanes<W>::P <= 16;
+    const bool fetch = few_points ? !(W >= 128 && grid.x > 768 && grid.x <= 1024) : grid.x <= 256;
+    auto go = [&](auto fetch_c) {
+      constexpr bool FETCH = decltype(fetch_c)::value != 0;
+      if (ra.part) hipLaunchKernelGGL((rows_inv_kernel<W, true, true, false, FETCH>), grid, dim3(256), 0, st, ra);
+      else hipLaunchKernelGGL((rows_inv_kernel<W, false, true, false, FETCH>), grid, dim3(256), 0, st, ra);
+    };
+    if (!uni) {
+      if (ra.part) hipLaunchKernelGGL((rows_inv_kernel<W, true, false>), grid, dim3(256), 0, st, ra);
       else hipLaunchKernelGGL((rows_inv_kernel<W, false, false>), grid, dim3(256), 0, st, ra);
+    } else if (fetch) {
+      go(IntC<1>{});
+    } else if constexpr (!few_points || W >= 128) {
+      go(IntC<0>{});
     }
     return launched("rows_inv");
   });
@@ -1624,7 +1627,7 @@ int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
     const dim3 grid(blocks_for(bucket * slot_pairs * Lanes<W>::TPR));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;
     if (uni) {
-      hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true>), grid, dim3(256), 0, st, ra);
+      hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, Lanes<W>::P <= 16>), grid, dim3(256), 0, st, ra);
     } else {
       hipLaunchKernelGGL((rows_inv_kernel<W, true, false, true>), grid, dim3(256), 0, st, ra);
     }

@@ -496,13 +496,30 @@ int by_length(int L, F&& f) {
   }
 }
 
-// Waves up to which a pass counts as a few worlds': two per SIMD (4 SIMDs x 256 CUs).  Up to there the
-// chip has idle issue slots for the repeated transforms and the barrier.  Beyond, measured at 12288 waves
-// (64 worlds of 256^2, 3 channels, 6 kernels, 10 steps): 2.28 ms with the general passes, 2.58 with these
-// rows, 3.08 with these lines.  Below, general -> these, us: inverse rows 10.2 -> 6.0 (1 x 256^2, one kernel),
-// 33 -> 7.9 (1 x 128^2, 3 channels, 15 kernels), 34 -> 23 (6 x 192 x 384, 5 kernels); convolution 6.7 -> 4.9,
-// 24 -> 4.9, 28 -> 12.
+// Waves up to which a pass counts as a few worlds': at most two per SIMD (4 SIMDs x 256 CUs).  The chip has
+// idle issue slots for the repeated transforms and the barriers up to a number that falls with the points a
+// lane holds and grows with the kernels per channel, which the general passes take in turn; measured (general
+// time / these, kernels spread over the channels) at 150 to 2000 waves of the general pass:
+//   inverse rows, 256 points: one kernel a channel 1.3 at 600, 0.95 at 1000; two 1.2 at 1000, 1.1 at 1500; five
+//     1.4 at 1000, 1.1 at 2000; 128 and 96 alike; 48 and 32 points above 1.1 throughout; 192: 1.0, 1.2 and 1.8
+//     at 1000 (one, two, five); 384: 1.1, 1.7, 2.7 at 300 and 0.7, 0.9, 1.3 at 1000
+//   convolution, 256 points: one kernel a channel 1.1 at 300 waves of its own, 0.9 at 600; two 1.2 at 1100;
+//     five 1.5 at 1450; 128: 1.06 at 600, 0.92 at 1000; 64 and fewer above 1.05 to 1500; 512: 1.04 at 300, 0.9 at
+//     600.
 constexpr int64_t kSmallWaves = 2048;
+
+int64_t small_conv_waves(int L, int C, int K) {
+  const int tpr = lx_row_tpr(L);
+  const int64_t one = tpr == 4 ? 2048 : tpr == 8 ? (L / tpr <= 16 ? 1024 : 512) : 384;
+  return std::min(kSmallWaves, one * std::max(C, K) / C);
+}
+
+// of the general pass, whose channels' waves count
+int64_t small_rows_waves(int W, int C, int K) {
+  const int tpr = lx_row_tpr(W), each = std::min(C, K);
+  const int64_t one = W <= 48 ? 2048 : W / tpr <= 16 ? 768 : tpr == 8 ? 512 : 256;
+  return std::min(kSmallWaves, one * (each + K) / (2 * each));
+}
 
 }  // namespace
 
@@ -511,7 +528,7 @@ int lx_small_conv(const LineArgs& a, int L, int64_t lines, bool list, hipStream_
   // spectra to keep are the single kernel's group's to write
   if (a.mode != 0 || (a.FA && !(a.C == 1 && a.K == 1)) || (a.dspec && (a.FA || a.kquad || list))) return LX_OK;
   const int64_t groups = lines / a.C * a.K, per = 64 / lx_row_tpr(L);
-  if ((groups + per - 1) / per > kSmallWaves) return LX_OK;
+  if ((groups + per - 1) / per > small_conv_waves(L, a.C, a.K)) return LX_OK;
   LxPassTables tb;
   if (int rc = lx_pass_tables(L, st, &tb)) return rc;
   SmallConv c;
@@ -542,8 +559,7 @@ int lx_small_rows(const RowArgs& a, int W, int64_t images, bool list, hipStream_
   *taken = 0;
   const int tpr = lx_row_tpr(W), K = a.K, C = a.C;
   const int64_t pairs = images / C * (a.rows / 2);
-  // the general pass takes a channel's kernels in turn, so its waves count
-  if (pairs * std::min(C, K) * tpr > kSmallWaves * 64) return LX_OK;
+  if (pairs * std::min(C, K) * tpr > small_rows_waves(W, C, K) * 64) return LX_OK;
   if (std::max({a.gf_bs, a.w_bs, a.dt_bs}) > INT32_MAX) return LX_OK;
   // 16-byte accesses: states, fields and potentials start on 16 bytes (rows are multiples of 4 floats)
   const auto wide = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
