@@ -1627,7 +1627,10 @@ int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
     const dim3 grid(blocks_for(bucket * slot_pairs * Lanes<W>::TPR));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;
     if (uni) {
-      hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, Lanes<W>::P <= 16>), grid, dim3(256), 0, st, ra);
+      if (Lanes<W>::P <= 16 || grid.x <= 256)  // early loads as in launch_rows_inv
+        hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, true>), grid, dim3(256), 0, st, ra);
+      else
+        hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, Lanes<W>::P <= 16>), grid, dim3(256), 0, st, ra);
     } else {
       hipLaunchKernelGGL((rows_inv_kernel<W, true, false, true>), grid, dim3(256), 0, st, ra);
     }
