@@ -272,9 +272,11 @@ constexpr int bitrev_n(int v, int n) {  // reverse the low log2(n) bits
 // Cross-lane DFT of size TPR over the lanes of a group, as a radix-2 network.
 // forward (decimation in frequency): natural lane order in, X_s at lane bitrev(s) out.
 // inverse (decimation in time):      X_s at lane bitrev(s) in, natural order out, x TPR.
-// Stage H pairs lane t with t ^ H; the upper lane's twiddle W_{2H}^(t mod H) is read from
-// the length-L table ``tw``.  Lower lanes use the twiddle 1 (an exact multiply), so the
-// stage needs no lane selects.  SPREAD = true: for 8-lane groups whose bit 2 is lane
+// Stage H pairs lane t with t ^ H; the upper lane's twiddle is read from the length-L table
+// ``tw``.  Lower lanes use the twiddle 1 (an exact multiply), so the stage needs no lane
+// selects.  Forward, where P is a multiple of TPR (lengths that fft_xlds takes as well), the
+// twiddle comes before the butterfly, as in fft_reg: both forms of a length then round alike,
+// and a step's result does not depend on which of them its pass uses.  SPREAD = true: for 8-lane groups whose bit 2 is lane
 // bit 3 (lanes {0..3, 8..11} + offset), so that t ^ 4 is one DPP row rotate.
 template <int H, bool SPREAD>
 LX_DEV float2 group_xor(float2 v, int lane) {
@@ -282,29 +284,34 @@ LX_DEV float2 group_xor(float2 v, int lane) {
   else return xor_fetch2<H>(v, lane);
 }
 
+// Twiddle of stage H in lane t: the factor of the lane's value before (FIRST) or after the butterfly
+template <int P, int TPR, bool INV, int H>
+struct LaneTwiddle {
+  static constexpr int L = P * TPR;
+  static constexpr bool CT = !INV && P % TPR == 0;
+  static constexpr bool FIRST = INV || CT, ANY = CT ? 2 * H < TPR : H > 1;
+  static LX_DEV float2 get(int t, const float2* tw) {
+    float2 w = make_float2(1.f, 0.f);
+    if constexpr (ANY) {
+      const float2 tv = tw[CT ? bitrev_n(t / (2 * H), TPR / (2 * H)) * (P * H) : (t & (H - 1)) * (L / (2 * H))];
+      w = (t & H) != 0 ? make_float2(tv.x, INV ? -tv.y : tv.y) : w;
+    }
+    return w;
+  }
+};
+
 template <int P, int TPR, int L, bool INV, int H, bool SPREAD>
 LX_DEV void lane_stage(float2* x, int t, int lane, const float2* tw) {
-  const bool upper = (t & H) != 0;
-  const float sgn = upper ? -1.f : 1.f;
-  float2 w = make_float2(1.f, 0.f);
-  if constexpr (H > 1) {
-    const float2 tv = tw[(t & (H - 1)) * (L / (2 * H))];
-    w = upper ? make_float2(tv.x, INV ? -tv.y : tv.y) : w;
-  }
-  if constexpr (!INV) {
+  using LT = LaneTwiddle<P, TPR, INV, H>;
+  static_assert(L == LT::L, "the table is of the network's own length");
+  const float sgn = (t & H) != 0 ? -1.f : 1.f;
+  const float2 w = LT::get(t, tw);
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
-      const float2 p = group_xor<H, SPREAD>(x[k], lane);
-      const float2 v = make_float2(fmaf(sgn, x[k].x, p.x), fmaf(sgn, x[k].y, p.y));
-      x[k] = (H > 1) ? cmul(v, w) : v;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < P; ++k) {
-      const float2 o = (H > 1) ? cmul(x[k], w) : x[k];
-      const float2 p = group_xor<H, SPREAD>(o, lane);
-      x[k] = make_float2(fmaf(sgn, o.x, p.x), fmaf(sgn, o.y, p.y));
-    }
+  for (int k = 0; k < P; ++k) {
+    const float2 o = LT::ANY && LT::FIRST ? cmul(x[k], w) : x[k];
+    const float2 p = group_xor<H, SPREAD>(o, lane);
+    const float2 v = make_float2(fmaf(sgn, o.x, p.x), fmaf(sgn, o.y, p.y));
+    x[k] = LT::ANY && !LT::FIRST ? cmul(v, w) : v;
   }
 }
 

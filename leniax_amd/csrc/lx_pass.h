@@ -82,18 +82,14 @@ LX_DEV float strided_pair(float v, float sgn, int lane) {
 // lane_stage (lx_device.h) over strided groups: the same arithmetic
 template <int P, int T, int L, bool INV, int H>
 LX_DEV void strided_stage(float2* x, int t, int lane, const float2* tw) {
-  const bool upper = (t & H) != 0;
-  const float sgn = upper ? -1.f : 1.f;
-  float2 w = make_float2(1.f, 0.f);
-  if constexpr (H > 1) {
-    const float2 tv = tw[(t & (H - 1)) * (L / (2 * H))];
-    w = upper ? make_float2(tv.x, INV ? -tv.y : tv.y) : w;
-  }
+  using LT = LaneTwiddle<P, T, INV, H>;
+  const float sgn = (t & H) != 0 ? -1.f : 1.f;
+  const float2 w = LT::get(t, tw);
 #pragma unroll
   for (int k = 0; k < P; ++k) {
-    const float2 o = INV && H > 1 ? cmul(x[k], w) : x[k];
+    const float2 o = LT::ANY && LT::FIRST ? cmul(x[k], w) : x[k];
     const float2 v = make_float2(strided_pair<H * (64 / T)>(o.x, sgn, lane), strided_pair<H * (64 / T)>(o.y, sgn, lane));
-    x[k] = !INV && H > 1 ? cmul(v, w) : v;
+    x[k] = LT::ANY && !LT::FIRST ? cmul(v, w) : v;
   }
 }
 template <int P, int T, int L, bool INV, int H>

@@ -6,7 +6,7 @@
 //   plane_inv:  half spectra -> columns along H -> rows along W -> growth, weighted sum, update
 //                                                                               (lines along H + rows_inv)
 //
-// Transforms run over lane groups with the cross-lane step on the DPP network (no exchange scratch, so that
+// Transforms run over lane groups with the cross-lane step between registers (no exchange scratch, so that
 // a plane of 96 x 96 takes 40 KB and four workgroups share a CU).  A plane's rows have stride 4 mod 8
 // complex: the 8 rows x 4 columns that 32 lanes read at once lie in different banks.
 // Measured, us, the passes they replace -> these: 16 worlds of 96^3, forward 46 -> 29 (115 MB: 4.0 TB/s), inverse
@@ -22,15 +22,18 @@ constexpr int plane_stride(int W) { return (W / 2 + 1 - 4 + 7) / 8 * 8 + 4; }
 constexpr size_t plane_lds(int H, int W) {  // the plane, then the tables of both axes (one if they are equal)
   return (size_t(H) * plane_stride(W) + H + (H == W ? 0 : W)) * sizeof(float2);
 }
-// threads: a lane group per row pair, 256 at most (96 x 96: 109 and 113 VGPRs, four workgroups of four waves
+// threads: a lane group per row pair, 256 at most (96 x 96: 103 and 128 VGPRs, four workgroups of four waves
 // per CU; 384 threads in one round of row pairs left two workgroups of six)
 constexpr int plane_threads(int H, int W) {
   return H / 2 * row_tpr(W) < 64 ? 64 : (H / 2 * row_tpr(W) > 256 ? 256 : (H / 2 * row_tpr(W) + 63) / 64 * 64);
 }
 
-template <int L>
+// A plane's transforms are spread over lanes as the rows' and the lines' of the passes are (lx_fft.hip), so that a
+// step rounds alike whichever takes it: columns of 96 points on 4 lanes (one round of 64 groups for 49 columns
+// instead of two of 32: a step of 16 worlds of 96^3 133 -> 129 us, gradients of 8 1517 -> 1481 us).
+template <int L, int T = row_tpr(L)>
 struct PlaneFft {
-  static constexpr int TPR = row_tpr(L), P = L / TPR;
+  static constexpr int TPR = T, P = L / TPR;
   // frequency held by register e of lane t
   static LX_DEV int freq(int t, int e) { return e + P * bitrev_n(t, TPR); }
 };
@@ -94,7 +97,7 @@ LX_DEV void pair_inverse(float2* x, int t, int lane, const float2* tw, const flo
 // Columns of the plane in LDS -> half spectra of the plane in memory
 template <int H, int W>
 LX_DEV void columns_out(const float2* plane, const float2* tw, float2* S) {
-  using F = PlaneFft<H>;
+  using F = PlaneFft<H, line_tpr(H, 1)>;
   constexpr int TPR = F::TPR, P = F::P, WH = W / 2 + 1, RS = plane_stride(W), NC = plane_threads(H, W) / TPR;
   using SG = Strided<TPR>;  // a wave's lanes: neighbouring columns side by side
 #pragma unroll 1
@@ -117,7 +120,7 @@ LX_DEV void columns_out(const float2* plane, const float2* tw, float2* S) {
 // Half spectra of the plane in memory -> columns transformed back in LDS
 template <int H, int W>
 LX_DEV void columns_in(float2* plane, const float2* tw, const float2* U) {
-  using F = PlaneFft<H>;
+  using F = PlaneFft<H, line_tpr(H, 2)>;
   constexpr int TPR = F::TPR, P = F::P, WH = W / 2 + 1, RS = plane_stride(W), NC = plane_threads(H, W) / TPR;
   using SG = Strided<TPR>;  // a wave's lanes: neighbouring columns side by side
 #pragma unroll 1

@@ -1,0 +1,83 @@
+"""One 3-D step gives the same bits whichever entry point takes it: whole planes (lx_plane.hip: lx_update on
+arrays that start on 16 bytes), the passes for rows and lines (arrays that do not; steps with statistics),
+and the live list of lx_run.  Every side that the plane kernels take, with one channel and kernel (the update
+inside the plane kernel) and with several (the update from the potentials)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from test_gpu_plane import _shifted
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip('torch')
+
+SIDES = (32, 48, 64, 96, 128)
+
+
+def _case(dims, B, C, K, gf='gaussian', average=False, seed=0):
+    from leniax_amd import _lib, engine
+    rng = np.random.default_rng(seed + dims[1] + 1000 * dims[2])
+    rule = engine.make_rule(list(dims), C, [k % C for k in range(K)], [_lib.GROWTH_IDS[gf]] * K, 0, average)
+    kern = rng.random((K,) + dims)
+    half = np.fft.rfftn(kern / kern.sum(axis=(1, 2, 3), keepdims=True), axes=(1, 2, 3))
+    Kh = torch.as_tensor(half.astype(np.complex64)).cuda()[None].contiguous()
+    gfd = torch.as_tensor(rng.uniform(0.3, 0.6, (K, 2)).astype(np.float32)).cuda()
+    w = torch.as_tensor(rng.uniform(0.2, 1, (C, K)).astype(np.float32)).cuda()
+    A = torch.as_tensor(rng.random((B, C) + dims, dtype=np.float32)).cuda()
+    return rule, Kh, gfd, w, A
+
+
+def _update(rule, Kh, gf, w, A, dt=0.1, pot=True, move=lambda t: t):
+    """lx_update_dt's state, field and (pot) potentials."""
+    from leniax_amd import _lib, core, engine
+    B, dims = A.shape[0], tuple(A.shape[2:])
+    A = move(A)
+    new, field = move(torch.empty_like(A)), move(torch.empty_like(A))
+    u = move(torch.empty((B, rule.K) + dims, device='cuda')) if pot else None
+    _lib.call('lx_update_dt', ctypes.byref(rule), engine.ptr(A), B, engine.ptr(Kh), 0, engine.ptr(gf), 0,
+              engine.ptr(w), 0, dt, engine.ptr(new), engine.ptr(field), engine.ptr(u),
+              engine.ptr(core._workspace(rule, B)), engine.stream_ptr())
+    return (new, field, u) if pot else (new, field)
+
+
+@pytest.mark.parametrize('C,K', [(1, 1), (2, 2)])
+@pytest.mark.parametrize('H', SIDES)
+def test_entry_points_agree_bit_for_bit(H, C, K):
+    from leniax_amd import engine, runner
+    for W in SIDES:
+        print('same bits', (16, H, W), C, K, flush=True)
+        rule, Kh, gf, w, A = _case((16, H, W), 3, C, K)
+        planes = _update(rule, Kh, gf, w, A)
+        general = _update(rule, Kh, gf, w, A, move=_shifted)
+        bad = [n for n, a, b in zip(('state', 'field', 'potential'), planes, general) if not torch.equal(a, b)]
+        assert not bad, ('planes against rows and lines', H, W, bad)
+        dt = torch.tensor([0.1]).cuda()
+        rows, n, fin, hist = runner._scan_plain(rule, None, A, Kh, 0, gf, w, dt, 1, 9., 10., True)
+        assert torch.equal(fin, planes[0]) and torch.equal(hist[1][0], planes[1]) and torch.equal(hist[2][0], planes[2])
+        second = _update(rule, Kh, gf, w, planes[0])[0]
+        # fewer slots than worlds: the live list
+        r = engine.run_batched(rule, A, Kh, False, gf[None], w[None], dt, 2, 'none', 0, 9., 10., slots=2)
+        assert torch.equal(r['cells'], second), ('live list', H, W)
+
+
+@pytest.mark.parametrize('dims', [(16, 32, 128), (32, 128, 96), (96, 96, 96), (48, 64, 64), (128, 48, 128)])
+def test_transforms_agree_bit_for_bit(dims):
+    """rfftn and irfftn of arrays that start on 16 bytes (planes) and of arrays that do not."""
+    from leniax_amd import _lib, engine
+    print('same bits, transforms', dims, flush=True)
+    rng = np.random.default_rng(1)
+    x = torch.as_tensor(rng.random((2,) + dims, dtype=np.float32)).cuda()
+    cd = (ctypes.c_int32 * 3)(*dims)
+    spectra, backs = [], []
+    for move in (lambda t: t, _shifted):
+        a = move(x)
+        X = torch.empty((2,) + dims[:2] + (dims[2] // 2 + 1,), dtype=torch.complex64, device='cuda')
+        _lib.call('lx_rfft2', 3, cd, 2, engine.ptr(a), engine.ptr(X), engine.stream_ptr())
+        back, work = move(torch.empty_like(x)), torch.empty_like(X)
+        _lib.call('lx_irfft2', 3, cd, 2, engine.ptr(X), engine.ptr(back), engine.ptr(work), engine.stream_ptr())
+        spectra.append(X)
+        backs.append(back)
+    assert torch.equal(torch.view_as_real(spectra[0]), torch.view_as_real(spectra[1]))
+    assert torch.equal(backs[0], backs[1])
