@@ -299,8 +299,11 @@ __global__ __launch_bounds__(plane_threads(H, W)) void plane_inv_kernel(PlaneInv
       const int64_t o = row * W + col;
       if (a.pot) *reinterpret_cast<float4*>(a.pot + p * a.pot_stride + o) = u;
       if (!a.update) continue;
-      growth(u);
-      float4 g = add_weighted(make_float4(0.f, 0.f, 0.f, 0.f), wk, u);
+      float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (wk != 0.f || a.pot) {  // a kernel without weight counts (times 0) only where its potential is wanted
+        growth(u);
+        g = add_weighted(g, wk, u);
+      }
       if (a.average) {
         const float den = add_nc(0.f, wk);
         g = make_float4(g.x / den, g.y / den, g.z / den, g.w / den);

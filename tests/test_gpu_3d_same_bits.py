@@ -81,3 +81,21 @@ def test_transforms_agree_bit_for_bit(dims):
         backs.append(back)
     assert torch.equal(torch.view_as_real(spectra[0]), torch.view_as_real(spectra[1]))
     assert torch.equal(backs[0], backs[1])
+
+
+@pytest.mark.parametrize('average', [False, True])
+def test_a_kernel_without_weight_adds_nothing(average):
+    """One channel, one kernel of weight 0, a state with a NaN: where no potential is asked for, the kernel is
+    left out (0 times its growth would be NaN in every cell), by planes as by the row pass; where one is, it
+    counts as 0 times the growth in both."""
+    print('weight 0', average, flush=True)
+    rule, Kh, gf, w, A = _case((16, 32, 48), 2, 1, 1, average=average)
+    w.zero_()
+    A[0, 0, 3, 5, 7] = float('nan')
+    for pot in (False, True):
+        outs = [_update(rule, Kh, gf, w, A, pot=pot, move=move) for move in (lambda t: t, _shifted)]
+        for a, b in zip(*outs):
+            assert torch.equal(a.isnan(), b.isnan())
+            assert torch.equal(a.nan_to_num(nan=-7.), b.nan_to_num(nan=-7.))
+        if not pot and not average:
+            assert int(outs[0][0].isnan().sum()) == 1
