@@ -315,7 +315,8 @@ __global__ __launch_bounds__(plane_threads(H, W)) void plane_inv_kernel(PlaneInv
 }
 
 // The update from the potentials of several kernels: growth, weighted sum in the kernels' order, state.
-// One block per four-point slice of one channel image (grid: slices x B C).
+// One block per 256 four-point items of one channel image, then of the image gridDim.y further on (images are
+// any number, a grid's y dimension is at most kGridY).
 struct Points {
   const float* pot;  // kernel k of world b, plane d at pot + ((b K + k) D + d) pot_stride
   int64_t pot_stride;
@@ -327,17 +328,21 @@ struct Points {
   const float* dt;
   uint64_t kinds, cins;
   int64_t gf_bs, w_bs, dt_bs;
+  int64_t images;
   int D, cells, C, K, state_fn, average, sel, want_all;  // cells: of a plane; want_all: potentials are the caller's
   float dt_val;
 };
 
-__global__ __launch_bounds__(256) void points_kernel(Points a) {
-  const int b = blockIdx.y / a.C, c = blockIdx.y - b * a.C;
+constexpr int64_t kGridY = 65535;
+
+LX_DEV void points_of(const Points& a, int64_t img) {
+  const int64_t b = img / a.C;
+  const int c = int(img - b * a.C);
   const int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x;  // four-point item of the image
   const int per_plane = a.cells / 4;
   if (q >= int64_t(a.D) * per_plane) return;
   const int d = int(q / per_plane);
-  const int64_t o = (q - int64_t(d) * per_plane) * 4, io = int64_t(blockIdx.y) * a.D * a.cells + q * 4;
+  const int64_t o = (q - int64_t(d) * per_plane) * 4, io = img * a.D * a.cells + q * 4;
   const float* w = a.sel ? nullptr : a.w + b * a.w_bs;
   const float* gf = a.sel ? nullptr : a.gf + b * a.gf_bs;
   const float4 v = *reinterpret_cast<const float4*>(a.A + io);
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(256) void points_kernel(Points a) {
       for (int cc = 1; cc < a.C && !skip; ++cc) skip = w[cc * a.K + k] != 0.f;
       if (skip) continue;
     }
-    float4 u = *reinterpret_cast<const float4*>(a.pot + ((int64_t(b) * a.K + k) * a.D + d) * a.pot_stride + o);
+    float4 u = *reinterpret_cast<const float4*>(a.pot + ((b * a.K + k) * a.D + d) * a.pot_stride + o);
     if (!a.sel) Growth(int(a.kinds >> (4 * k)) & 15, gf[2 * k], gf[2 * k + 1])(u);
     G = add_weighted(G, wk, u);
   }
@@ -360,6 +365,10 @@ __global__ __launch_bounds__(256) void points_kernel(Points a) {
   if (a.field) *reinterpret_cast<float4*>(a.field + io) = G;
   const float dtw = a.sel ? 1.f : a.dt ? a.dt[b * a.dt_bs] : a.dt_val;
   *reinterpret_cast<float4*>(a.A_out + io) = step_four(a.state_fn, v, G, dtw);
+}
+
+__global__ __launch_bounds__(256) void points_kernel(Points a) {
+  for (int64_t img = blockIdx.y; img < a.images; img += gridDim.y) points_of(a, img);
 }
 
 // One channel, one kernel, reverse: the planes of rows_fwd_adj_kernel (lx_fft.hip) and of the lines beside
@@ -665,10 +674,12 @@ int lx_plane_inv(const RowArgs& a, int D, int H, int W, int64_t images, hipStrea
     q.kinds |= uint64_t(a.gfk[k] & 15) << (4 * k);
     q.cins |= uint64_t(a.cin[k] & 15) << (4 * k);
   }
-  q.D = D; q.cells = H * W; q.C = a.C; q.K = a.K; q.state_fn = a.state_fn; q.average = a.average; q.sel = a.sel;
+  q.images = images; q.D = D; q.cells = H * W; q.C = a.C; q.K = a.K;
+  q.state_fn = a.state_fn; q.average = a.average; q.sel = a.sel;
   q.want_all = a.pot != nullptr; q.dt_val = a.dt_val;
   const int64_t items = int64_t(D) * H * W / 4;
-  hipLaunchKernelGGL(points_kernel, dim3(unsigned((items + 255) / 256), unsigned(images)), dim3(256), 0, st, q);
+  hipLaunchKernelGGL(points_kernel, dim3(unsigned((items + 255) / 256), unsigned(std::min(images, kGridY))),
+                     dim3(256), 0, st, q);
   return launched("points");
 }
 
@@ -678,7 +689,7 @@ int lx_shared_conv(const LineArgs& a, int L, int64_t images, hipStream_t st, int
   SharedConv c;
   c.lines = a.A * a.WH; c.st = int(a.st);
   // lines of an image are contiguous where the convolution axis is the outermost of three
-  if (a.A < 2 || a.a_stride != a.WH || images > 65535) return LX_OK;
+  if (a.A < 2 || a.a_stride != a.WH || images > kGridY) return LX_OK;
   const int64_t waves = images * c.lines * lx_row_tpr(L) / 64;
   // worlds per group: as many as leave about three waves per SIMD (16 worlds of 96^3: 1, 2, 3, 4, 8 worlds
   // 38.7, 33.8, 32.1, 35.3, 46.1 us)

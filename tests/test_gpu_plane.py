@@ -106,3 +106,16 @@ def test_reverse_steps_agree_with_the_general_passes(slug, ste):
         print(slug, ste, name, err, flush=True)
         # five steps of float32 transforms either way: 1e-4 is the single steps' own bound against float64
         assert err <= 1e-4 or name == 'w', (name, err)
+
+
+def test_more_images_than_a_grid_dimension_holds():
+    """32770 worlds of two channels (65540 images, past the 65535 of a grid's y dimension): five different worlds
+    over and over, each copy equal to the world stepped in a batch of five."""
+    from test_gpu_3d_same_bits import _case, _update
+    rule, Kh, gf, w, A = _case((16, 32, 32), 5, 2, 1)
+    few = _update(rule, Kh, gf, w, A, pot=False)
+    copies = 6554
+    many = _update(rule, Kh, gf, w, A.repeat(copies, 1, 1, 1, 1), pot=False)
+    for a, b in zip(few, many):
+        b = b.view((copies,) + tuple(a.shape))
+        assert bool((b == a).all())
