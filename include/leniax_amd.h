@@ -389,14 +389,18 @@ int lx_run_static(const lx_rule* rule, const lx_run_args* args, void* stream);
  *                  lane, transpose through LDS) or 8 (12 points, DPP network);
  *   "fused_probe"  fused early-stop run: first launch steps every world max_steps / value steps
  *                  (0: one launch);
- *   "graph_steps"  multi-pass lx_run: steps per captured graph.
+ *   "graph_steps"  multi-pass lx_run: steps per captured graph (a run without a stop policy and with every
+ *                  world in flight captures none unless the knob is pinned).
  * LX_TUNE_OFF (the default, or LENIAX_AMD_TUNE=0): fixed rules.  LX_TUNE_ON: the first call of a
  * shape times the candidates on its own inputs (outside stream capture) and keeps the fastest, in
  * memory and in the cache file (LENIAX_AMD_TUNE_CACHE or lx_tune_cache).  LX_TUNE_CACHED: decisions
- * from memory / the cache file, fixed rules otherwise.  lx_tune_force pins a knob for every shape
- * (value < 0 unpins).  lx_autotune returns the previous mode; lx_tune_report writes "knob key value"
- * lines (forced knobs first) and returns the text's length.  No counterpart in leniax, whose
- * schedules are XLA's (leniax/core.py:76-87). */
+ * from memory / the cache file, fixed rules otherwise.  Passes of a few worlds, of 3-D worlds that share
+ * a spectrum and of whole 3-D planes have kernels of their own without these variants, chosen by shape
+ * before a decision is asked for; lines96_tpr is no candidate for planes that those kernels take (every
+ * entry point then rounds alike).  lx_tune_force pins a knob for every shape, these included: their
+ * passes then run in the pinned variant (value < 0 unpins).  lx_autotune returns the previous mode;
+ * lx_tune_report writes "knob key value" lines (forced knobs first) and returns the text's length.  No
+ * counterpart in leniax, whose schedules are XLA's (leniax/core.py:76-87). */
 #define LX_TUNE_OFF 0
 #define LX_TUNE_ON 1
 #define LX_TUNE_CACHED 2

@@ -838,11 +838,20 @@ void lines_key(char* key, size_t n, const LineArgs& la, int L, int64_t lines, bo
            list ? "list" : "plain", la.mode == 0 && la.kquad ? ":quadrant" : "");
 }
 
+// Whether a knob that a line pass of length L has is pinned: it then holds for every shape, so the pass is
+// lines_kernel's or conv_staged_kernel's, not one without such variants (a few worlds, a shared spectrum, planes).
+bool line_knob_pinned(const LineArgs& la, int L) {
+  return lx_tune_forced("line_xcd") || (L == 96 && lx_tune_forced("lines96_tpr")) ||
+         (staged_eligible(la, L) && lx_tune_forced("conv_staged"));
+}
+
 // The variant of a line pass: forced knobs, then a recorded decision, then (tuning on) the fastest
 // candidate timed by run(v) -- which launches v on buffers it may overwrite -- then the fixed rule.
+// planes: lines along H of planes that the plane kernels take where they can: at 96 points these keep the
+// planes' factorisation unless the knob is pinned, so that a step's bits do not depend on its entry point.
 template <class Run>
-LineVariant choose_lines(const LineArgs& la, int L, int64_t lines, bool list, bool can_time, hipStream_t st,
-                         Run&& run) {
+LineVariant choose_lines(const LineArgs& la, int L, int64_t lines, bool list, bool planes, bool can_time,
+                         hipStream_t st, Run&& run) {
   char key[160];
   lines_key(key, sizeof(key), la, L, lines, list);
   LineVariant d = default_variant(la, L, lines), v = d;
@@ -851,12 +860,13 @@ LineVariant choose_lines(const LineArgs& la, int L, int64_t lines, bool list, bo
   if (hs) fs = val;
   const bool hx = lx_tune_lookup("line_xcd", key, &val) != 0;
   if (hx) fx = val;
-  const bool ht = lx_tune_lookup("lines96_tpr", key, &val) != 0;
+  const bool fixed96 = planes && !lx_tune_forced("lines96_tpr");
+  const bool ht = !fixed96 && lx_tune_lookup("lines96_tpr", key, &val) != 0;
   if (ht) ft = val;
   if (hs) v.staged = staged_eligible(la, L) && fs != 0;
   if (hx) v.xcd = fx != 0;
   if (ht && L == 96) v.tpr = ft == 4 ? 4 : 8;
-  const bool all_known = (hs || !staged_eligible(la, L)) && hx && (ht || L != 96);
+  const bool all_known = (hs || !staged_eligible(la, L)) && hx && (ht || fixed96 || L != 96);
   if (all_known || !can_time || !lx_tune_should_time(st)) return v;
   // time every candidate the known values leave open
   LineVariant best = v;
@@ -868,7 +878,7 @@ LineVariant choose_lines(const LineArgs& la, int L, int64_t lines, bool list, bo
       if (hx && x != v.xcd) continue;
       for (int t : {4, 8, 16}) {
         if (L == 96 ? (t != 4 && t != 8) : t != row_tpr(L)) continue;
-        if (ht && L == 96 && t != v.tpr) continue;
+        if ((ht || fixed96) && L == 96 && t != v.tpr) continue;
         if (s && t != line_tpr(L, 0)) continue;
         LineVariant c{s, x, t};
         const float ms = lx_time_ms(st, 3, [&] { return run(c); });
@@ -882,7 +892,7 @@ LineVariant choose_lines(const LineArgs& la, int L, int64_t lines, bool list, bo
   if (best_ms < 0.f) return d;
   if (staged_eligible(la, L)) lx_tune_record("conv_staged", key, best.staged);
   lx_tune_record("line_xcd", key, best.xcd);
-  if (L == 96) lx_tune_record("lines96_tpr", key, best.tpr);
+  if (L == 96 && !fixed96) lx_tune_record("lines96_tpr", key, best.tpr);
   return best;
 }
 
@@ -892,9 +902,12 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
   la.k_elems = la.kquad ? int64_t(g.L[0] / 2 + 1) * g.WH : g.half;
   la.nlines = nimg * g.A[axis] * int64_t(g.WH);
   const int L = g.L[axis];
-  int taken = 0;
-  if (int rc = lx_small_conv(la, L, la.nlines, false, st, &taken); rc || taken) return rc;
-  if (int rc = lx_shared_conv(la, L, nimg, st, &taken); rc || taken) return rc;
+  const bool planes = axis == 1 && lx_plane_takes(g.L[1], g.W);
+  if (!line_knob_pinned(la, L)) {
+    int taken = 0;
+    if (int rc = lx_small_conv(la, L, la.nlines, false, st, &taken); rc || taken) return rc;
+    if (int rc = lx_shared_conv(la, L, nimg, st, &taken); rc || taken) return rc;
+  }
   if (int rc = dispatch_len(L, [&](auto l) { return ensure_tw<decltype(l)::value>(st); })) return rc;
   // timing is safe where the pass can run again on its own inputs: a convolution into another
   // buffer with no accumulated kernel gradient, an out-of-place inverse; in-place passes are timed
@@ -913,7 +926,8 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
     char key[160];
     lines_key(key, sizeof(key), la, L, la.nlines, false);
     int val = 0;
-    const bool known = lx_tune_lookup("line_xcd", key, &val) && (L != 96 || lx_tune_lookup("lines96_tpr", key, &val));
+    const bool known = lx_tune_lookup("line_xcd", key, &val) &&
+                       (L != 96 || planes || lx_tune_lookup("lines96_tpr", key, &val));
     if (!known && hipMalloc(reinterpret_cast<void**>(&tmp), bytes) == hipSuccess) {
       if (hipMemcpyAsync(tmp, la.S, bytes, hipMemcpyDeviceToDevice, st) != hipSuccess) {
         hipFree(tmp);
@@ -923,7 +937,7 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
       tmp = nullptr;
     }
   }
-  const LineVariant v = choose_lines(la, L, la.nlines, false, can_time && (idem || tmp), st, run);
+  const LineVariant v = choose_lines(la, L, la.nlines, false, planes, can_time && (idem || tmp), st, run);
   if (tmp) {
     hipStreamSynchronize(st);
     hipFree(tmp);
@@ -986,9 +1000,13 @@ RowArgs row_args(const lx_rule* rule) {
   return ra;
 }
 
-// Whether a 3-D pass takes the plane kernels: their sides, and arrays that start on 16 bytes.
+// Whether a 3-D pass takes the plane kernels: their sides, arrays that start on 16 bytes, no pinned knob of the
+// lines along H.
 bool takes_planes(const Geom& g, std::initializer_list<const void*> arrays) {
   if (g.naxes != 2 || !lx_plane_takes(g.L[1], g.W)) return false;
+  LineArgs along_h = line_args();
+  along_h.mode = 1;
+  if (line_knob_pinned(along_h, g.L[1])) return false;
   for (const void* p : arrays)
     if (reinterpret_cast<uintptr_t>(p) % 16) return false;
   return true;
@@ -1527,11 +1545,12 @@ int run_lines(const PassesRun& r, const RunView& rv, int bucket, int axis, LineA
   la.list = rv.list; la.nlive = rv.nlive;
   const int L = g.L[axis];
   const int64_t lines = la.nlines * bucket;
-  if (!tune) {
+  const bool planes = axis == 1 && lx_plane_takes(g.L[1], g.W);
+  if (!tune && !line_knob_pinned(la, L)) {
     int taken = 0;
     if (int rc = lx_small_conv(la, L, lines, true, st, &taken); rc || taken) return rc;
   }
-  const LineVariant v = choose_lines(la, L, lines, true, tune, st,
+  const LineVariant v = choose_lines(la, L, lines, true, planes, tune, st,
                                      [&](LineVariant c) { return launch_lines_v<true>(la, L, lines, c, st); });
   return tune ? LX_OK : launch_lines_v<true>(la, L, lines, v, st);
 }
@@ -1787,7 +1806,7 @@ int lx_passes_run(const lx_rule* rule, const lx_run_args* a, hipStream_t st) {
     r.rv[p] = RunView{p ? r.ctl.list1 : r.ctl.list0, r.ctl.nlive + p, r.ctl.carry, X0, X1, elems};
   int rc = warm_tables(r.g, st);
   if (rc) return rc;
-  if (a->stop_policy == LX_STOP_NONE && a->B == cap) {
+  if (a->stop_policy == LX_STOP_NONE && a->B == cap && !lx_tune_forced("graph_steps")) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
       return lx_fail(LX_EDEVICE, "lx_run: the multi-pass run cannot be captured");

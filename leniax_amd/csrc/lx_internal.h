@@ -383,9 +383,10 @@ float* lx_adj_work_11(const lx_rule* r, int64_t B, void* work);
 
 // Autotuner (lx_tune.hip): knob values by launch shape.  lx_tune_lookup gives a forced or recorded
 // value (1) or nothing (0); lx_tune_should_time says whether a launcher may time its candidates now
-// (tuning on, stream not capturing).
+// (tuning on, stream not capturing); lx_tune_forced says whether the knob is pinned.
 int lx_tune_mode();
 int lx_tune_lookup(const char* knob, const char* key, int* value);
+bool lx_tune_forced(const char* knob);
 void lx_tune_record(const char* knob, const char* key, int value);
 bool lx_tune_should_time(hipStream_t st);
 // While one of these lives on a thread, lx_tune_should_time is false there: the launches it covers

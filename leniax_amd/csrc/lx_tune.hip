@@ -12,6 +12,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -23,6 +24,7 @@ namespace {
 struct Store {
   std::mutex mu;
   std::map<std::string, int> forced;     // knob -> value
+  std::atomic<int> nforced{0};           // its size, read without the lock
   std::map<std::string, int> decided;    // "knob key" -> value
   std::string path;
   bool loaded = false;
@@ -78,6 +80,13 @@ int lx_tune_lookup(const char* knob, const char* key, int* value) {
   if (d == s.decided.end()) return 0;
   *value = d->second;
   return 1;
+}
+
+bool lx_tune_forced(const char* knob) {
+  Store& s = store();
+  if (!s.nforced.load(std::memory_order_acquire)) return false;
+  std::lock_guard<std::mutex> lock(s.mu);
+  return s.forced.count(knob) != 0;
 }
 
 void lx_tune_record(const char* knob, const char* key, int value) {
@@ -136,6 +145,7 @@ extern "C" int lx_tune_force(const char* knob, int32_t value) {
   std::lock_guard<std::mutex> lock(s.mu);
   if (value < 0) s.forced.erase(knob);
   else s.forced[knob] = value;
+  s.nforced.store(int(s.forced.size()), std::memory_order_release);
   return LX_OK;
 }
 

@@ -174,3 +174,73 @@ def test_autotune_records_reuses_and_agrees(knobs, tmp_path):
     for x, y in zip(again, ref):
         assert torch.equal(x, y)
     assert len(cache.read_text().splitlines()) == len(lines)  # nothing timed again
+
+
+def _kernels(fn):
+    """The names of the kernels that fn launches (a graph's included)."""
+    from torch.profiler import ProfilerActivity, profile
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    return {e.key for e in p.key_averages()}
+
+
+def _potential(dims, B, K=1):
+    """lx_potential of B one-channel worlds as a call, and its output."""
+    from leniax_amd import core, engine, _lib
+    rng = np.random.default_rng(len(dims) + B)
+    axes = tuple(range(1, len(dims) + 1))
+    kern = rng.random((K,) + dims)
+    Kh = torch.as_tensor(np.fft.rfftn(kern / kern.sum(axis=axes, keepdims=True), axes=axes).astype(np.complex64)).cuda()
+    rule = engine.make_rule(list(dims), 1, [0] * K, [_lib.GROWTH_IDS['gaussian']] * K, 0, 1)
+    A = torch.as_tensor(rng.random((B, 1) + dims, dtype=np.float32)).cuda()
+    pot = torch.empty((B, K) + dims, device='cuda')
+    work = core._workspace(rule, B)
+    return lambda: _lib.call('lx_potential', ctypes.byref(rule), engine.ptr(A), B, engine.ptr(Kh), 0, engine.ptr(pot),
+                             engine.ptr(work), engine.stream_ptr()), pot
+
+
+@pytest.mark.parametrize('dims,B,knob,value,own,pinned', [
+    ((256, 256), 1, 'conv_staged', 1, 'small_conv_kernel<256', 'conv_staged_kernel<256'),
+    ((256, 256), 1, 'conv_staged', 0, 'small_conv_kernel<256', 'lines_kernel<256, 0'),
+    ((64, 64), 2, 'line_xcd', 0, 'small_conv_kernel<64', 'lines_kernel<64, 0'),
+    ((96, 64), 2, 'lines96_tpr', 4, 'small_conv_kernel<96', 'lines_kernel<96, 0, false, 4'),
+    ((32, 96, 96), 16, 'line_xcd', 1, 'plane_fwd_kernel<96, 96', 'lines_kernel<96, 1'),
+    ((96, 96, 96), 12, 'lines96_tpr', 8, 'shared_conv_kernel<96', 'lines_kernel<96, 0, false, 8'),
+    ((16, 96, 32), 2, 'lines96_tpr', 4, 'plane_inv_kernel<96, 32', 'lines_kernel<96, 2, false, 4'),
+    ((16, 96, 32), 2, 'lines96_tpr', 8, 'plane_inv_kernel<96, 32', 'lines_kernel<96, 2, false, 8')])
+def test_a_pinned_knob_holds_for_every_shape(knobs, dims, B, knob, value, own, pinned):
+    """Also for the shapes that have kernels of their own without the variant (a few worlds, a shared
+    spectrum, planes); the potential's bits stay, but for the other factorisation of 96 points."""
+    print('pinned', dims, B, knob, value, flush=True)
+    call, pot = _potential(dims, B)
+    has = lambda names, part: any(part in n for n in names)  # noqa: E731
+    names = _kernels(call)
+    assert has(names, own) and not has(names, pinned), names
+    ref = pot.clone()
+    knobs.tune_force(knob, value)
+    names = _kernels(call)
+    assert has(names, pinned) and not has(names, own), names
+    if knob != 'lines96_tpr':
+        assert torch.equal(pot, ref)
+    else:
+        assert float((pot - ref).abs().max()) <= 4e-6 * float(ref.abs().max())  # each within 2e-6 of the oracle
+
+
+def test_pinned_graph_steps_hold_without_a_stop_policy(knobs):
+    from test_gpu_run import _uneven_case
+    from leniax_amd import engine
+    rule, Kh, gf, w, a0 = _uneven_case()
+    dt = torch.tensor([0.1], device=a0.device)
+    res = {}
+
+    def run():
+        res.update(engine.run_batched(rule, a0, Kh, True, gf, w, dt, 9, 'none', 0, 10., 10., want_stats=True))
+    assert not any('run_control_kernel' in n for n in _kernels(run))
+    ref = dict(res)
+    knobs.tune_force('graph_steps', 4)
+    assert any('run_control_kernel' in n for n in _kernels(run))
+    for key in ('cells', 'stats', 'n', 'steps'):
+        assert torch.equal(res[key], ref[key]), key
