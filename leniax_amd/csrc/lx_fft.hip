@@ -945,6 +945,18 @@ int launch_lines(const Geom& g, int axis, LineArgs la, int64_t nimg, hipStream_t
   return launch_lines_v<false>(la, L, la.nlines, v, st);
 }
 
+// Whether the inverse rows of so many workgroups load ahead (FETCH).  Up to 16 points a lane: unless the chip
+// holds the grid at once without early loads (4 waves per SIMD on 256 CUs) but not with them (3), where they
+// take a second, mostly empty round: 98 against 104 us a step for 42 3-channel 6-kernel worlds of 256^2 (1008
+// blocks), 115 against 123 with a live list; 768 blocks and from 1536 on they win (96 -> 87 and 191 -> 179 us).
+// 24 and 32 points: only where every CU has one block at most (1.25 to 1.5 times as fast there), as they hold
+// more registers than two blocks leave.
+template <int W>
+bool rows_load_ahead(unsigned blocks) {
+  if (Lanes<W>::P <= 16) return !(W >= 128 && blocks > 768 && blocks <= 1024);
+  return blocks <= 256;
+}
+
 int launch_rows_inv(const Geom& g, RowArgs ra, int64_t nimg, hipStream_t st) {
   ra.rows = g.rows;
   ra.npairs = nimg * (g.rows / 2);
@@ -956,13 +968,8 @@ int launch_rows_inv(const Geom& g, RowArgs ra, int64_t nimg, hipStream_t st) {
     if (int rc = ensure_tw<W>(st)) return rc;
     const dim3 grid(blocks_for(ra.npairs * Lanes<W>::TPR) + unsigned(ra.fin.blocks));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;  // waves never straddle images
-    // Early loads (FETCH).  Up to 16 points a lane: unless the chip holds the grid at once without them (4
-    // waves per SIMD on 256 CUs) but not with them (3), where they take a second, mostly empty round: 98
-    // against 104 us a step for 42 3-channel 6-kernel worlds of 256^2 (1008 blocks); 768 blocks and from 1536
-    // on they win (96 -> 87 and 191 -> 179 us).  24 and 32 points: only where every CU has one block at most
-    // (1.25 to 1.5 times as fast there), as they hold more registers than two blocks leave.
     constexpr bool few_points = Lanes<W>::P <= 16;
-    const bool fetch = few_points ? !(W >= 128 && grid.x > 768 && grid.x <= 1024) : grid.x <= 256;
+    const bool fetch = rows_load_ahead<W>(grid.x);
     auto go = [&](auto fetch_c) {
       constexpr bool FETCH = decltype(fetch_c)::value != 0;
       if (ra.part) hipLaunchKernelGGL((rows_inv_kernel<W, true, true, false, FETCH>), grid, dim3(256), 0, st, ra);
@@ -1645,14 +1652,11 @@ int enqueue_step(const PassesRun& r, int par, int bucket, hipStream_t st) {
     constexpr int W = decltype(w)::value;
     const dim3 grid(blocks_for(bucket * slot_pairs * Lanes<W>::TPR));
     const bool uni = (ra.rows / 2) % (64 / Lanes<W>::TPR) == 0;
-    if (uni) {
-      if (Lanes<W>::P <= 16 || grid.x <= 256)  // early loads as in launch_rows_inv
-        hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, true>), grid, dim3(256), 0, st, ra);
-      else
-        hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, Lanes<W>::P <= 16>), grid, dim3(256), 0, st, ra);
-    } else {
-      hipLaunchKernelGGL((rows_inv_kernel<W, true, false, true>), grid, dim3(256), 0, st, ra);
-    }
+    if (!uni) hipLaunchKernelGGL((rows_inv_kernel<W, true, false, true>), grid, dim3(256), 0, st, ra);
+    else if (rows_load_ahead<W>(grid.x))
+      hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, true>), grid, dim3(256), 0, st, ra);
+    else if constexpr (Lanes<W>::P > 16 || W >= 128)
+      hipLaunchKernelGGL((rows_inv_kernel<W, true, true, true, false>), grid, dim3(256), 0, st, ra);
     return launched("rows_inv (run)");
   });
   if (rc) return rc;
