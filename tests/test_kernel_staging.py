@@ -37,3 +37,11 @@ def test_mappings_of_a_batch():
             want.kernels_weight_per_channel[p['c_out']][i] = p['h']
         want.true_channels = [True] * 3 + [False] * 3 + [True, False, False]
         assert m == want
+
+
+@pytest.mark.parametrize('r', [2.0 ** 29, 2.0 ** 40, 1e300])
+def test_a_radius_past_32_bits_is_a_value_error(r):
+    """As every other radius that does not fit its world (the C field has 32 bits)."""
+    p = {'k_slug': 'circle_2d', 'k_params': [r, [1.0]], 'kf_slug': 'gauss', 'kf_params': [4.]}
+    with pytest.raises(ValueError, match='radius'):
+        kernels.kernel_desc(p, 13.)
