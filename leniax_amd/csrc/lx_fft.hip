@@ -1047,7 +1047,9 @@ int fwd_all(const Geom& g, const float* A, float2* X, int64_t nimg, hipStream_t 
 // asks for, over nimg images
 int inv_inner(const Geom& g, RowArgs ra, int64_t nk, int64_t nimg, hipStream_t st) {
   ra.rows = g.rows;
-  if (!ra.part && takes_planes(g, {ra.A, ra.A_out, ra.field, ra.pot}))
+  // (several kernels without potentials of the caller's: they go over the planes' own spectra)
+  const void* over = ra.C * ra.K > 1 && !ra.pot ? ra.U : nullptr;
+  if (!ra.part && takes_planes(g, {ra.A, ra.A_out, ra.field, ra.pot, over}))
     return lx_plane_inv(ra, g.L[0], g.L[1], g.W, nimg, st);
   if (g.naxes == 2) {
     LineArgs la = line_args();

@@ -99,3 +99,20 @@ def test_a_kernel_without_weight_adds_nothing(average):
             assert torch.equal(a.nan_to_num(nan=-7.), b.nan_to_num(nan=-7.))
         if not pot and not average:
             assert int(outs[0][0].isnan().sum()) == 1
+
+
+def test_a_workspace_that_starts_on_8_bytes():
+    """Several kernels without the caller's potentials: they are kept in the workspace, with 16-byte accesses only
+    where it starts on 16 bytes."""
+    from leniax_amd import _lib, core, engine
+    rule, Kh, gf, w, A = _case((16, 32, 48), 2, 2, 2)
+    ref = _update(rule, Kh, gf, w, A, pot=False)[0]
+    nb = ctypes.c_size_t(0)
+    _lib.call('lx_workspace_size', ctypes.byref(rule), 2, ctypes.byref(nb))
+    buf = torch.empty(nb.value + 16, dtype=torch.uint8, device='cuda')
+    work = buf[(8 - buf.data_ptr()) % 16:]
+    assert work.data_ptr() % 16 == 8
+    new = torch.empty_like(A)
+    _lib.call('lx_update_dt', ctypes.byref(rule), engine.ptr(A), 2, engine.ptr(Kh), 0, engine.ptr(gf), 0,
+              engine.ptr(w), 0, 0.1, engine.ptr(new), None, None, engine.ptr(work), engine.stream_ptr())
+    assert torch.equal(new, ref)
