@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void conv_staged_kernel(LineArgs a) {
 // the whole wave: the wave copies them into LDS once instead of loading them from global memory
 // in each kernel iteration, and its branches on them are uniform.
 template <int W, bool STATS, bool UNI, bool LIST = false, bool FETCH = true>
-__global__ __launch_bounds__(256, FETCH || Lanes<W>::P > 16 ? 1 : 4) void rows_inv_kernel(RowArgs a) {
+__global__ __launch_bounds__(256, Lanes<W>::P > 16 ? 1 : FETCH ? 3 : 4) void rows_inv_kernel(RowArgs a) {
   using LC = Lanes<W>;
   constexpr int TPR = LC::TPR, P = LC::P, WH = W / 2 + 1, NPRE = (WH + TPR - 1) / TPR;
   constexpr bool PRE = FETCH && UNI;
@@ -595,7 +595,9 @@ __global__ __launch_bounds__(256, FETCH || Lanes<W>::P > 16 ? 1 : 4) void rows_i
   // that a wave waits for memory once per channel instead of once per kernel and once for the state.  168
   // VGPRs (3 waves per SIMD) instead of 127 (4): 79 -> 66 us for 64 3-channel 6-kernel worlds of 256^2 with
   // statistics, whose 6144 waves are then two full rounds; not where a wave's lanes differ in their kernels
-  // (137 -> 175 VGPRs there).  launch_rows_inv says for which grids.
+  // (137 -> 175 VGPRs there).  rows_load_ahead says for which grids.  The launch bounds hold 12 points a lane
+  // of 8 (96) to 3 waves as well, at 4 to 6 registers in scratch: with the 174 that it would take, 2 waves, the
+  // 513th to 768th workgroup were a second round (a step of 155 3-channel 6-kernel worlds of 96^2 83 -> 71 us).
   float2 pre0[NPRE], pre1[NPRE];
   auto fetch = [&](int k, int t) {
     const float2* u0 = a.U + ((b * a.K + k) * a.rows + r2) * WH;

@@ -21,7 +21,8 @@ torch = pytest.importorskip('torch')
     ((32, 512), 250, '512, true, true, true, true'), ((32, 512), 270, '512, true, true, true, false'),
     ((32, 256), 700, '256, true, true, true, true'), ((32, 256), 900, '256, true, true, true, false'),
     ((32, 256), 1030, '256, true, true, true, true'), ((32, 128), 1000, '128, true, true, true, true'),
-    ((32, 128), 1800, '128, true, true, true, false'), ((48, 64), 700, '64, true, false, true, true')])
+    ((32, 128), 1800, '128, true, true, true, false'), ((32, 96), 1300, '96, true, true, true, true'),
+    ((48, 64), 700, '64, true, false, true, true')])
 def test_live_list_equals_the_step_loop(dims, slots, kernel):
     from leniax_amd import _lib, engine, runner
     print('live list', dims, slots, flush=True)
