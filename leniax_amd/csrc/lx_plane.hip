@@ -623,6 +623,20 @@ int plane_tables_of(int H, int W, hipStream_t st, PlaneTables* tb) {
 
 bool lx_plane_takes(int H, int W) { return by_plane(H, W, [](auto, auto) {}); }
 
+// A plane is one workgroup's: up to 6144 points it takes no longer than the rows' and lines' passes do on any
+// number of CUs; a larger one is a chain of 32 to 64 points a lane, which pays once most CUs have one, and from
+// 9216 points up in the reverse once they have two (LDS leaves two workgroups per CU of 128-point rows, and 96
+// rows of them are a round and a half).  Measured, us of these kernels against rows and lines for 16, 128, 192,
+// 256, 512, 1024 planes: update of 96 x 96 23 / 19, 26 / 26, 27.5 / 32, 29 / 34, 35 / 49, 51 / 85; of 128 x 128
+// 36 / 18, 41 / 33, 42 / 38, 44 / 45, 58 / 71, 113 / 123; four steps and their reverse of 96 x 96 210 / 164,
+// 242 / 220, 254 / 260, 261 / 280, 327 / 404; of 128 x 128 327 / 161, 368 / 268, 380 / 315, 398 / 361, 544 / 611,
+// 1082 / 1075; 64 x 64 19 / 19, 20 / 20, 20 / 22, 21 / 23.
+bool lx_plane_pays(int H, int W, int64_t planes, bool reverse) {
+  const int points = H * W;
+  if (points <= 6144) return true;
+  return planes >= (points <= 9216 ? 192 : reverse ? 512 : 256);
+}
+
 int lx_plane_fwd(int H, int W, const float* A, float2* S, int64_t planes, hipStream_t st) {
   PlaneTables tb;
   if (int rc = plane_tables_of(H, W, st, &tb)) return rc;

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from test_gpu_plane import _shifted
+from test_gpu_tune import _kernels, knobs  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -48,7 +49,9 @@ def test_entry_points_agree_bit_for_bit(H, C, K):
     from leniax_amd import engine, runner
     for W in SIDES:
         print('same bits', (16, H, W), C, K, flush=True)
-        rule, Kh, gf, w, A = _case((16, H, W), 3, C, K)
+        rule, Kh, gf, w, A = _case((16, H, W), 3 if H * W <= 6144 else 33, C, K)  # planes enough to be taken
+        names = _kernels(lambda: _update(rule, Kh, gf, w, A))
+        assert any(f'plane_inv_kernel<{H}, {W}>' in n for n in names), names
         planes = _update(rule, Kh, gf, w, A)
         general = _update(rule, Kh, gf, w, A, move=_shifted)
         bad = [n for n, a, b in zip(('state', 'field', 'potential'), planes, general) if not torch.equal(a, b)]
@@ -62,21 +65,22 @@ def test_entry_points_agree_bit_for_bit(H, C, K):
         assert torch.equal(r['cells'], second), ('live list', H, W)
 
 
-@pytest.mark.parametrize('dims', [(16, 32, 128), (32, 128, 96), (96, 96, 96), (48, 64, 64), (128, 48, 128)])
-def test_transforms_agree_bit_for_bit(dims):
+@pytest.mark.parametrize('dims,n', [((16, 32, 128), 2), ((32, 128, 96), 16), ((96, 96, 96), 2), ((48, 64, 64), 2),
+                                    ((128, 48, 128), 2)])
+def test_transforms_agree_bit_for_bit(dims, n):
     """rfftn and irfftn of arrays that start on 16 bytes (planes) and of arrays that do not."""
     from leniax_amd import _lib, engine
     print('same bits, transforms', dims, flush=True)
     rng = np.random.default_rng(1)
-    x = torch.as_tensor(rng.random((2,) + dims, dtype=np.float32)).cuda()
+    x = torch.as_tensor(rng.random((n,) + dims, dtype=np.float32)).cuda()
     cd = (ctypes.c_int32 * 3)(*dims)
     spectra, backs = [], []
     for move in (lambda t: t, _shifted):
         a = move(x)
-        X = torch.empty((2,) + dims[:2] + (dims[2] // 2 + 1,), dtype=torch.complex64, device='cuda')
-        _lib.call('lx_rfft2', 3, cd, 2, engine.ptr(a), engine.ptr(X), engine.stream_ptr())
+        X = torch.empty((n,) + dims[:2] + (dims[2] // 2 + 1,), dtype=torch.complex64, device='cuda')
+        _lib.call('lx_rfft2', 3, cd, n, engine.ptr(a), engine.ptr(X), engine.stream_ptr())
         back, work = move(torch.empty_like(x)), torch.empty_like(X)
-        _lib.call('lx_irfft2', 3, cd, 2, engine.ptr(X), engine.ptr(back), engine.ptr(work), engine.stream_ptr())
+        _lib.call('lx_irfft2', 3, cd, n, engine.ptr(X), engine.ptr(back), engine.ptr(work), engine.stream_ptr())
         spectra.append(X)
         backs.append(back)
     assert torch.equal(torch.view_as_real(spectra[0]), torch.view_as_real(spectra[1]))
@@ -116,3 +120,41 @@ def test_a_workspace_that_starts_on_8_bytes():
     _lib.call('lx_update_dt', ctypes.byref(rule), engine.ptr(A), 2, engine.ptr(Kh), 0, engine.ptr(gf), 0,
               engine.ptr(w), 0, 0.1, engine.ptr(new), None, None, engine.ptr(work), engine.stream_ptr())
     assert torch.equal(new, ref)
+
+
+@pytest.mark.parametrize('dims,few,many', [((16, 128, 128), 1, 17), ((16, 96, 96), 11, 12), ((32, 64, 128), 5, 6)])
+def test_few_large_planes_take_rows_and_lines(dims, few, many):
+    """A large plane is one workgroup's long chain: below a count the passes spread over the chip instead, with the
+    same bits."""
+    print('few planes', dims, few, many, flush=True)
+    rule, Kh, gf, w, A = _case(dims, many, 1, 1)
+    names = _kernels(lambda: _update(rule, Kh, gf, w, A))
+    assert any('plane_fwd' in n for n in names) and any('plane_inv' in n for n in names), names
+    ref = _update(rule, Kh, gf, w, A)
+    B = A[:few].contiguous()
+    names = _kernels(lambda: _update(rule, Kh, gf, w, B))
+    assert not any('plane' in n for n in names), names
+    for a, b in zip(ref, _update(rule, Kh, gf, w, B)):
+        assert torch.equal(a[:few], b)
+
+
+@pytest.mark.parametrize('dims,B', [((16, 96, 96), 12), ((16, 128, 128), 32)])
+def test_reverse_through_large_planes_gives_the_same_bits(knobs, dims, B):  # noqa: F811
+    """dL/dA0 of a run of whole planes against rows and lines (a pinned knob of the lines turns the planes off)."""
+    from leniax_amd import autograd as AG
+    print('reverse', dims, B, flush=True)
+    rng = np.random.default_rng(3)
+    kern = rng.random(dims)
+    K = torch.as_tensor(np.fft.fftn(kern / kern.sum()).astype(np.complex64)).cuda()[None, None, None]
+    A0 = torch.as_tensor(rng.random((B, 1) + dims, dtype=np.float32)).cuda().requires_grad_()
+    cot = torch.as_tensor(rng.normal(size=(B, 1) + dims).astype(np.float32)).cuda()
+    gf, w = torch.tensor([[0.5, 0.1]], device='cuda'), torch.ones((1, 1), device='cuda')
+
+    def gradient():
+        out = AG.run(A0, K, gf, w, torch.tensor(0.1, device='cuda'), 3, state_slug='v2', ckpt_every=2)
+        return torch.autograd.grad((out * cot).sum(), A0)[0]
+    assert any('plane_adj_kernel' in n for n in _kernels(gradient))
+    planes = gradient()
+    knobs.tune_force('line_xcd', 1)
+    assert not any('plane' in n for n in _kernels(gradient))
+    assert torch.equal(planes, gradient())
