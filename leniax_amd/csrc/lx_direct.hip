@@ -7,8 +7,10 @@
 //
 // The potential and its reverse are sums of products over a sliding window: contractions of the
 // staged image with a Toeplitz matrix of the taps, taken on the matrix cores in float32
-// (v_mfma_f32_4x4x1: 16 independent 4 x 4 outer products per instruction, twice the rate of the
-// vector unit's multiply-adds).  Any world size; kernels up to 64 x 64.
+// (v_mfma_f32_4x4x1: 16 independent 4 x 4 outer products, 512 flop in about 9 cycles; the vector
+// unit does as many in FMAs of registers, 2.2 cycles each, and half with a scalar operand, 4.1, as a
+// tap is; what the matrix form saves are the operands: one LDS read of a lane feeds 16 products).
+// Kernels of at most 5 columns stay on the vector unit.  Any world size; kernels up to 64 x 64.
 #include <algorithm>
 #include <type_traits>
 
@@ -23,12 +25,12 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 // pieces that 16 lanes read at once lie in different banks
 __host__ __device__ inline int bank_stride(int need) { return (need - 16 + 31) / 32 * 32 + 16; }
 
+LX_DEV bool not_finite(float v) { return !(fabsf(v) <= 3.402823466e38f); }
+
 // Stage rows [y0 - qh, y0 - qh + trows) x columns [x0 - qw, x0 - qw + tcols) of an H x W
 // image, wrapped, into tile[trows][stride]: each thread keeps one column (one modulo per thread,
 // not per element) and walks rows nsplit apart.  tcols <= 256.  Returns whether this thread met a
 // value that is not finite.
-LX_DEV bool not_finite(float v) { return !(fabsf(v) <= 3.402823466e38f); }
-
 LX_DEV bool stage_tile(float* tile, const float* img, int H, int W, int y0, int x0, int qh, int qw, int trows,
                        int tcols, int stride) {
   const int nsplit = 256 / tcols;
@@ -80,6 +82,44 @@ size_t direct_lds(int R, int kh, int kw) {
   return (size_t(16 * R + kh - 1) * direct_stride(kw) + size_t(kh + 1) * tap_stride(kw)) * sizeof(float);
 }
 
+// The potential of kernels at most 5 columns wide: a workgroup stages 16 rows x 64 columns with their halo, a
+// thread computes four neighbouring outputs from an 8-wide window of each row and uniform taps.  The matrix
+// form pays for its zero-padded tap rows and the extra quad there: 128 worlds of 128^2, 1, 3 and 5 taps a side,
+// us of the matrix form against these: 9.9 / 6.5, 12.0 / 7.1, 13.3 / 8.4; one world of 64^2 1 us less each.
+constexpr int kNarrow = 5, kNarrowStride = TX + 8;
+
+template <int KW>
+__global__ __launch_bounds__(256) void direct_narrow_kernel(DirectArgs a, const float* in, float* out) {
+  extern __shared__ __align__(16) float tile[];  // (16 + kh - 1) rows
+  const int x0 = blockIdx.x * TX, y0 = blockIdx.y * 16;
+  const int64_t b = blockIdx.z / a.K;
+  const int k = int(blockIdx.z - b * a.K);
+  stage_tile(tile, in + (b * a.C + a.cin[k]) * int64_t(a.H) * a.W, a.H, a.W, y0, x0, a.ph, a.pw, 16 + a.kh - 1, TX + 4,
+             kNarrowStride);
+  __syncthreads();
+  const int y = y0 + threadIdx.x / (TX / 4), x = threadIdx.x % (TX / 4) * 4;
+  const float* row = tile + (y - y0) * kNarrowStride + x;
+  const float* kk = a.kern + int64_t(k) * a.kh * KW;
+  f4v acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < a.kh; ++i, row += kNarrowStride, kk += KW) {
+    const float4 lo = *reinterpret_cast<const float4*>(row), hi = *reinterpret_cast<const float4*>(row + 4);
+    const float w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+    for (int j = 0; j < KW; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(kk[j], w[e + j], acc[e]);
+  }
+  if (y >= a.H || x0 + x >= a.W) return;
+  float* dst = out + (int64_t(blockIdx.z) * a.H + y) * a.W + x0 + x;
+  if (a.vec) {
+    *reinterpret_cast<f4v*>(dst) = acc;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (x0 + x + e < a.W) dst[e] = acc[e];
+  }
+}
+
 // The potential (ADJ: the state side of its reverse, dA[b][c] = sum over the kernels k fed by c of the
 // correlation of dU[b][k] with the flipped kernel, wrap-padded with kh - 1 - ph before).  A workgroup
 // computes 16 R rows x 64 columns of one image, a wave 4 R x 64: in lane 4 b + n, accumulator g holds
@@ -90,9 +130,10 @@ size_t direct_lds(int R, int kh, int kw) {
 // block, so 7 quads of columns take 28 tap columns for a 25-tap row (1.12x the products).  Each output
 // adds its products in the order of i, then j.  A tile that holds a value that is not finite is summed
 // product by product, so that none meets a zero beside the kernel.
-// Measured, 128 worlds of 128^2, 25 x 25 taps, R = 2: potential 60 -> 52 us (50 TFLOP/s of the taps), state
-// side 94 -> 54 us (the vector units' window kernel before took its flipped taps one by one); 12 us of
-// it stage the tiles, the instructions themselves need 25.
+// Measured, 128 worlds of 128^2, 25 x 25 taps, R = 2: potential 60 -> 41 us (64 TFLOP/s of the taps), state
+// side 94 -> 42 us (the vector units' window kernel before took its flipped taps one by one); 12 us of
+// it stage the tiles, the instructions themselves need 25.  Groups of equal size rather than of four quads with
+// a partly empty last one: 47 -> 41 us there, 72 -> 57 at 33 taps a side, 149 -> 122 at 48.
 template <int R, bool ADJ>
 __global__ __launch_bounds__(256) void direct_mfma_kernel(DirectArgs a, const float* in, float* out) {
   extern __shared__ __align__(16) float lds[];
@@ -129,35 +170,50 @@ __global__ __launch_bounds__(256) void direct_mfma_kernel(DirectArgs a, const fl
       const float* tcol = taps + ((lane >> 2) & 3) - n + 3;
       const float* col = tile + (wy + n) * S + 4 * blk;
       const int last = a.kh - 1 + 4 * (R - 1);
-      for (int s = 0; s <= last; ++s) {
-        const int ti = unsigned(s - 4 * tg) < unsigned(a.kh) ? s - 4 * tg : a.kh;  // row kh holds zeros
-        const float* trow = tcol + ti * TS;
-        const float* irow = col + s * S;
-        // 4 quads' reads are in flight together, then their instructions
-        for (int q0 = 0; q0 < Q; q0 += 4) {
-          float4 v[4];
-          float t[4];
+      // the quads in groups of at most 4 and as equal as can be (`more` groups of each + 1, then groups of each):
+      // a group's reads are in flight together, then its instructions
+      const int groups = (Q + 3) / 4, each = Q / groups, more = Q - groups * each;
+      auto rows_of = [&](auto each_c) {
+        constexpr int EACH = decltype(each_c)::value;
+        for (int s = 0; s <= last; ++s) {
+          const int ti = unsigned(s - 4 * tg) < unsigned(a.kh) ? s - 4 * tg : a.kh;  // row kh holds zeros
+          const float* trow = tcol + ti * TS;
+          const float* irow = col + s * S;
+          auto group = [&](auto n_c) {
+            constexpr int N = decltype(n_c)::value;
+            float4 v[N];
+            float t[N];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int q = q0 + u < Q ? q0 + u : 0;
-            v[u] = *reinterpret_cast<const float4*>(irow + 4 * q);
-            t[u] = trow[4 * q];
-          }
-          __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < N; ++u) {
+              v[u] = *reinterpret_cast<const float4*>(irow + 4 * u);
+              t[u] = trow[4 * u];
+            }
+            irow += 4 * N;
+            trow += 4 * N;
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if (q0 + u >= Q) break;
-            auto column = [&](auto e_c, float x) {
-              constexpr int E = decltype(e_c)::value;
-              acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(t[u], x, acc[0], 4, E, 0);
-              if constexpr (R > 1) acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(t[u], x, acc[1], 4, 4 + E, 0);
-            };
-            column(std::integral_constant<int, 0>{}, v[u].x);
-            column(std::integral_constant<int, 1>{}, v[u].y);
-            column(std::integral_constant<int, 2>{}, v[u].z);
-            column(std::integral_constant<int, 3>{}, v[u].w);
-          }
+            for (int u = 0; u < N; ++u) {
+              auto column = [&](auto e_c, float x) {
+                constexpr int E = decltype(e_c)::value;
+                acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(t[u], x, acc[0], 4, E, 0);
+                if constexpr (R > 1) acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(t[u], x, acc[1], 4, 4 + E, 0);
+              };
+              column(std::integral_constant<int, 0>{}, v[u].x);
+              column(std::integral_constant<int, 1>{}, v[u].y);
+              column(std::integral_constant<int, 2>{}, v[u].z);
+              column(std::integral_constant<int, 3>{}, v[u].w);
+            }
+          };
+          if constexpr (EACH < 4)
+            for (int g = 0; g < more; ++g) group(std::integral_constant<int, EACH + 1>{});
+          for (int g = more; g < groups; ++g) group(std::integral_constant<int, EACH>{});
         }
+      };
+      switch (each) {
+        case 4: rows_of(std::integral_constant<int, 4>{}); break;
+        case 3: rows_of(std::integral_constant<int, 3>{}); break;
+        case 2: rows_of(std::integral_constant<int, 2>{}); break;
+        default: rows_of(std::integral_constant<int, 1>{}); break;
       }
     } else {
       for (int i = 0; i < a.kh; ++i)
@@ -188,25 +244,45 @@ __global__ __launch_bounds__(256) void direct_mfma_kernel(DirectArgs a, const fl
   }
 }
 
-// The launch for `images` output images: R = 2 halves the LDS reads per instruction (52 against 64 us at
-// the size above; R = 4 measured 58, its tiles leave two workgroups per CU); R = 1 where R = 2 would
-// leave CUs with fewer than two workgroups (512) or its tile exceeds 64 KB of LDS.
+// The launch for `images` output images: R = 2 halves the LDS reads per instruction (with groups
+// of four quads 52 against 64 us at the size above; R = 4 measured 58, its tiles leave two workgroups per CU); R = 1 where R = 2 would
+// leave CUs with fewer than two workgroups (512).  Its tile takes up to 75 KB of LDS (64 taps a side: still two
+// workgroups per CU); with R = 1 beyond 64 KB the same 128 worlds took 389 us for 64 x 64 taps, 182 now.
 template <bool ADJ>
-void launch_direct(DirectArgs a, int64_t images, const float* in, float* out, hipStream_t st) {
+int launch_direct(DirectArgs a, int64_t images, const float* in, float* out, hipStream_t st) {
   a.vec = a.W % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
   auto grid = [&](int R) {
     return dim3(unsigned((a.W + TX - 1) / TX), unsigned((a.H + 16 * R - 1) / (16 * R)), unsigned(images));
   };
-  auto fits = [&](int R) {
-    const dim3 g = grid(R);
-    return int64_t(g.x) * g.y * g.z >= 512 && direct_lds(R, a.kh, a.kw) <= 65536;
-  };
+  if constexpr (!ADJ) {
+    auto narrow = [&](auto kw_c) {
+      constexpr int KW = decltype(kw_c)::value;
+      hipLaunchKernelGGL((direct_narrow_kernel<KW>), grid(1), dim3(256),
+                         size_t(16 + a.kh - 1) * kNarrowStride * sizeof(float), st, a, in, out);
+      return LX_OK;
+    };
+    static_assert(kNarrow == 5, "one case per width");
+    switch (a.kw) {
+      case 1: return narrow(std::integral_constant<int, 1>{});
+      case 2: return narrow(std::integral_constant<int, 2>{});
+      case 3: return narrow(std::integral_constant<int, 3>{});
+      case 4: return narrow(std::integral_constant<int, 4>{});
+      case 5: return narrow(std::integral_constant<int, 5>{});
+      default: break;
+    }
+  }
   auto go = [&](auto r_c) {
     constexpr int R = decltype(r_c)::value;
-    hipLaunchKernelGGL((direct_mfma_kernel<R, ADJ>), grid(R), dim3(256), direct_lds(R, a.kh, a.kw), st, a, in, out);
+    const size_t lds = direct_lds(R, a.kh, a.kw);
+    if (lds > 65536 &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(direct_mfma_kernel<R, ADJ>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess)
+      return lx_fail(LX_EDEVICE, "direct potential: %zu bytes of LDS refused", lds);
+    hipLaunchKernelGGL((direct_mfma_kernel<R, ADJ>), grid(R), dim3(256), lds, st, a, in, out);
+    return int(LX_OK);
   };
-  if (fits(2)) go(std::integral_constant<int, 2>{});
-  else go(std::integral_constant<int, 1>{});
+  const dim3 two = grid(2);
+  return int64_t(two.x) * two.y * two.z >= 512 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
 }
 
 // Reverse of the direct potential, kernel side: dK[k][i][j] = sum over worlds and cells of
@@ -416,7 +492,7 @@ int direct_adjoint(const char* fn, const lx_rule* rule, const float* state_d, in
   if (B * rule->C > 65535) return lx_fail(LX_ENOTSUP, "%s: B * C > 65535", fn);
   const DirectArgs a = direct_args(rule, state_d, kern_d, kh, kw);
   if (dstate_d) {
-    launch_direct<true>(a, B * rule->C, dpot_d, dstate_d, st);
+    if ((rc = launch_direct<true>(a, B * rule->C, dpot_d, dstate_d, st))) return rc;
   }
   if (dkern_d && work) {
     const int64_t rows = kgrad_part_rows(rule, B, kh, kw);
@@ -484,7 +560,7 @@ extern "C" int lx_potential_direct(const lx_rule* rule, const float* state_d, in
   if (!state_d || !kern_d || !potential_d) return lx_fail(LX_EINVAL, "NULL pointer");
   if (B * rule->K > 65535) return lx_fail(LX_ENOTSUP, "lx_potential_direct: B * K > 65535");
   const DirectArgs a = direct_args(rule, state_d, kern_d, kh, kw);
-  launch_direct<false>(a, B * rule->K, state_d, potential_d, (hipStream_t)stream);
+  if ((rc = launch_direct<false>(a, B * rule->K, state_d, potential_d, (hipStream_t)stream))) return rc;
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? LX_OK : lx_fail(LX_EDEVICE, "direct potential launch: %s", hipGetErrorString(e));
 }

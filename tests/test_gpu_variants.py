@@ -149,3 +149,48 @@ def test_direct_adjoint_without_a_workspace(B, C, maxk, H, W, kh, kw):
     ref = _kernel_gradient(A, dU, kh, kw, maxk)
     bound = (B * -(-H * W // 256) + 10) * 2.0 ** -24
     assert float(np.max(np.abs(outs[0][1] - ref) / ref)) <= bound
+
+
+DIRECT = ([(2, 1, 1, 17, 65, 7, 1), (1, 2, 2, 33, 70, 1, 2), (3, 1, 1, 40, 63, 64, 3), (1, 1, 1, 8, 8, 5, 4),
+           (2, 1, 1, 64, 64, 5, 5)] + [(2, 1, 1, 50, 130, 3, kw) for kw in (6, 9, 12, 16, 17, 21, 25, 33, 37, 41, 48, 49, 64)] +
+          [(64, 1, 1, 128, 128, 64, 64), (65, 1, 1, 100, 128, 53, 57)])
+
+
+@pytest.mark.parametrize('B,C,maxk,H,W,kh,kw', DIRECT)
+def test_direct_potential_by_width(B, C, maxk, H, W, kh, kw):
+    """Kernels of 1 to 5 columns (direct_narrow_kernel), every split of the tap quads into groups, tiles beyond 64 KB of
+    LDS: the potential and its state gradient against float64 correlations.  Every output is kh kw (times the
+    kernels of a channel) multiply-adds of positive terms in a row."""
+    from leniax_amd import core
+    print('direct by width', (B, C, maxk, H, W, kh, kw), flush=True)
+    rng = np.random.default_rng(kh * 100 + kw)
+    A = rng.uniform(0.5, 1, size=(B, C, H, W)).astype(np.float32)
+    K = rng.uniform(0.5, 1, size=(C * maxk, 1, kh, kw)).astype(np.float32)
+    dU = rng.uniform(0.5, 1, size=(B, C * maxk, H, W)).astype(np.float32)
+    pad = tuple([(0, 0), (0, 0)] + [(d // 2, d // 2 - 1) if d % 2 == 0 else (d // 2, d // 2) for d in (kh, kw)])
+    tA = torch.as_tensor(A).cuda().requires_grad_()
+    pot = core.get_potential(tA, torch.as_tensor(K).cuda(), pad)
+    dA = torch.autograd.grad(pot, tA, torch.as_tensor(dU).cuda())[0].cpu().numpy()
+    # U[y][x] = sum k[i][j] A[y + i - kh // 2][x + j - kw // 2], the kernel's taps past the world wrapped onto it
+    taps = np.zeros((C * maxk, H, W))
+    for i in range(kh):
+        for j in range(kw):
+            taps[:, (i - kh // 2) % H, (j - kw // 2) % W] += K[:, 0, i, j]
+    spec = np.fft.rfft2(taps)
+    U64 = np.fft.irfft2(np.fft.rfft2(np.repeat(A.astype(np.float64), maxk, 1)) * np.conj(spec), s=(H, W))
+    A64 = np.fft.irfft2(np.fft.rfft2(dU.astype(np.float64)) * spec, s=(H, W)).reshape(B, C, maxk, H, W).sum(2)
+    assert float(np.max(np.abs(pot.detach().cpu().numpy() - U64) / U64)) <= kh * kw * 2.0 ** -24
+    assert float(np.max(np.abs(dA - A64) / A64)) <= kh * kw * maxk * 2.0 ** -24
+
+
+def test_narrow_potential_of_a_state_that_is_not_finite():
+    """Exactly the cells whose window holds the infinite cell are infinite."""
+    from leniax_amd import core
+    A = np.full((1, 1, 40, 80), 0.5, np.float32)
+    A[0, 0, 7, 60] = np.inf
+    pot = core.get_potential(torch.as_tensor(A).cuda(), torch.full((1, 1, 5, 4), 0.25).cuda(),
+                             ((0, 0), (0, 0), (2, 2), (2, 1)))[0, 0].cpu().numpy()
+    rows, cols = np.nonzero(~np.isfinite(pot))
+    assert not np.isnan(pot).any()
+    assert sorted(set(rows)) == list(range(5, 10)) and sorted(set(cols)) == list(range(59, 63)) and len(rows) == 20
+    assert np.array_equal(pot[np.isfinite(pot)], np.full(3180, 20 * 0.125, np.float32))
