@@ -326,14 +326,21 @@ __global__ __launch_bounds__(256) void direct_kgrad_kernel(DirectArgs a, int64_t
 // kernel above re-reads both images for every tap with a division and two remainders per product).
 // Measured, 128 worlds of 128^2 with a 25 x 25 kernel: 3457 -> 59 + 5 us (2.6 GFLOP of taps: 41 TFLOP/s),
 // error against 64 bits 1.6e-6 -> 4.7e-7 (shorter chains of additions).
+// Few worlds take other chains, so that no size is summed less accurately than by one block per tap, whose
+// threads add every 256th cell: up to 2^17 cells a row's cells go into four sums of their own (a lane's chain is
+// 16 + 2 + 4 additions of a tile instead of 256; two worlds of 167 x 82, 25 taps a side: 2.2e-7 -> 1.3e-7, one block
+// per tap 1.4e-7; 7% of the time there, 25% for many worlds, whose waves are fewer by its 135 VGPRs), and up to 6144
+// cells with up to 1200 taps one block per tap is the faster too (one world of 64^2, 5, 25 and 33 taps a side: 7.9,
+// 10 and 13.5 against 11.6, 16.9 and 17.3 us).
 constexpr int kGY = 16, kGX = 64, kGridRows = 1024, kGSets = 4;
 
 __host__ __device__ inline int kgrad_stride(int kw) { return bank_stride(kGX + ((kw + 3) & ~3)); }
 __host__ __device__ inline int kgrad_rows(int kh) { return kGY - 1 + ((kh + 3) & ~3); }
 constexpr int kGDU = kGX + 4;  // dU tile row: 3 columns before, one spare
 
-// NS: sets of 16 (ib, jb) pairs per block; blockIdx.y = k * groups + group of NS sets
-template <int NS>
+// NS: sets of 16 (ib, jb) pairs per block; blockIdx.y = k * groups + group of NS sets.  FINE: a row's cells in four
+// chains of additions that start anew, for few cells (kgrad_fine)
+template <int NS, bool FINE>
 __global__ __launch_bounds__(256) void direct_kgrad_mfma_kernel(DirectArgs a, int64_t B, const float* dU, float* part,
                                                                 int groups, int tx, int64_t ntiles) {
   extern __shared__ __align__(16) float lds[];
@@ -368,6 +375,12 @@ __global__ __launch_bounds__(256) void direct_kgrad_mfma_kernel(DirectArgs a, in
     const int rows = min(kGY, a.H - y0), cols = min(kGX, a.W - x0);
     if (!slow) {
       for (int r = wave; r < rows; r += 4) {
+        f4v part[FINE ? NS : 1][4];  // FINE: sums of every fourth cell of the row
+        if constexpr (FINE)
+#pragma unroll
+          for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[s][e] = f4v{0.f, 0.f, 0.f, 0.f};
         for (int xg = 0; xg < cols; xg += 16) {
           const int p = lane >> 2;
           // cells past the image's last column count nothing
@@ -378,23 +391,27 @@ __global__ __launch_bounds__(256) void direct_kgrad_mfma_kernel(DirectArgs a, in
             float4 v[NS];
 #pragma unroll
             for (int s = 0; s < NS; ++s) v[s] = *reinterpret_cast<const float4*>(row + off[s] + 4 * Q);
+            auto cell = [&](auto e_c, auto of) {
+              constexpr int E = decltype(e_c)::value;
 #pragma unroll
-            for (int s = 0; s < NS; ++s) acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(g, v[s].x, acc[s], 4, 4 * Q, 0);
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-              acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(g, v[s].y, acc[s], 4, 4 * Q + 1, 0);
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-              acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(g, v[s].z, acc[s], 4, 4 * Q + 2, 0);
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-              acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(g, v[s].w, acc[s], 4, 4 * Q + 3, 0);
+              for (int s = 0; s < NS; ++s) {
+                f4v& sum = FINE ? part[FINE ? s : 0][E] : acc[s];
+                sum = __builtin_amdgcn_mfma_f32_4x4x1f32(g, of(v[s]), sum, 4, 4 * Q + E, 0);
+              }
+            };
+            cell(std::integral_constant<int, 0>{}, [](const float4& w) { return w.x; });
+            cell(std::integral_constant<int, 1>{}, [](const float4& w) { return w.y; });
+            cell(std::integral_constant<int, 2>{}, [](const float4& w) { return w.z; });
+            cell(std::integral_constant<int, 3>{}, [](const float4& w) { return w.w; });
           };
           quad(std::integral_constant<int, 0>{});
           quad(std::integral_constant<int, 1>{});
           quad(std::integral_constant<int, 2>{});
           quad(std::integral_constant<int, 3>{});
         }
+        if constexpr (FINE)
+#pragma unroll
+          for (int s = 0; s < NS; ++s) acc[s] += (part[s][0] + part[s][1]) + (part[s][2] + part[s][3]);
       }
     } else {
       // a state that is not finite: product by product, so that none is taken with the zero of a
@@ -455,6 +472,10 @@ int kgrad_tiles_x(int W) { return (W + kGX - 1) / kGX; }
 int64_t kgrad_tiles(const lx_rule* r, int64_t B) {
   return B * kgrad_tiles_x(r->dims[1]) * ((r->dims[0] + kGY - 1) / kGY);
 }
+bool kgrad_fine(const lx_rule* r, int64_t B) { return B * r->dims[0] * r->dims[1] <= (1 << 17); }
+bool kgrad_by_tap(const lx_rule* r, int64_t B, int kh, int kw) {
+  return B * r->dims[0] * r->dims[1] <= 6144 && r->K * kh * kw <= 1200;
+}
 // blocks of NS = kgrad_ns(sets) sets per kernel and rows of partial sums: enough blocks to fill 256 CUs
 // a few times over, no more than tiles; at most kGridRows x 16 kGSets taps x 16 B of partial sums
 int kgrad_sets(int kh, int kw) { return (((kh + 3) / 4) * ((kw + 3) / 4) + 15) / 16; }
@@ -494,7 +515,7 @@ int direct_adjoint(const char* fn, const lx_rule* rule, const float* state_d, in
   if (dstate_d) {
     if ((rc = launch_direct<true>(a, B * rule->C, dpot_d, dstate_d, st))) return rc;
   }
-  if (dkern_d && work) {
+  if (dkern_d && work && !kgrad_by_tap(rule, B, kh, kw)) {
     const int64_t rows = kgrad_part_rows(rule, B, kh, kw);
     const int sets = kgrad_sets(kh, kw);
     auto go = [&](auto ns_c) {
@@ -502,8 +523,15 @@ int direct_adjoint(const char* fn, const lx_rule* rule, const float* state_d, in
       const int groups = (sets + NS - 1) / NS;
       const size_t tiles = size_t(kgrad_rows(kh)) * kgrad_stride(kw) + size_t(kGY) * kGDU;
       const size_t lds = std::max(tiles, size_t(4) * NS * 256) * sizeof(float);
-      hipLaunchKernelGGL((direct_kgrad_mfma_kernel<NS>), dim3(unsigned(rows), unsigned(rule->K * groups)), dim3(256),
-                         lds, st, a, B, dpot_d, work, groups, kgrad_tiles_x(a.W), kgrad_tiles(rule, B));
+      const dim3 grid{unsigned(rows), unsigned(rule->K * groups)};
+      const int tx = kgrad_tiles_x(a.W);
+      const int64_t ntiles = kgrad_tiles(rule, B);
+      if (kgrad_fine(rule, B))
+        hipLaunchKernelGGL((direct_kgrad_mfma_kernel<NS, true>), grid, dim3(256), lds, st, a, B, dpot_d, work, groups, tx,
+                           ntiles);
+      else
+        hipLaunchKernelGGL((direct_kgrad_mfma_kernel<NS, false>), grid, dim3(256), lds, st, a, B, dpot_d, work, groups,
+                           tx, ntiles);
     };
     switch (kgrad_ns(sets)) {
       case 1: go(std::integral_constant<int, 1>{}); break;

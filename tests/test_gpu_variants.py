@@ -194,3 +194,31 @@ def test_narrow_potential_of_a_state_that_is_not_finite():
     assert not np.isnan(pot).any()
     assert sorted(set(rows)) == list(range(5, 10)) and sorted(set(cols)) == list(range(59, 63)) and len(rows) == 20
     assert np.array_equal(pot[np.isfinite(pot)], np.full(3180, 20 * 0.125, np.float32))
+
+
+@pytest.mark.parametrize('B,H,W,k', [(1, 40, 40, 5), (1, 52, 96, 32), (1, 64, 100, 9), (2, 167, 82, 25), (2, 195, 58, 18),
+                                     (4, 42, 177, 19), (3, 159, 154, 8), (1, 128, 128, 40), (2, 256, 256, 13),
+                                     (20, 86, 218, 7)])
+def test_kernel_gradient_is_as_accurate_as_tap_by_tap(B, H, W, k):
+    """The kernel gradient with a workspace is no further from float64 than one block per tap (the entry without one),
+    whatever the number of cells: terms of both signs, so a sum's error goes with its longest chains of additions;
+    a quarter of room for the sample of k^2 taps."""
+    from leniax_amd import core, engine, _lib
+    print('kernel gradient accuracy', (B, H, W, k), flush=True)
+    rng = np.random.default_rng(k)
+    A = rng.uniform(size=(B, 1, H, W)).astype(np.float32)
+    dU = rng.normal(size=(B, 1, H, W)).astype(np.float32)
+    rule = core._rule((H, W), 1, 1, [0])
+    tA, tU, tk = torch.as_tensor(A).cuda(), torch.as_tensor(dU).cuda(), torch.zeros((1, k, k), device='cuda')
+    nb = ctypes.c_size_t(0)
+    _lib.call('lx_potential_direct_adjoint_size', ctypes.byref(rule), B, k, k, ctypes.byref(nb))
+    work = torch.empty(nb.value, dtype=torch.uint8, device='cuda')
+    ref = _kernel_gradient(A, dU, k, k, 1)
+    errs = []
+    for entry, tail in (('lx_potential_direct_adjoint', ()), ('lx_potential_direct_adjoint_work', (engine.ptr(work),))):
+        dk = torch.empty_like(tk)
+        _lib.call(entry, ctypes.byref(rule), engine.ptr(tA), B, engine.ptr(tk), k, k, engine.ptr(tU), None, engine.ptr(dk),
+                  *tail, engine.stream_ptr())
+        errs.append(float(np.linalg.norm(dk.cpu().numpy() - ref) / np.linalg.norm(ref)))
+    print('  by tap, with a workspace', errs)
+    assert errs[1] <= 1.25 * errs[0]
