@@ -166,7 +166,8 @@ int lx_potential_direct(const lx_rule* rule, const float* state_d, int64_t B, co
 /* Reverse of lx_potential_direct (what jax.grad gives through leniax/core.py:105-146): with
  * dpot_d = dL/dpotential [B][K][H][W], dstate_d [B][C][H][W] = dL/dstate (overwritten: for each
  * channel the correlation of its kernels' dpot with the flipped kernels) and dkern_d [K][kh][kw] =
- * dL/dkernel summed over worlds (overwritten).  Either output may be NULL. */
+ * dL/dkernel summed over worlds (overwritten).  Either output may be NULL.  dkern_d takes one workgroup per
+ * tap over all worlds: for many worlds lx_potential_direct_adjoint_work (leniax_amd_ext.h) is 50 times as fast. */
 int lx_potential_direct_adjoint(const lx_rule* rule, const float* state_d, int64_t B, const float* kern_d,
                                 int32_t kh, int32_t kw, const float* dpot_d, float* dstate_d, float* dkern_d,
                                 void* stream);

@@ -10,8 +10,8 @@ extern "C" {
 #endif
 
 /* lx_potential_direct_adjoint with a workspace of lx_potential_direct_adjoint_size bytes for the kernel side's partial
- * sums, which then runs on the matrix cores over tiles of the worlds (without one: one workgroup per
- * kernel tap over all worlds).  Deterministic: the partial sums are added in a fixed order. */
+ * sums, which then runs on the matrix cores over tiles of the worlds (without one, and for few cells and taps:
+ * one workgroup per kernel tap over all worlds).  Deterministic: the partial sums are added in a fixed order. */
 int lx_potential_direct_adjoint_size(const lx_rule* rule, int64_t B, int32_t kh, int32_t kw, size_t* bytes);
 int lx_potential_direct_adjoint_work(const lx_rule* rule, const float* state_d, int64_t B, const float* kern_d,
                                      int32_t kh, int32_t kw, const float* dpot_d, float* dstate_d,

@@ -293,7 +293,8 @@ struct LaneTwiddle {
   static LX_DEV float2 get(int t, const float2* tw) {
     float2 w = make_float2(1.f, 0.f);
     if constexpr (ANY) {
-      const float2 tv = tw[CT ? bitrev_n(t / (2 * H), TPR / (2 * H)) * (P * H) : (t & (H - 1)) * (L / (2 * H))];
+      const int j = CT ? bitrev_n(t / (2 * H), TPR / (2 * H)) * (P * H) : (t & (H - 1)) * (L / (2 * H));
+      const float2 tv = tw[j];
       w = (t & H) != 0 ? make_float2(tv.x, INV ? -tv.y : tv.y) : w;
     }
     return w;

@@ -244,10 +244,10 @@ __global__ __launch_bounds__(256) void direct_mfma_kernel(DirectArgs a, const fl
   }
 }
 
-// The launch for `images` output images: R = 2 halves the LDS reads per instruction (with groups
-// of four quads 52 against 64 us at the size above; R = 4 measured 58, its tiles leave two workgroups per CU); R = 1 where R = 2 would
-// leave CUs with fewer than two workgroups (512).  Its tile takes up to 75 KB of LDS (64 taps a side: still two
-// workgroups per CU); with R = 1 beyond 64 KB the same 128 worlds took 389 us for 64 x 64 taps, 182 now.
+// The launch for `images` output images: R = 2 halves the LDS reads per instruction (with groups of four quads 52
+// against 64 us at the size above; R = 4 measured 58, its tiles leave two workgroups per CU); R = 1 where R = 2
+// would leave CUs with fewer than two workgroups (512).  R = 2's tile takes up to 75 KB of LDS (64 taps a side:
+// still two workgroups per CU); with R = 1 beyond 64 KB the same 128 worlds took 389 us for 64 x 64 taps, 182 now.
 template <bool ADJ>
 int launch_direct(DirectArgs a, int64_t images, const float* in, float* out, hipStream_t st) {
   a.vec = a.W % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
@@ -282,7 +282,8 @@ int launch_direct(DirectArgs a, int64_t images, const float* in, float* out, hip
     return int(LX_OK);
   };
   const dim3 two = grid(2);
-  return int64_t(two.x) * two.y * two.z >= 512 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
+  if (int64_t(two.x) * two.y * two.z >= 512) return go(std::integral_constant<int, 2>{});
+  return go(std::integral_constant<int, 1>{});
 }
 
 // Reverse of the direct potential, kernel side: dK[k][i][j] = sum over worlds and cells of
@@ -527,8 +528,8 @@ int direct_adjoint(const char* fn, const lx_rule* rule, const float* state_d, in
       const int tx = kgrad_tiles_x(a.W);
       const int64_t ntiles = kgrad_tiles(rule, B);
       if (kgrad_fine(rule, B))
-        hipLaunchKernelGGL((direct_kgrad_mfma_kernel<NS, true>), grid, dim3(256), lds, st, a, B, dpot_d, work, groups, tx,
-                           ntiles);
+        hipLaunchKernelGGL((direct_kgrad_mfma_kernel<NS, true>), grid, dim3(256), lds, st, a, B, dpot_d, work, groups,
+                           tx, ntiles);
       else
         hipLaunchKernelGGL((direct_kgrad_mfma_kernel<NS, false>), grid, dim3(256), lds, st, a, B, dpot_d, work, groups,
                            tx, ntiles);

@@ -12,9 +12,10 @@ namespace lx_pass {
 // SIMD instead of 2)
 constexpr int row_tpr(int L) { return L <= 64 ? 4 : (L <= 192 ? 8 : 16); }
 // lanes per transform of the line passes: as the rows, except the plain forward and inverse
-// passes (modes 1 and 2) at 96 points, which take 4 x 24 through LDS: they stay at 4 waves per
-// SIMD there (101 and 112 VGPRs) and run 10% faster than on the network (the convolution pass,
-// at 173 VGPRs with 4 lanes, is as fast on 8)
+// passes (modes 1 and 2) at 96 points, which take 4 x 24 through LDS, as the columns of the plane
+// kernels do (a step's bits are then the same either way).  The strided groups below bound both
+// forms by memory: 16 worlds of 96^3 22.3 and 23.4 us forward and inverse (101 and 113 VGPRs)
+// against 21.7 and 22.1 on 8 lanes (59 and 65); the convolution pass takes 114 VGPRs on 8 lanes, 173 on 4
 constexpr int line_tpr(int L, int mode) { return L == 96 && mode != 0 ? 4 : row_tpr(L); }
 
 template <int L, int T = row_tpr(L)>
@@ -88,7 +89,8 @@ LX_DEV void strided_stage(float2* x, int t, int lane, const float2* tw) {
 #pragma unroll
   for (int k = 0; k < P; ++k) {
     const float2 o = LT::ANY && LT::FIRST ? cmul(x[k], w) : x[k];
-    const float2 v = make_float2(strided_pair<H * (64 / T)>(o.x, sgn, lane), strided_pair<H * (64 / T)>(o.y, sgn, lane));
+    const float2 v =
+        make_float2(strided_pair<H * (64 / T)>(o.x, sgn, lane), strided_pair<H * (64 / T)>(o.y, sgn, lane));
     x[k] = LT::ANY && !LT::FIRST ? cmul(v, w) : v;
   }
 }

@@ -600,7 +600,7 @@ bool by_plane(int H, int W, F&& f) {
   return ok;
 }
 
-// a kernel's dynamic LDS beyond 64 KB (planes of 128 x 128) is asked for once per kernel
+// a kernel's dynamic LDS beyond 64 KB (planes of 128 x 128) is asked for before its launches
 template <typename K>
 int allow_lds(K kernel, size_t bytes) {
   if (bytes <= 65536) return LX_OK;

@@ -266,8 +266,10 @@ def _desc_bytes(param: Dict, R: float):
     if not 1 <= nb <= _lib.LX_MAX_RINGS:
         raise ValueError(f'1..{_lib.LX_MAX_RINGS} rings supported, got {nb}')
     kr = math.ceil(kp[0] * R)
-    if not 1 <= kr < 2**31:
-        raise ValueError(f'kernel radius ceil(r R) = {kr} < 1' if kr < 1 else f'kernel radius ceil(r R) = {kr} too large')
+    if kr < 1:
+        raise ValueError(f'kernel radius ceil(r R) = {kr} < 1')
+    if kr >= 2**31:
+        raise ValueError(f'kernel radius ceil(r R) = {kr} too large')
     a, b, theta = (0., 0., 0.) if shape == 0 else (float(kp[2]), float(kp[3]), float(kp[4]))
     k0, k1 = (kfp + [0., 0.])[:2]
     return _DESC.pack(shape, kf, nb, kr, float(kp[0]), a, b, theta, k0, k1, *bs, *_NO_RINGS[nb:]), kr

@@ -30,8 +30,8 @@ def _gradients(dims, growth, average, slug, ste):
     K, A0, cot = _inputs(dims)
     leaves = [torch.as_tensor(x).cuda().requires_grad_()
               for x in (A0, K, np.array([[M, S]], np.float32), np.array([[W]], np.float32), np.float32(DT))]
-    out = AG.run(*leaves, STEPS, growth_fn_t=(growth,), weighted_fn=core.weighted_mean if average else core.weighted_sum,
-                 state_slug=slug, ste=ste, ckpt_every=CKPT)
+    weighted = core.weighted_mean if average else core.weighted_sum
+    out = AG.run(*leaves, STEPS, growth_fn_t=(growth,), weighted_fn=weighted, state_slug=slug, ste=ste, ckpt_every=CKPT)
     return [g.cpu().numpy() for g in torch.autograd.grad((out * torch.as_tensor(cot).cuda()).sum(), leaves)]
 
 

@@ -120,7 +120,8 @@ def test_few_worlds_at_the_most_items_a_thread_takes():
     check((64, 512), 4, 6, 'v1', True, False)
 
 
-@pytest.mark.parametrize('B,C,maxk,H,W,kh,kw', [(2, 2, 1, 17, 65, 5, 7), (1, 1, 2, 40, 24, 1, 8), (3, 1, 1, 8, 8, 13, 13)])
+@pytest.mark.parametrize('B,C,maxk,H,W,kh,kw', [(2, 2, 1, 17, 65, 5, 7), (1, 1, 2, 40, 24, 1, 8),
+                                                (3, 1, 1, 8, 8, 13, 13)])
 def test_direct_adjoint_without_a_workspace(B, C, maxk, H, W, kh, kw):
     """lx_potential_direct_adjoint (one workgroup per tap) against float64 sums and the entry with a workspace:
     positive terms, a thread adds B ceil(H W / 256) of them in a row, then six rounds of lanes and four waves."""
@@ -152,7 +153,8 @@ def test_direct_adjoint_without_a_workspace(B, C, maxk, H, W, kh, kw):
 
 
 DIRECT = ([(2, 1, 1, 17, 65, 7, 1), (1, 2, 2, 33, 70, 1, 2), (3, 1, 1, 40, 63, 64, 3), (1, 1, 1, 8, 8, 5, 4),
-           (2, 1, 1, 64, 64, 5, 5)] + [(2, 1, 1, 50, 130, 3, kw) for kw in (6, 9, 12, 16, 17, 21, 25, 33, 37, 41, 48, 49, 64)] +
+           (2, 1, 1, 64, 64, 5, 5)] +
+          [(2, 1, 1, 50, 130, 3, kw) for kw in (6, 9, 12, 16, 17, 21, 25, 33, 37, 41, 48, 49, 64)] +
           [(64, 1, 1, 128, 128, 64, 64), (65, 1, 1, 100, 128, 53, 57)])
 
 
@@ -196,9 +198,9 @@ def test_narrow_potential_of_a_state_that_is_not_finite():
     assert np.array_equal(pot[np.isfinite(pot)], np.full(3180, 20 * 0.125, np.float32))
 
 
-@pytest.mark.parametrize('B,H,W,k', [(1, 40, 40, 5), (1, 52, 96, 32), (1, 64, 100, 9), (2, 167, 82, 25), (2, 195, 58, 18),
-                                     (4, 42, 177, 19), (3, 159, 154, 8), (1, 128, 128, 40), (2, 256, 256, 13),
-                                     (20, 86, 218, 7)])
+@pytest.mark.parametrize('B,H,W,k', [(1, 40, 40, 5), (1, 52, 96, 32), (1, 64, 100, 9), (2, 167, 82, 25),
+                                     (2, 195, 58, 18), (4, 42, 177, 19), (3, 159, 154, 8), (1, 128, 128, 40),
+                                     (2, 256, 256, 13), (20, 86, 218, 7)])
 def test_kernel_gradient_is_as_accurate_as_tap_by_tap(B, H, W, k):
     """The kernel gradient with a workspace is no further from float64 than one block per tap (the entry without one),
     whatever the number of cells: terms of both signs, so a sum's error goes with its longest chains of additions;
@@ -217,8 +219,8 @@ def test_kernel_gradient_is_as_accurate_as_tap_by_tap(B, H, W, k):
     errs = []
     for entry, tail in (('lx_potential_direct_adjoint', ()), ('lx_potential_direct_adjoint_work', (engine.ptr(work),))):
         dk = torch.empty_like(tk)
-        _lib.call(entry, ctypes.byref(rule), engine.ptr(tA), B, engine.ptr(tk), k, k, engine.ptr(tU), None, engine.ptr(dk),
-                  *tail, engine.stream_ptr())
+        _lib.call(entry, ctypes.byref(rule), engine.ptr(tA), B, engine.ptr(tk), k, k, engine.ptr(tU), None,
+                  engine.ptr(dk), *tail, engine.stream_ptr())
         errs.append(float(np.linalg.norm(dk.cpu().numpy() - ref) / np.linalg.norm(ref)))
     print('  by tap, with a workspace', errs)
     assert errs[1] <= 1.25 * errs[0]
