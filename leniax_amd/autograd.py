@@ -403,6 +403,8 @@ def ring_basis(R, r, nb_rings, kf_slug, kf_params, world_size, host=False):
 
 def ring_kernel(b, basis):
     """circle_2d's kernel, padded and fftshift-ed, as a differentiable function of ``b``."""
+    if b.dim() != 1 or b.dtype != basis.dtype:  # the product below would broadcast and promote
+        raise RuntimeError(f'ring weights: one {basis.dtype} per ring expected, got {b.dtype} {list(b.shape)}')
     # products and a sum over the few rings: the einsum's gradient of b is a library matrix product with one
     # row per ring and a reduction over all cells (91 us for three rings of 256 x 256, 18 us this way)
     raw = (b[:, None, None] * basis).sum(0)

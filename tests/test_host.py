@@ -378,3 +378,19 @@ def test_tuner_controls_without_a_device(tmp_path):
     finally:
         _lib.call('lx_tune_cache', None)
         engine.autotune(prev)
+
+
+@pytest.mark.parametrize('b', [[[1.], [0.5], [0.25]], 1., [1., 0.5]])
+def test_ring_kernel_refuses_weights_that_are_not_one_per_ring(b):
+    torch = pytest.importorskip('torch')
+    from leniax_amd import autograd as AG
+    with pytest.raises(RuntimeError):
+        AG.ring_kernel(torch.tensor(b), torch.rand(3, 4, 4))
+
+
+@pytest.mark.parametrize('dtype', ['float64', 'float16', 'int64'])
+def test_ring_kernel_refuses_weights_of_another_type_than_the_basis(dtype):
+    torch = pytest.importorskip('torch')
+    from leniax_amd import autograd as AG
+    with pytest.raises(RuntimeError):
+        AG.ring_kernel(torch.ones(3, dtype=getattr(torch, dtype)), torch.rand(3, 4, 4))
