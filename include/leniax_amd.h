@@ -329,6 +329,8 @@ int lx_adjoint_step(const lx_rule* rule, int64_t B, const float* state_d, const 
  *    refills their slots from the queue of worlds not yet started (at most `slots` in flight), and
  *    the step loop is replayed from HIP graphs of several steps.  This path waits on the stream
  *    between graph replays to read the live count (it returns once the last replay is enqueued).
+ *    Without a stop policy and with every world in flight no world retires early: the steps are
+ *    enqueued one after another and the call does not wait.  Neither form can be captured.
  * The statistics rows after a world's last step are left as the caller put them. */
 typedef struct lx_run_args {
   const float* cells0_d;   /* [B][C][dims] initial states */

@@ -130,8 +130,8 @@ __global__ __launch_bounds__(256) void direct_narrow_kernel(DirectArgs a, const 
 // block, so 7 quads of columns take 28 tap columns for a 25-tap row (1.12x the products).  Each output
 // adds its products in the order of i, then j.  A tile that holds a value that is not finite is summed
 // product by product, so that none meets a zero beside the kernel.
-// Measured, 128 worlds of 128^2, 25 x 25 taps, R = 2: potential 60 -> 41 us (64 TFLOP/s of the taps), state
-// side 94 -> 42 us (the vector units' window kernel before took its flipped taps one by one); 12 us of
+// Measured, 128 worlds of 128^2, 25 x 25 taps, R = 2: potential 60 -> 41 us (64 TFLOP/s of the taps; 45 beside
+// the gradients' kernels), state side 94 -> 42 us (the vector units' window kernel before took its flipped taps one by one); 12 us of
 // it stage the tiles, the instructions themselves need 25.  Groups of equal size rather than of four quads with
 // a partly empty last one: 47 -> 41 us there, 72 -> 57 at 33 taps a side, 149 -> 122 at 48.
 template <int R, bool ADJ>

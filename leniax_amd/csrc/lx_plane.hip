@@ -9,8 +9,8 @@
 // Transforms run over lane groups with the cross-lane step between registers (no exchange scratch, so that
 // a plane of 96 x 96 takes 40 KB and four workgroups share a CU).  A plane's rows have stride 4 mod 8
 // complex: the 8 rows x 4 columns that 32 lanes read at once lie in different banks.
-// Measured, us, the passes they replace -> these: 16 worlds of 96^3, forward 46 -> 29 (115 MB: 4.0 TB/s), inverse
-// with field and potential written 111 -> 67 (284 MB: 4.2 TB/s); 8 worlds, a chained reverse step 72 -> 49 (143 MB).
+// Measured, us, the passes they replace -> these: 16 worlds of 96^3, forward 46 -> 27 (115 MB: 4.3 TB/s), inverse
+// with field and potential written 111 -> 64 (284 MB: 4.4 TB/s); 8 worlds, a chained reverse step 72 -> 48 (143 MB).
 #include <algorithm>
 
 #include "lx_pass.h"
