@@ -1009,11 +1009,10 @@ RowArgs row_args(const lx_rule* rule) {
   return ra;
 }
 
-// Whether a 3-D pass over so many images takes the plane kernels: their sides, enough planes, arrays that start on
-// 16 bytes, no pinned knob of the lines along H.
-bool takes_planes(const Geom& g, int64_t nimg, std::initializer_list<const void*> arrays, bool reverse = false) {
+// Whether a 3-D pass can take the plane kernels: their sides, arrays that start on 16 bytes, no pinned knob of the
+// lines along H.
+bool takes_planes(const Geom& g, std::initializer_list<const void*> arrays) {
   if (g.naxes != 2 || !lx_plane_takes(g.L[1], g.W)) return false;
-  if (!lx_plane_pays(g.L[1], g.W, nimg * g.L[0], reverse)) return false;
   LineArgs along_h = line_args();
   along_h.mode = 1;
   if (line_knob_pinned(along_h, g.L[1])) return false;
@@ -1026,7 +1025,7 @@ bool takes_planes(const Geom& g, int64_t nimg, std::initializer_list<const void*
 // step before)
 int fwd_inner(const Geom& g, const float* A, float2* S, int64_t nimg, hipStream_t st,
               const RunStatArgs* prev = nullptr) {
-  if (takes_planes(g, nimg, {A})) {
+  if (takes_planes(g, {A}) && lx_plane_pays(g.L[1], g.W, nimg * g.L[0], false)) {
     if (prev)
       if (int rc = launch_run_stats(*prev, st)) return rc;
     return lx_plane_fwd(g.L[1], g.W, A, S, nimg * g.L[0], st);
@@ -1052,7 +1051,8 @@ int inv_inner(const Geom& g, RowArgs ra, int64_t nk, int64_t nimg, hipStream_t s
   ra.rows = g.rows;
   // (several kernels without potentials of the caller's: they go over the planes' own spectra)
   const void* over = ra.C * ra.K > 1 && !ra.pot ? ra.U : nullptr;
-  if (!ra.part && takes_planes(g, nk, {ra.A, ra.A_out, ra.field, ra.pot, over}))
+  if (!ra.part && takes_planes(g, {ra.A, ra.A_out, ra.field, ra.pot, over}) &&
+      lx_plane_pays(g.L[1], g.W, nk * g.L[0], true))
     return lx_plane_inv(ra, g.L[0], g.L[1], g.W, nimg, st);
   if (g.naxes == 2) {
     LineArgs la = line_args();
@@ -2076,7 +2076,7 @@ int lx_adj11_init(const lx_rule* rule, int64_t B, const float* gf_d, int64_t gf_
   c->lam = lambda_d; c->g_gf = grad_gf_d; c->g_w = grad_w_d; c->g_dt = grad_dt_d;
   c->X = work_d;
   c->part = lx_adj_work_11(rule, B, adj_work_d);
-  c->planes = takes_planes(g, B, {lambda_d, U, A}, true);
+  c->planes = takes_planes(g, {lambda_d, U, A}) && lx_plane_pays_reverse(g.L[0], g.L[1], g.W);
   const int64_t pairs_per_block = 256 / lx_row_tpr(g.W);
   c->bpw = c->planes ? int(g.L[0]) : int((g.rows / 2 + pairs_per_block - 1) / pairs_per_block);
   return LX_OK;

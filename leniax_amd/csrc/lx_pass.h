@@ -332,7 +332,8 @@ int lx_small_rows(const RowArgs& a, int W, int64_t images, bool list, hipStream_
 // states, fields and potentials start on 16 bytes), and the convolution along the outer one for worlds
 // that share a spectrum (*taken as above).
 bool lx_plane_takes(int H, int W);
-bool lx_plane_pays(int H, int W, int64_t planes, bool reverse);  // the planes are enough to fill the chip
+bool lx_plane_pays(int H, int W, int64_t planes, bool inverse);  // the planes are enough to fill the chip
+bool lx_plane_pays_reverse(int D, int H, int W);
 int lx_plane_fwd(int H, int W, const float* A, float2* S, int64_t planes, hipStream_t st);
 int lx_plane_inv(const RowArgs& a, int D, int H, int W, int64_t images, hipStream_t st);
 struct LxPlaneAdj {

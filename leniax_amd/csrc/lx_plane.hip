@@ -623,19 +623,26 @@ int plane_tables_of(int H, int W, hipStream_t st, PlaneTables* tb) {
 
 bool lx_plane_takes(int H, int W) { return by_plane(H, W, [](auto, auto) {}); }
 
-// A plane is one workgroup's: up to 6144 points it takes no longer than the rows' and lines' passes do on any
-// number of CUs; a larger one is a chain of 32 to 64 points a lane, which pays once most CUs have one, and from
-// 9216 points up in the reverse once they have two (LDS leaves two workgroups per CU of 128-point rows, and 96
-// rows of them are a round and a half).  Measured, us of these kernels against rows and lines for 16, 128, 192,
-// 256, 512, 1024 planes: update of 96 x 96 23 / 19, 26 / 26, 27.5 / 32, 29 / 34, 35 / 49, 51 / 85; of 128 x 128
-// 36 / 18, 41 / 33, 42 / 38, 44 / 45, 58 / 71, 113 / 123; four steps and their reverse of 96 x 96 210 / 164,
-// 242 / 220, 254 / 260, 261 / 280, 327 / 404; of 128 x 128 327 / 161, 368 / 268, 380 / 315, 398 / 361, 544 / 611,
-// 1082 / 1075; 64 x 64 19 / 19, 20 / 20, 20 / 22, 21 / 23.
-bool lx_plane_pays(int H, int W, int64_t planes, bool reverse) {
-  const int points = H * W;
-  if (points <= 6144) return true;
-  return planes >= (points <= 9216 ? 192 : reverse ? 512 : 256);
+// A plane is one workgroup's: a chain of up to 64 points a lane whatever the number of planes, where rows and lines
+// spread over the chip (and a few worlds' rows have kernels of their own).  Small planes are no slower at any count,
+// large ones once most CUs have one.  Measured, us of these kernels against rows and lines for 16, 64, 128, 160, 256,
+// 512 planes: forward of 96 x 96 7.6 / 8.9, 8.5 / 9.6, 9.2 / 11.2, 9.8 / 12.2, 10.4 / 13.1, 12.6 / 19.5, of 128 x 96
+// 9.4 / 8.7, 10.3 / 9.7, 11.7 / 11.6, 11.8 / 12.3, 12.3 / 14.8, 16.6 / 24.1, of 128 x 128 13.1 / 8.7, 14.6 / 10.3,
+// 15.2 / 12.2, 15.5 / 13.5, 17.4 / 17.9, 23.1 / 27.3; inverse with the update of 96 x 64 11.8 / 9.9, 12.1 / 11.6,
+// 12.3 / 12.6, 12.6 / 13.0, 13.4 / 14.7, 17.7 / 25.0, of 96 x 96 15.5 / 10.5, 15.9 / 13.7, 16.5 / 14.9, 16.8 / 17.2,
+// 18.1 / 20.7, 22.4 / 29.3, of 128 x 128 23.3 / 9.7, 24.0 / 12.6, 25.1 / 20.3, 25.6 / 22.3, 26.4 / 26.3, 34.9 / 43.1.
+bool lx_plane_pays(int H, int W, int64_t planes, bool inverse) {
+  if (!inverse) return H * W <= 9216 || planes >= (W < 128 ? 96 : 256);
+  return H * W <= 6144 || planes >= (W < 128 || H < 96 ? 160 : 256);
 }
+
+// The reverse sums a world's gradient scalars in an order that its route fixes, and a world's gradients do not
+// depend on the batch it is in: the route goes by the world's size alone.  Large planes of worlds of 64 planes up,
+// but not 128-point rows by 96 or more (LDS leaves two workgroups per CU, and 96 rows are a round and a half).
+// Measured as above, four steps and their reverse: 96 x 96 210 / 164, 242 / 220, 254 / 260, 261 / 280, 327 / 404,
+// 534 / 712; 128 x 96 236 / 160, 276 / 231, 287 / 287, 298 / 312, 398 / 518, 747 / 880; 128 x 128 327 / 161, 368 / 268,
+// 380 / 315, 398 / 361, 544 / 611, 1082 / 1075.
+bool lx_plane_pays_reverse(int D, int H, int W) { return H * W <= 6144 || (D >= 64 && !(W >= 128 && H >= 96)); }
 
 int lx_plane_fwd(int H, int W, const float* A, float2* S, int64_t planes, hipStream_t st) {
   PlaneTables tb;

@@ -122,7 +122,8 @@ def test_a_workspace_that_starts_on_8_bytes():
     assert torch.equal(new, ref)
 
 
-@pytest.mark.parametrize('dims,few,many', [((16, 128, 128), 1, 17), ((16, 96, 96), 11, 12), ((32, 64, 128), 5, 6)])
+@pytest.mark.parametrize('dims,few,many', [((16, 128, 128), 1, 17), ((16, 96, 96), 9, 10), ((32, 64, 128), 4, 5),
+                                           ((16, 128, 96), 5, 10)])
 def test_few_large_planes_take_rows_and_lines(dims, few, many):
     """A large plane is one workgroup's long chain: below a count the passes spread over the chip instead, with the
     same bits."""
@@ -133,12 +134,12 @@ def test_few_large_planes_take_rows_and_lines(dims, few, many):
     ref = _update(rule, Kh, gf, w, A)
     B = A[:few].contiguous()
     names = _kernels(lambda: _update(rule, Kh, gf, w, B))
-    assert not any('plane' in n for n in names), names
+    assert not any('plane_inv' in n or dims[1] * dims[2] > 9216 and 'plane' in n for n in names), names
     for a, b in zip(ref, _update(rule, Kh, gf, w, B)):
         assert torch.equal(a[:few], b)
 
 
-@pytest.mark.parametrize('dims,B', [((16, 96, 96), 12), ((16, 128, 128), 32)])
+@pytest.mark.parametrize('dims,B', [((64, 96, 96), 3), ((96, 128, 96), 3), ((64, 64, 128), 3)])
 def test_reverse_through_large_planes_gives_the_same_bits(knobs, dims, B):  # noqa: F811
     """dL/dA0 of a run of whole planes against rows and lines (a pinned knob of the lines turns the planes off)."""
     from leniax_amd import autograd as AG

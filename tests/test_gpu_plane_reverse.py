@@ -70,3 +70,39 @@ def test_planes_against_rows_and_lines_and_float64(knobs, growth, average, slug,
             assert err <= 2 * 128 * 2.0 ** -24 * DT * total  # of both signs, each at most dt |dL/dz|
         else:
             assert err <= 4 * env + 1e-4 * np.abs(r64).max(), name
+
+
+@pytest.mark.parametrize('dims,many', [((16, 128, 128), 33), ((16, 96, 96), 13), ((64, 96, 96), 9), ((32, 64, 128), 9),
+                                       ((16, 32, 48), 5)])
+def test_a_worlds_gradients_do_not_depend_on_its_batch(dims, many):
+    """lx_adjoint_step of 3-D worlds with parameters of their own, in a batch and alone: dL/d(state in), the
+    kernel-spectrum gradient and the gradient scalars of the first worlds bit for bit."""
+    import ctypes
+    from leniax_amd import _lib, autograd as AG, engine
+    print('gradients alone and in a batch', dims, many, flush=True)
+    rng = np.random.default_rng(dims[1])
+    rule = engine.make_rule(list(dims), 1, [0], [_lib.GROWTH_IDS['gaussian']], _lib.STATE_FN['v2'], 0)
+    Kh = torch.as_tensor(np.fft.rfftn(rng.random(dims) / np.prod(dims)).astype(np.complex64)).cuda()[None, None]
+    A = torch.rand((many, 1) + dims, device='cuda')
+    U, lam0 = 0.4 * torch.rand((many, 1) + dims, device='cuda'), torch.randn((many, 1) + dims, device='cuda')
+    gf = torch.tensor([[0.2, 0.05]], device='cuda').repeat(many, 1)
+    w, dt = torch.full((many,), 0.7, device='cuda'), torch.full((many,), 0.1, device='cuda')
+    FA = AG.rfftn(A, 3)
+    outs = []
+    for B in (many, 1):
+        nb = ctypes.c_size_t(0)
+        _lib.call('lx_workspace_size', ctypes.byref(rule), B, ctypes.byref(nb))
+        work = torch.empty(nb.value, dtype=torch.uint8, device='cuda')
+        _lib.call('lx_adjoint_workspace_size', ctypes.byref(rule), B, ctypes.byref(nb))
+        aw = torch.empty(nb.value, dtype=torch.uint8, device='cuda')
+        lam = lam0[:B].clone()
+        ggf, gw, gdt = torch.zeros_like(gf[:B]), torch.zeros_like(w[:B]), torch.zeros_like(dt[:B])
+        dspec = torch.zeros((B, 1) + tuple(FA.shape[2:]), dtype=torch.complex64, device='cuda')
+        _lib.call('lx_adjoint_step', ctypes.byref(rule), B, engine.ptr(A), None, engine.ptr(U), engine.ptr(gf), 2,
+                  engine.ptr(w), 1, engine.ptr(dt), 1, engine.ptr(Kh), 0, 1, engine.ptr(FA), engine.ptr(dspec),
+                  engine.ptr(lam), None, engine.ptr(ggf), engine.ptr(gw), engine.ptr(gdt), engine.ptr(work),
+                  engine.ptr(aw), engine.stream_ptr())
+        outs.append([x[:1].cpu().numpy() for x in (lam, dspec, ggf, gw, gdt)])
+    for x, y in zip(*outs):
+        assert np.array_equal(x, y)
+    assert all(np.abs(x).max() > 0 for x in outs[1])
